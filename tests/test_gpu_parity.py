@@ -207,6 +207,19 @@ def test_fp64_ill_conditioned_mode_bitexact(cuda_device):
     assert np.abs(out[True] - out[False]).max() > 1e-4
 
 
+@pytest.mark.parametrize("mass", [1.0e-2, 1.0e-3, 1.0e-4, 1.0e-5, 1.0e-6])
+def test_condition_screen_bitexact(cuda_device, mass):
+    """Block conditions from about 1 to 1e4, on both sides of the single-precision screen (2e5 at most) that lets
+    well-conditioned blocks skip the double-precision estimate: the oracle always evaluates that estimate."""
+    from newton_amd import scenes
+
+    model, state, info = scenes.bead_rope_light(cuda_device, mass=mass)
+    q0, qd0 = initial(state)
+    q_gpu, qd_gpu, _ = gpu_run(model, state, info, 10, solver_kwargs={"fp64_ill_conditioned": True})
+    q_ref, qd_ref, _ = oracle_run(model, q0, qd0, info, 10, fp64_ill_conditioned=True)
+    assert np.array_equal(q_gpu, q_ref) and np.array_equal(qd_gpu, qd_ref)
+
+
 def test_penalty_ramp_bitexact(cuda_device):
     """rigid_avbd_beta > 0 exercises the per-iteration penalty update (rigid_vbd_kernels.py:4861-4926)."""
     model, state, info = _scene("strip", cuda_device)
