@@ -201,14 +201,24 @@ __device__ __forceinline__ float portable_atan2f(float y, float x) {
 // element force / Hessian contributions for one (vertex, element) pair
 // ---------------------------------------------------------------------------
 
-// Stable Neo-Hookean membrane, particle_vbd_kernels.py:502-632.
-__device__ void eval_membrane(V3 X0, V3 X1, V3 X2, const float* __restrict__ qp, int i0, int i1, int i2,
-                              const float* __restrict__ pose, float area, float mu, float lmbd, float damping, float dt,
-                              int v_order, V3& f_out, M3& h_out) {
+// vbd_layout::lame_sum / rest_ratio for the generic path, which reads the model's materials
+__device__ __forceinline__ float lame_sum(float mu, float lambda) { return lambda + mu; }
+__device__ __forceinline__ float rest_ratio(float mu, float lambda) {
+    const float l_nh = lame_sum(mu, lambda);
+    const float l_safe = (l_nh < 0.0f ? -1.0f : 1.0f) * fmaxf(fabsf(l_nh), 1.0e-6f);
+    return 1.0f + mu / l_safe;
+}
+
+// Stable Neo-Hookean membrane, particle_vbd_kernels.py:502-632.  l_nh = lambda + mu and alpha = 1 + mu / l_nh
+// come from the caller (vbd_layout::lame_sum, rest_ratio), inv_dt = 1 / dt from the host; prev(k) gives the
+// previous position of corner k (read for damped elements only).
+template <typename Prev>
+__device__ __forceinline__ void eval_membrane(V3 X0, V3 X1, V3 X2, Prev prev, float D00, float D01, float D10,
+                                              float D11, float area, float mu, float l_nh, float alpha, float damping,
+                                              float inv_dt, int v_order, V3& f_out, M3& h_out) {
     V3 x0 = X0;
     V3 x01 = sub(X1, x0);
     V3 x02 = sub(X2, x0);
-    float D00 = pose[0], D01 = pose[1], D10 = pose[2], D11 = pose[3];
     V3 f0 = add(scl(x01, D00), scl(x02, D10));
     V3 f1 = add(scl(x01, D01), scl(x02, D11));
     float f0f0 = dot(f0, f0), f1f1 = dot(f1, f1), f0f1 = dot(f0, f1);
@@ -217,9 +227,6 @@ __device__ void eval_membrane(V3 X0, V3 X1, V3 X2, const float* __restrict__ qp,
     float Js = sqrtf(Jsq);
     float invJ = 1.0f / Js;
     float mu_nh = mu;
-    float l_nh = lmbd + mu;
-    float l_safe = (l_nh < 0.0f ? -1.0f : 1.0f) * fmaxf(fabsf(l_nh), 1.0e-6f);
-    float alpha = 1.0f + mu_nh / l_safe;
     V3 g0 = scl(sub(scl(f0, f1f1), scl(f1, f0f1)), invJ);
     V3 g1 = scl(sub(scl(f1, f0f0), scl(f0, f0f1)), invJ);
     float s = l_nh * (Js - alpha);
@@ -244,8 +251,7 @@ __device__ void eval_membrane(V3 X0, V3 X1, V3 X2, const float* __restrict__ qp,
             hess.m[i][j] = (I_coeff * (i == j ? 1.0f : 0.0f) + c1 * (comp(dJ, i) * comp(dJ, j))) -
                            r * (comp(w, i) * comp(w, j));
     if (damping > 0.0f) {
-        float inv_dt = 1.0f / dt;
-        V3 A0 = ld3(qp, i0), A1 = ld3(qp, i1), A2 = ld3(qp, i2);
+        V3 A0 = prev(0), A1 = prev(1), A2 = prev(2);
         V3 x01p = sub(A1, A0);
         V3 x02p = sub(A2, A0);
         V3 f0p = add(scl(x01p, D00), scl(x02p, D10));
@@ -292,14 +298,13 @@ __device__ __forceinline__ M3 nvd_skew(float len, V3 nh, V3 v) {
 // (zero where the reference uses a zero matrix, :730-741) the reference's
 // products are reproduced term for term; the terms it adds for the other
 // slots, and its 0/1 mask selection, contribute signed zeros only.
-__device__ void eval_bending(const float* __restrict__ q, const float* __restrict__ qp, int i0, int i1, int i2,
-                             int i3, float rest_angle, float rest_length, float stiffness, float damping, float dt,
-                             int v_order, V3& f_out, M3& h_out) {
+// k = ke * rest_length and kdl = kd * rest_length come from the caller.
+template <typename Prev>
+__device__ __forceinline__ void eval_bending(V3 x0, V3 x1, V3 x2, V3 x3, Prev prev, float rest_angle, float k,
+                                             float kdl, bool damped, float inv_dt, int v_order, V3& f_out, M3& h_out) {
     f_out = v3(0.0f, 0.0f, 0.0f);
     h_out = mzero();
-    if (i0 == -1 || i1 == -1) return;
     const float eps = 1.0e-6f;
-    V3 x0 = ld3(q, i0), x1 = ld3(q, i1), x2 = ld3(q, i2), x3 = ld3(q, i3);
     V3 x02 = sub(x2, x0), x03 = sub(x3, x0), x13 = sub(x3, x1), x12 = sub(x2, x1), e = sub(x3, x2);
     V3 n1 = cross(x02, x03), n2 = cross(x13, x12);
     float n1n = length(n1), n2n = length(n2), en = length(e);
@@ -308,7 +313,6 @@ __device__ void eval_bending(const float* __restrict__ q, const float* __restric
     float sin_t = dot(cross(n1h, n2h), eh);
     float cos_t = dot(n1h, n2h);
     float theta = portable_atan2f(sin_t, cos_t);
-    float k = stiffness * rest_length;
     float dE = k * (theta - rest_angle);
     // per-component selects (the compiler turns selects of whole vectors into branches)
     const bool o0 = v_order == 0, o1 = v_order == 1, o2 = v_order == 2;
@@ -338,9 +342,8 @@ __device__ void eval_bending(const float* __restrict__ q, const float* __restric
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j) bh.m[i][j] = k * (comp(dth, i) * comp(dth, j));
-    if (damping > 0.0f) {
-        float inv_dt = 1.0f / dt;
-        V3 p0 = ld3(qp, i0), p1 = ld3(qp, i1), p2 = ld3(qp, i2), p3 = ld3(qp, i3);
+    if (damped) {
+        V3 p0 = prev(0), p1 = prev(1), p2 = prev(2), p3 = prev(3);
         V3 x02p = sub(p2, p0), x03p = sub(p3, p0), x13p = sub(p3, p1), x12p = sub(p2, p1), ep = sub(p3, p2);
         V3 n1pr = cross(x02p, x03p), n2pr = cross(x13p, x12p);
         float n1pn = length(n1pr), n2pn = length(n2pr), epn = length(ep);
@@ -355,8 +358,8 @@ __device__ void eval_bending(const float* __restrict__ q, const float* __restric
             else if (dtheta < -3.141592653589793f)
                 dtheta = dtheta + 6.283185307179586f;
             float dtheta_dt = dtheta * inv_dt;
-            bf = add(bf, scl(dth, -damping * rest_length * dtheta_dt));
-            float hs = damping * rest_length * inv_dt;
+            bf = add(bf, scl(dth, -kdl * dtheta_dt));
+            float hs = kdl * inv_dt;
 #pragma unroll
             for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -367,17 +370,12 @@ __device__ void eval_bending(const float* __restrict__ q, const float* __restric
     h_out = bh;
 }
 
-// Volumetric stable Neo-Hookean tetrahedron, particle_vbd_kernels.py:76-292, :347-367.
-__device__ void eval_tet(const float* __restrict__ q, const float* __restrict__ qp, const int* __restrict__ ti,
-                         const float* __restrict__ dm, float mu, float lmbd, float damping, float dt, int v_order,
-                         V3& f_out, M3& h_out) {
-    M3 Dm;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) Dm.m[i][j] = dm[3 * i + j];
-    float rest_volume = 1.0f / (mdet(Dm) * 6.0f);
-    V3 X0 = ld3(q, ti[0]), X1 = ld3(q, ti[1]), X2 = ld3(q, ti[2]), X3 = ld3(q, ti[3]);
+// Volumetric stable Neo-Hookean tetrahedron, particle_vbd_kernels.py:76-292, :347-367; rest_volume, l_nh and
+// alpha come from the caller (vbd_layout.h).
+template <typename Prev>
+__device__ __forceinline__ void eval_tet(V3 X0, V3 X1, V3 X2, V3 X3, Prev prev, const M3& Dm, float rest_volume,
+                                         float mu, float l_nh, float alpha, float damping, float inv_dt, int v_order,
+                                         V3& f_out, M3& h_out) {
     V3 c0 = sub(X1, X0), c1 = sub(X2, X0), c2 = sub(X3, X0);
     M3 Ds;
     Ds.m[0][0] = c0.x; Ds.m[0][1] = c1.x; Ds.m[0][2] = c2.x;
@@ -395,9 +393,6 @@ __device__ void eval_tet(const float* __restrict__ q, const float* __restrict__ 
         for (int r = 0; r < 3; ++r) f9[3 * c + r] = F.m[r][c];
     float J = mdet(F);
     float mu_nh = mu;
-    float l_nh = lmbd + mu;
-    float l_safe = (l_nh < 0.0f ? -1.0f : 1.0f) * fmaxf(fabsf(l_nh), 1.0e-6f);
-    float alpha = 1.0f + mu_nh / l_safe;
     float F11 = F.m[0][0], F21 = F.m[1][0], F31 = F.m[2][0];
     float F12 = F.m[0][1], F22 = F.m[1][1], F32 = F.m[2][1];
     float F13 = F.m[0][2], F23 = F.m[1][2], F33 = F.m[2][2];
@@ -445,8 +440,7 @@ __device__ void eval_tet(const float* __restrict__ q, const float* __restrict__ 
                            m3 * (VBD_H9(r, c + 6) * m1 + VBD_H9(r + 3, c + 6) * m2 + VBD_H9(r + 6, c + 6) * m3);
 #undef VBD_H9
     if (damping > 0.0f) {
-        float inv_dt = 1.0f / dt;
-        V3 P0 = ld3(qp, ti[0]), P1 = ld3(qp, ti[1]), P2 = ld3(qp, ti[2]), P3 = ld3(qp, ti[3]);
+        V3 P0 = prev(0), P1 = prev(1), P2 = prev(2), P3 = prev(3);
         V3 d0 = sub(P1, P0), d1 = sub(P2, P0), d2 = sub(P3, P0);
         M3 Dsp;
         Dsp.m[0][0] = d0.x; Dsp.m[0][1] = d1.x; Dsp.m[0][2] = d2.x;
@@ -626,8 +620,43 @@ __device__ bool block_solve(const M3& h, V3 f, int fp64_ill, V3& dx) {
 // kernels
 // ---------------------------------------------------------------------------
 struct KParams {
-    int N;
+    // What every color pass reads, first and together: a work-group's scalar loads of its arguments are its first
+    // round trip, and each cache line of them a miss.
+    // pass layout (vbd_layout.h)
+    const int* batch_blk;
+    const int* item_rec;    // [B * lanes] 16-byte items
+    const int* list;        // [B * list_stride] vertex lists
+    const int* tri_rec;     // [B * (tri_hi - tri_lo)] and so on: the wider parts of the records
+    const int* tet_rec;
+    const int* spr_rec;
+    const float* hinge_damp;
+    const int* bat_cinfo;   // per batch {first packed contact, contact count} (k_batch_contacts)
+    const int* bat_coff;    // per batch, max_v + 1 contact offsets relative to the first
+    const int* batch_list;  // when set: launches enumerate these batch indices (live worlds only)
+    // per-world freezing (batched iterate-to-tolerance): when w_active is set, vertices of
+    // worlds with w_active[p_world[v]] == 0 are neither solved nor re-evaluated
+    const int* w_active;
+    float* q_prev;
+    float* inertia;
+    float* disp;
     const float* mass;
+    float* crows;         // full-surface contexts: every packed entry's row (force 3 + Hessian 9), evaluated
+                          // by k_contact_rows at the pass start and read back in the serial sum
+    int list_stride;
+    int tri_hi, hinge_lo, hinge_hi, tet_lo, tet_hi, spr_lo, spr_hi;  // lanes that hold each kind (tri_lo = 0)
+    int hinge_damped;      // hinge_damp is read
+    int prev;              // some item reads previous positions
+    float inv_dt, dtr;     // 1 / dt and 1 / (dt * dt) of the launch
+    // self-contact rows per color position (vbd_self.h) and whether the pass writes q
+    int has_self;
+    int write_q;
+    const int* so_off;
+    const float* so_rows;
+    const float* cpack;    // contacts packed per color position (k_contact_sort, k_contact_pack)
+    float friction_epsilon;
+    int fp64_ill;
+    // the rest
+    int N;
     const float* inv_mass;
     const float* radius;
     const int* flags;
@@ -651,21 +680,7 @@ struct KParams {
     int has_tri, has_edge, has_tet;
     const int* color_particles;
     const float* gravity;
-    float* q_prev;
-    float* inertia;
-    float* disp;
-    // pass layout (vbd_layout.h)
-    const int* batch_blk;
-    const int* batch_list;  // when set: launches enumerate these batch indices (live worlds only)
-    int aligned;            // item ranges of a batch start on wave boundaries (layout built so)
-    const int* bat_cinfo;  // per batch {first packed contact, contact count} (k_batch_contacts)
-    const int* bat_coff;   // per batch, max_v + 1 contact offsets relative to the first
     const int* vert_rec;
-    const int* tri_rec;
-    const int* edge_rec;
-    const int* edge_meta;
-    const int* tet_rec;
-    const int* tet_meta;
     const int* slow_pos;
     // springs: model arrays, batch items, same-color pre items and their rows, slow-vertex lists
     int has_spring;
@@ -673,20 +688,11 @@ struct KParams {
     const float* spring_rest;
     const float* spring_ke;
     const float* spring_kd;
-    const int* spr_rec;
     const int* pre_item;
     float* spr_rows;
     const int* slow_spr_off;
     const int* slow_spr;
-    // self-contact rows per color position (vbd_self.h) and whether the pass writes q
-    int has_self;
-    const int* so_off;
-    const float* so_rows;
-    int write_q;
-    // per-world freezing (batched iterate-to-tolerance): when w_active is set, vertices of
-    // worlds with w_active[p_world[v]] == 0 are neither solved nor re-evaluated
     const int* p_world;
-    const int* w_active;
     // per-contact state
     const float* c_pk;
     const float* c_kd;
@@ -695,16 +701,10 @@ struct KParams {
     const float* c_body_pos;
     const float* c_body_vel;
     const float* c_normal;
-    // contacts packed per color position (k_contact_sort, k_contact_pack)
     const int* pos_coff;
-    const float* cpack;
     const int* cpack_ef;  // per packed entry of an edge/face record: {c0, c1, c2, corner} {w0, w1, w2, 0}
-    float* crows;         // full-surface contexts: every packed entry's row (force 3 + Hessian 9), evaluated
-                          // by k_contact_rows at the pass start and read back in the serial sum
     const float* shape_margin;
     int shape_count;
-    float friction_epsilon;
-    int fp64_ill;
 };
 
 // packed contact record (one per corner entry): 4 x float4
@@ -713,8 +713,6 @@ struct KParams {
 // the largest corner radius and kContactEF, and their corners and weights in cpack_ef
 constexpr int kContactWords = 16;
 constexpr int kContactEF = 1 << 30;
-
-__device__ __forceinline__ int wave_align(int n) { return (n + 63) & ~63; }
 
 __device__ __forceinline__ bool particle_active(const KParams& P, int v) {
     return (P.flags[v] & 1) && P.mass[v] != 0.0f;
@@ -740,11 +738,6 @@ __device__ __forceinline__ void store_row(float* __restrict__ row, V3 f, const M
         for (int j = 0; j < 3; ++j) row[3 + 3 * i + j] = h.m[i][j];
 }
 
-__device__ __forceinline__ void store_force(float* __restrict__ row, V3 f) {
-    row[0] = f.x;
-    row[1] = f.y;
-    row[2] = f.z;
-}
 
 // component c (0..11) of a row {f, H row-major}, by selects (no dynamic register indexing)
 __device__ __forceinline__ float row_component(V3 f, const M3& h, int c) {
@@ -845,17 +838,21 @@ __device__ __forceinline__ void eval_spring(V3 x0, V3 x1, V3 a0, V3 a1, float re
     h = madd(hs, hd);
 }
 
-// Spring item: in-pass evaluation (pre_row < 0) or the pre-pass row.
+__device__ __forceinline__ void load_row(const float* __restrict__ row, V3& f, M3& h) {
+    const float4* r4 = reinterpret_cast<const float4*>(row);
+    const float4 A = r4[0], B = r4[1], C = r4[2];
+    f = v3(A.x, A.y, A.z);
+    h.m[0][0] = A.w; h.m[0][1] = B.x; h.m[0][2] = B.y;
+    h.m[1][0] = B.z; h.m[1][1] = B.w; h.m[1][2] = C.x;
+    h.m[2][0] = C.y; h.m[2][1] = C.z; h.m[2][2] = C.w;
+}
+
+// Spring item of a generic-path vertex: evaluated here (pre_row < 0) or the pre-pass row.
 __device__ __forceinline__ void spring_item(const KParams& P, const float* __restrict__ q, int v0, int v1,
                                             int endpoint, int pre_row, float rest, float ke, float kd, float dt,
                                             V3& f, M3& h) {
     if (pre_row >= 0) {
-        const float4* r4 = reinterpret_cast<const float4*>(P.spr_rows) + 3 * (size_t)pre_row;
-        const float4 A = r4[0], B = r4[1], C = r4[2];
-        f = v3(A.x, A.y, A.z);
-        h.m[0][0] = A.w; h.m[0][1] = B.x; h.m[0][2] = B.y;
-        h.m[1][0] = B.z; h.m[1][1] = B.w; h.m[1][2] = C.x;
-        h.m[2][0] = C.y; h.m[2][1] = C.z; h.m[2][2] = C.w;
+        load_row(P.spr_rows + 12 * (size_t)pre_row, f, h);
     } else {
         eval_spring(ld3(q, v0), ld3(q, v1), ld3(P.q_prev, v0), ld3(P.q_prev, v1), rest, ke, kd, dt, endpoint, f, h);
     }
@@ -921,54 +918,131 @@ __device__ __forceinline__ float add_rows_in_order(float ca, const float* __rest
 }
 
 // One color pass over packed batches (mode 0: solve and update; mode 1: write the assembled force g).
-// The work-group's global reads form three dependent round trips:
-//   1  the batch block (header + vertex records) and the batch's contact ranges (indexed by batch)
-//   2  each lane's item record (triangle / edge / tet / packed contact) and, for lanes t < nv, the
-//      vertex's mass, inertia target, position, q_prev and displacement
-//   3  the positions (and q_prev when damped) of the items' vertices
+// The work-group's global reads form two dependent round trips:
+//   1  everything found from the batch number alone: the batch block (header + vertex records), the
+//      contact ranges, each lane's item record and its entry of the batch's vertex list
+//   2  the positions (and q_prev when an item reads it) of the listed vertices, staged in LDS for the
+//      items, the packed contacts, and for lanes t < nv the vertex's mass, inertia target and displacement
 // then, in LDS:
 //   a  every lane evaluates its item into the item's canonical row
 //   b  lane (vertex s, component c) sums component c of s's rows serially, in canonical order,
 //      starting from the inertia term; contacts are summed from zero and added afterwards
 //   c  the vertex's lane solves the 3x3 block and writes displacement and position
+// Bound: vector instructions and the waits of one work-group's chain.  The items are read coalesced from fixed
+// slots and the positions once per batch, no load waits for another's branch, and six to seven waves a SIMD cover
+// what waits are left: 936 k cloth vertices in 512 worlds, 60.7 us a pass (65.2 us with element records found through
+// the header and positions gathered per element), 256x256 cloth 8.7 us (10.9).
 constexpr int kBatchHdr = vbd_layout::kBatchWords;
 
-// BLOCK lanes per work-group: 256 (batches of <= 21 vertices / 256 items) or
-// 128 (<= 10 vertices / 128 items).  LDS holds the static items plus 64 contact rows (17 KB at
-// 256 lanes), so LDS does not bound occupancy; WAVES is the register budget's occupancy target:
-// 1 leaves it to the compiler (77 VGPRs, six waves per SIMD), 7 fits seven waves per SIMD at the
-// price of a few values kept in scratch -- faster on cloth, slower on tets (whose evaluation then
-// spills more).  The autotuner picks the shape per model.
+// Element kinds a pass holds.  Every contribution of a cloth pass (triangles, hinges, springs, contacts with
+// shapes) has a Hessian that is symmetric bit for bit, so its rows hold 9 numbers instead of 12: less LDS
+// (more work-groups per CU) and fewer lanes in the sums.  Tet and self-contact Hessians are symmetric
+// only up to rounding.
+enum PassKinds { kClothKinds = 0, kClothSpringKinds = 1, kTetKinds = 2, kAllKinds = 3 };
+
+// component k of a row -> its place in {f (3), H row-major (9)}
+template <bool SYM>
+__device__ __forceinline__ int full_component(int k) {
+    if (!SYM) return k;
+    return k < 6 ? k : (k < 8 ? k + 1 : 11);  // H00 H01 H02 H11 H12 H22
+}
+
+// data that no kernel writes while it reads it, at an address that a whole wave shares: scalar loads
+typedef const __attribute__((address_space(4))) int* UniformInts;
+__device__ __forceinline__ UniformInts uniform_ints(const int* p) { return (UniformInts)(uintptr_t)p; }
+
+template <bool SYM, bool FORCE_ONLY>
+__device__ __forceinline__ void put_row(float* __restrict__ row, V3 f, const M3& h) {
+    row[0] = f.x;
+    row[1] = f.y;
+    row[2] = f.z;
+    if constexpr (FORCE_ONLY) return;
+    int k = 3;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = SYM ? i : 0; j < 3; ++j) row[k++] = h.m[i][j];
+}
+
+// BLOCK lanes per work-group: 256 (batches of <= 21 vertices / 256 items), 192 or 128 (<= 10 vertices /
+// 128 items).  LDS holds the static items' rows plus 64 contact rows and the staged positions;
+// WAVES is the register budget's occupancy target: 1 leaves it to the compiler, 7 asks for seven
+// waves per SIMD.  The autotuner picks the shape per model.
 // FORCE_ONLY (the residual, mode 1): only the force rows are stored and summed, so the Hessian
 // arithmetic of every item is dead code; the force bits are those of the solving pass.
-template <int BLOCK, int WAVES, bool FORCE_ONLY = false>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_solve_fast(KParams P, float* __restrict__ q, int batch_base, int nb,
-                                                      float dt, int mode, float* __restrict__ g_out) {
+template <int BLOCK, int WAVES, int KINDS, bool FORCE_ONLY = false>
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_solve_fast(
+    float* __restrict__ q, int batch_base, int nb, float dt, int mode, float* __restrict__ g_out, KParams P) {
+    constexpr bool CLOTH = KINDS != kTetKinds;
+    constexpr bool TET = KINDS == kTetKinds || KINDS == kAllKinds;
+    constexpr bool SPRING = KINDS == kClothSpringKinds || KINDS == kAllKinds;
+    constexpr bool SELF = KINDS == kAllKinds;
+    constexpr bool SYM = KINDS == kClothKinds || KINDS == kClothSpringKinds;
+    constexpr int NC = FORCE_ONLY ? 3 : (SYM ? 9 : 12);  // numbers per row
     constexpr int MAXV = BLOCK / kComp;
     constexpr int ROWS = BLOCK + 64;  // static items (<= BLOCK) + contacts evaluated in parallel
     constexpr int BLK = kBatchHdr + 4 * MAXV;
+    constexpr int LIST = vbd_layout::list_cap(BLOCK);
     __shared__ int s_row[MAXV];
     __shared__ int s_nrow[MAXV];
     __shared__ int s_nspr[MAXV];
     __shared__ int s_cb[MAXV + 1];
     __shared__ int s_so[MAXV + 1];
-    __shared__ __align__(16) float s_rows[ROWS * kComp];
-    __shared__ float s_acc[MAXV * kComp];
+    __shared__ float4 s_q[LIST];    // positions of the listed vertices
+    __shared__ float4 s_p[LIST];    // their q_prev (own vertices always, the others when P.prev)
+    __shared__ __align__(16) float s_rows[ROWS * NC];
+    __shared__ float s_acc[MAXV * NC];
 
     const int t = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    // the arguments of the second round trip come in with those of the first
+    asm volatile("" ::"s"(q), "s"(P.q_prev), "s"(P.inertia), "s"(P.disp), "s"(P.mass), "s"(P.prev), "s"(P.dtr));
     const int bi = batch_base + xcd_remap(blockIdx.x, nb);
-    const int b = P.batch_list ? P.batch_list[bi] : bi;
-    // ---- round trip 1
+    const int b = P.batch_list ? uniform_ints(P.batch_list)[bi] : bi;
+    // ---- round trip 1.  No load sits under a per-lane condition (indexes are clamped instead, conditions
+    // are a whole wave's): a conditional load ends its block with a wait, and the loads would go out one
+    // after another.
     const int* blk = P.batch_blk + (size_t)b * BLK;
-    const int4 b0 = reinterpret_cast<const int4*>(blk)[0];
-    const int4 b1 = reinterpret_cast<const int4*>(blk)[1];
-    const int4 b2 = reinterpret_cast<const int4*>(blk)[2];
-    const int2 ci = reinterpret_cast<const int2*>(P.bat_cinfo)[b];
-    int4 vr = make_int4(0, 0, 0, 0);
-    if (t < MAXV) vr = reinterpret_cast<const int4*>(blk + kBatchHdr)[t];
-    int cbt = 0;
-    if (t <= MAXV) cbt = P.bat_coff[(size_t)b * (MAXV + 1) + t];
-    const int nv = b0.y, tri_b = b0.z, ntri = b0.w, edge_b = b1.x, nedge = b1.y, tet_b = b1.z, ntet = b1.w;
+    const int v_begin = uniform_ints(blk)[0], nv = uniform_ints(blk)[1], nstatic = uniform_ints(blk)[2];
+    const int cbeg = uniform_ints(P.bat_cinfo)[2 * (size_t)b], ncont = uniform_ints(P.bat_cinfo)[2 * (size_t)b + 1];
+    const int4 item = reinterpret_cast<const int4*>(P.item_rec)[(size_t)b * BLOCK + t];
+    const int id = P.list[(size_t)b * P.list_stride + min(t, P.list_stride - 1)];
+    int4 w0 = make_int4(0, 0, 0, 0), w1 = w0, w2 = w0;
+    float kdl = 0.0f;
+    if constexpr (CLOTH) {
+        if (64 * wave < P.tri_hi) {
+            const int4* r = reinterpret_cast<const int4*>(P.tri_rec) + 2 * ((size_t)b * P.tri_hi + min(t, P.tri_hi - 1));
+            w0 = r[0];
+            w1 = r[1];
+        }
+        if (P.hinge_damped) {
+            const int lane = min(max(t, P.hinge_lo), P.hinge_hi - 1) - P.hinge_lo;
+            kdl = P.hinge_damp[(size_t)b * (P.hinge_hi - P.hinge_lo) + lane];
+        }
+    }
+    if constexpr (TET) {
+        if (64 * wave < P.tet_hi && 64 * wave + 63 >= P.tet_lo) {
+            const int lane = min(max(t, P.tet_lo), P.tet_hi - 1) - P.tet_lo;
+            const int4* r = reinterpret_cast<const int4*>(P.tet_rec) + 3 * ((size_t)b * (P.tet_hi - P.tet_lo) + lane);
+            const int4 a0 = r[0], a1 = r[1], a2 = r[2];
+            // lanes of another kind keep their own record's words
+            const bool mine = !(CLOTH || SPRING) || item.y >> 12 == vbd_layout::kTet;
+            w0 = mine ? a0 : w0;
+            w1 = mine ? a1 : w1;
+            w2 = a2;
+        }
+    }
+    if constexpr (SPRING) {
+        if (P.spr_hi > P.spr_lo) {
+            const int lane = min(max(t, P.spr_lo), P.spr_hi - 1) - P.spr_lo;
+            const int2 r = reinterpret_cast<const int2*>(P.spr_rec)[(size_t)b * (P.spr_hi - P.spr_lo) + lane];
+            const bool mine = item.y >> 12 == vbd_layout::kSpring;
+            w0.x = mine ? r.x : w0.x;
+            w0.y = mine ? r.y : w0.y;
+        }
+    }
+    const int4 vr = reinterpret_cast<const int4*>(blk + kBatchHdr)[min(t, MAXV - 1)];
+    const int cbt = P.bat_coff[(size_t)b * (MAXV + 1) + min(t, MAXV)];
     // frozen worlds: a batch none of whose vertices is live ends here (uniformly)
     bool own_live = true;
     if (P.w_active) {
@@ -976,191 +1050,175 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
         if (t < nv) live = own_live = P.w_active[P.p_world[vr.x]] != 0;
         if (!__syncthreads_or(live)) return;
     }
-    const int spr_b = b2.x, nspr = b2.y;
-    const int nstatic = ntri + nedge + ntet + nspr;
-    const int cbeg = ci.x, ncont = ci.y;
     const bool par_contacts = !P.crows && nstatic + ncont <= ROWS;
-    const float dtr = 1.0f / (dt * dt);
+    const int npar = par_contacts ? ncont : 0;
 
-    // ---- round trip 2: item record of this lane (items 0..255), own-vertex state
-    int kind = 0;  // 1 triangle, 2 edge, 3 tet, 4 contact, 5 spring
-    int4 r0 = make_int4(0, 0, 0, 0), r1 = r0, r2 = r0, r3 = r0;
-    int meta = 0;
-    // first lane of each item range: packed, or each range on a wave boundary (a wave then runs
-    // one element kind only)
-    const int L1 = P.aligned ? wave_align(ntri) : ntri;
-    const int L2 = L1 + (P.aligned ? wave_align(nedge) : nedge);
-    const int L3 = L2 + (P.aligned ? wave_align(ntet) : ntet);
-    const int L4 = L3 + (P.aligned ? wave_align(nspr) : nspr);
-    if (t < ntri) {
-        kind = 1;
-        const int4* r4 = reinterpret_cast<const int4*>(P.tri_rec) + 3 * (size_t)(tri_b + t);
-        r0 = r4[0];
-        r1 = r4[1];
-        r2 = r4[2];
-    } else if (t >= L1 && t < L1 + nedge) {
-        kind = 2;
-        const int k = t - L1;
-        const int4* r4 = reinterpret_cast<const int4*>(P.edge_rec) + 2 * (size_t)(edge_b + k);
-        r0 = r4[0];
-        r1 = r4[1];
-        meta = P.edge_meta[edge_b + k];
-    } else if (t >= L2 && t < L2 + ntet) {
-        kind = 3;
-        const int k = t - L2;
-        const int4* r4 = reinterpret_cast<const int4*>(P.tet_rec) + 4 * (size_t)(tet_b + k);
-        r0 = r4[0];
-        r1 = r4[1];
-        r2 = r4[2];
-        r3 = r4[3];
-        meta = P.tet_meta[tet_b + k];
-    } else if (t >= L3 && t < L3 + nspr) {
-        kind = 5;
-        const int4* r4 = reinterpret_cast<const int4*>(P.spr_rec) + 2 * (size_t)(spr_b + t - L3);
-        r0 = r4[0];
-        r1 = r4[1];
-    } else if (par_contacts && t >= L4 && t - L4 < ncont) {
-        kind = 4;
-        const int4* c4 = reinterpret_cast<const int4*>(P.cpack) + 4 * (size_t)(cbeg + t - L4);
-        r0 = c4[0];
-        r1 = c4[1];
-        r2 = c4[2];
-        r3 = c4[3];
-    }
-    V3 own_x0 = v3(0.0f, 0.0f, 0.0f), own_d = own_x0;
+    // ---- round trip 2
+    const int kind = item.y >> 12;  // vbd_layout::ItemKind
     const int own_v = vr.x;
-    const bool own_active = ((vr.w >> 16) & 1) != 0;
-    if (t < nv) {
-        const float m = P.mass[own_v];
-        float* a = s_acc + t * kComp;
+    const V3 x = ld3(q, id);
+    // previous positions of the whole list, or of the batch's own vertices (the list's first)
+    const V3 xp = ld3(P.q_prev, P.prev || t < nv ? id : __builtin_amdgcn_readfirstlane(id));
+    const float m = P.mass[own_v];
+    const V3 y = ld3(P.inertia, own_v);
+    const V3 own_d = ld3(P.disp, own_v);
+    int so = 0;
+    if constexpr (SELF)  // self-contact row bounds of the batch's color positions (consecutive positions)
+        if (P.has_self) so = P.so_off[v_begin + min(t, nv)];
+    if (t < nv) {  // the list starts with the batch's own vertices: id == own_v
+        float* a = s_acc + t * NC;
+        a[0] = (m * (y.x - x.x)) * P.dtr;
+        a[1] = (m * (y.y - x.y)) * P.dtr;
+        a[2] = (m * (y.z - x.z)) * P.dtr;
+        if constexpr (!FORCE_ONLY) {
+            const float md = m * P.dtr;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) a[c] = (m * (P.inertia[3 * own_v + c] - q[3 * own_v + c])) * dtr;
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) a[3 + 3 * r + c] = (m * dtr) * (r == c ? 1.0f : 0.0f);
-        own_x0 = ld3(P.q_prev, own_v);
-        own_d = ld3(P.disp, own_v);
+            for (int k = 3; k < NC; ++k) {
+                const int e = full_component<SYM>(k) - 3;
+                a[k] = md * (e % 4 == 0 ? 1.0f : 0.0f);
+            }
+        }
         s_row[t] = vr.y;
         s_nrow[t] = vr.z;
         s_nspr[t] = vr.w >> 17;
     }
     if (t <= nv) {
         s_cb[t] = cbt;
-        // self-contact row bounds of the batch's color positions (consecutive positions)
-        if (P.has_self) s_so[t] = P.so_off[b0.x + t];
+        if constexpr (SELF) s_so[t] = so;
     }
+    if (64 * wave < LIST) {
+        s_q[t] = make_float4(x.x, x.y, x.z, 0.0f);
+        s_p[t] = make_float4(xp.x, xp.y, xp.z, 0.0f);
+    }
+    __syncthreads();
 
-    // ---- round trip 3 + phase a: evaluate the lane's item
+    // ---- phase a: evaluate the lane's item
+    auto at = [&](int i) {
+        const float4 v = s_q[(item.x >> (8 * i)) & 0xff];
+        return v3(v.x, v.y, v.z);
+    };
+    auto prev = [&](int i) {
+        const float4 v = s_p[(item.x >> (8 * i)) & 0xff];
+        return v3(v.x, v.y, v.z);
+    };
+    // a packed contact of one of the batch's own vertices (edge/face records never get here: their
+    // contexts evaluate every entry in k_contact_rows)
+    auto contact = [&](float4 A, float4 B, float4 C, float4 D, V3& f, M3& h) {
+        const int l = __float_as_int(A.y) & 0xffff;
+        const float4 v = s_q[l], p = s_p[l];
+        eval_contact(v3(v.x, v.y, v.z), v3(p.x, p.y, p.z), v3(B.w, C.x, C.y), v3(C.z, C.w, D.x), v3(D.y, D.z, D.w),
+                     B.z, B.y, A.z, A.w, B.x, P.friction_epsilon, dt, f, h);
+    };
+    // contacts first, from the second wave on (the first has the batch's own vertices to look after)
+    for (int k = t >= 64 ? t - 64 : t + BLOCK - 64; k < npar; k += BLOCK) {
+        const float4* c4 = reinterpret_cast<const float4*>(P.cpack) + 4 * (size_t)(cbeg + k);
+        V3 fe;
+        M3 he;
+        contact(c4[0], c4[1], c4[2], c4[3], fe, he);
+        put_row<SYM, FORCE_ONLY>(s_rows + (nstatic + k) * NC, fe, he);  // contact rows follow the static rows
+    }
     if (kind != 0) {
         V3 fe = v3(0.0f, 0.0f, 0.0f);
         M3 he = mzero();
-        int row;
-        if (kind == 1) {
-            float4 pz = __builtin_bit_cast(float4, r1);
-            float4 mt = __builtin_bit_cast(float4, r2);
-            row = r0.w & 0xffff;
-            float pose[4] = {pz.x, pz.y, pz.z, pz.w};
-            eval_membrane(ld3(q, r0.x), ld3(q, r0.y), ld3(q, r0.z), P.q_prev, r0.x, r0.y, r0.z, pose, mt.x, mt.y,
-                          mt.z, mt.w, dt, r0.w >> 16, fe, he);
-        } else if (kind == 2) {
-            float4 pr = __builtin_bit_cast(float4, r1);
-            row = meta & 0xffff;
-            eval_bending(q, P.q_prev, r0.x, r0.y, r0.z, r0.w, pr.x, pr.y, pr.z, pr.w, dt, meta >> 16, fe, he);
-        } else if (kind == 3) {
-            float4 d0 = __builtin_bit_cast(float4, r1);
-            float4 d1 = __builtin_bit_cast(float4, r2);
-            float4 d2 = __builtin_bit_cast(float4, r3);
-            int ti[4] = {r0.x, r0.y, r0.z, r0.w};
-            float dm[9] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w, d2.x};
-            row = meta & 0xffff;
-            eval_tet(q, P.q_prev, ti, dm, d2.y, d2.z, d2.w, dt, meta >> 16, fe, he);
-        } else if (kind == 5) {
-            const float4 pr = __builtin_bit_cast(float4, r1);
-            row = r0.z & 0xffff;
-            spring_item(P, q, r0.x, r0.y, r0.z >> 16, r0.w, pr.x, pr.y, pr.z, dt, fe, he);
-        } else {
-            eval_contact_rec(P, q, cbeg + t - L4, __builtin_bit_cast(float4, r0), __builtin_bit_cast(float4, r1),
-                             __builtin_bit_cast(float4, r2), __builtin_bit_cast(float4, r3), dt, fe, he);
-            row = nstatic + (t - L4);  // contact rows follow the static rows
+        const int row = item.y & 0x1ff;
+        const int slot = (item.y >> 9) & 3;
+        if constexpr (CLOTH) {
+            if (kind == vbd_layout::kTri) {
+                const float4 D = __builtin_bit_cast(float4, w0), mt = __builtin_bit_cast(float4, w1);
+                eval_membrane(at(0), at(1), at(2), prev, D.x, D.y, D.z, D.w, __int_as_float(item.z), mt.x, mt.y, mt.z,
+                              mt.w, P.inv_dt, slot, fe, he);
+            } else if (kind == vbd_layout::kHinge) {
+                eval_bending(at(0), at(1), at(2), at(3), prev, __int_as_float(item.z), __int_as_float(item.w), kdl,
+                             (item.y >> 11) & 1, P.inv_dt, slot, fe, he);
+            }
         }
-        if constexpr (FORCE_ONLY)
-            store_force(s_rows + row * kComp, fe);
-        else
-            store_row(s_rows + row * kComp, fe, he);
-    }
-    // contacts beyond the lanes left after the static items (only when L4 + ncont > BLOCK)
-    const int npar = par_contacts ? ncont : 0;
-    for (int ci = BLOCK - L4 + t; ci < npar; ci += BLOCK) {
-        V3 fe;
-        M3 he;
-        eval_packed_contact(P, q, cbeg + ci, dt, fe, he);
-        if constexpr (FORCE_ONLY)
-            store_force(s_rows + (nstatic + ci) * kComp, fe);
-        else
-            store_row(s_rows + (nstatic + ci) * kComp, fe, he);
+        if constexpr (TET) {
+            if (kind == vbd_layout::kTet) {
+                const float4 d0 = __builtin_bit_cast(float4, w0), d1 = __builtin_bit_cast(float4, w1),
+                             d2 = __builtin_bit_cast(float4, w2);
+                const M3 Dm = {{{d0.x, d0.y, d0.z}, {d0.w, d1.x, d1.y}, {d1.z, d1.w, d2.x}}};
+                eval_tet(at(0), at(1), at(2), at(3), prev, Dm, d2.y, __int_as_float(item.z), __int_as_float(item.w),
+                         d2.z, d2.w, P.inv_dt, slot, fe, he);
+            }
+        }
+        if constexpr (SPRING) {
+            if (kind == vbd_layout::kSpring) {
+                if (item.z >= 0)
+                    load_row(P.spr_rows + kComp * (size_t)item.z, fe, he);
+                else
+                    eval_spring(at(0), at(1), prev(0), prev(1), __int_as_float(item.w), __int_as_float(w0.x),
+                                __int_as_float(w0.y), dt, slot, fe, he);
+            }
+        }
+        put_row<SYM, FORCE_ONLY>(s_rows + row * NC, fe, he);
     }
     __syncthreads();
 
     // ---- phase b
-    const int cs = t / kComp;
-    const int cc = t - cs * kComp;
-    if (cs < nv && (!FORCE_ONLY || cc < 3)) {
-        float acc = s_acc[cs * kComp + cc];
+    const int cs = t / NC;
+    const int cc = t - cs * NC;
+    if (cs < nv) {
+        float acc = s_acc[t];
         const int q0 = s_row[cs], q1 = q0 + s_nrow[cs];
         // the LDS reads of four rows are issued together; the additions stay serial, in row order
         int r = q0;
         for (; r + 4 <= q1; r += 4) {
-            const float a0 = s_rows[r * kComp + cc], a1 = s_rows[(r + 1) * kComp + cc];
-            const float a2 = s_rows[(r + 2) * kComp + cc], a3 = s_rows[(r + 3) * kComp + cc];
+            const float a0 = s_rows[r * NC + cc], a1 = s_rows[(r + 1) * NC + cc];
+            const float a2 = s_rows[(r + 2) * NC + cc], a3 = s_rows[(r + 3) * NC + cc];
             acc = acc + a0;
             acc = acc + a1;
             acc = acc + a2;
             acc = acc + a3;
         }
-        for (; r < q1; ++r) acc = acc + s_rows[r * kComp + cc];
+        for (; r < q1; ++r) acc = acc + s_rows[r * NC + cc];
         // contacts from zero -- their LDS rows, or, when they did not fit, evaluated here by each of
-        // the vertex's 12 lanes (component cc kept) -- then the vertex's spring rows and
+        // the vertex's lanes (component cc kept) -- then the vertex's spring rows and
         // self-contact rows continue that sum, which is added to the element sum
-        const int c0 = s_cb[cs], c1 = s_cb[cs + 1];
+        const int c0 = s_cb[cs], c1 = s_cb[cs + 1], fc12 = full_component<SYM>(cc);
         float ca = 0.0f;
         if (par_contacts) {
-            for (int r = c0; r < c1; ++r) ca = ca + s_rows[(nstatic + r) * kComp + cc];
+            for (int r = c0; r < c1; ++r) ca = ca + s_rows[(nstatic + r) * NC + cc];
         } else if (P.crows) {
-            ca = add_rows_in_order(ca, P.crows + (size_t)kComp * cbeg, c0, c1, cc);
+            ca = add_rows_in_order(ca, P.crows + (size_t)kComp * cbeg, c0, c1, fc12);
         } else {
             for (int r = c0; r < c1; ++r) {
                 V3 fc;
                 M3 hc;
                 eval_packed_contact(P, q, cbeg + r, dt, fc, hc);
-                ca = ca + row_component(fc, hc, cc);
+                ca = ca + row_component(fc, hc, fc12);
             }
         }
-        for (int r = q1, re = q1 + s_nspr[cs]; r < re; ++r) ca = ca + s_rows[r * kComp + cc];
-        if (P.has_self) ca = add_rows_in_order(ca, P.so_rows, s_so[cs], s_so[cs + 1], cc);
+        if constexpr (SPRING)
+            for (int r = q1, re = q1 + s_nspr[cs]; r < re; ++r) ca = ca + s_rows[r * NC + cc];
+        if constexpr (SELF)
+            if (P.has_self) ca = add_rows_in_order(ca, P.so_rows, s_so[cs], s_so[cs + 1], fc12);
         acc = acc + ca;
-        s_acc[cs * kComp + cc] = acc;
+        s_acc[t] = acc;
     }
     __syncthreads();
 
     // ---- phase c
+    const bool own_active = ((vr.w >> 16) & 1) != 0;
     if (t < nv) {
-        const float* a = s_acc + t * kComp;
-        V3 f = v3(a[0], a[1], a[2]);
-        M3 h;
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) h.m[i][j] = a[3 + 3 * i + j];
+        const float* a = s_acc + t * NC;
+        const V3 f = v3(a[0], a[1], a[2]);
         if constexpr (FORCE_ONLY) {
             if (own_live) st3(g_out, own_v, own_active ? f : v3(0.0f, 0.0f, 0.0f));
         } else {
-            if (own_live) finish_vertex(P, q, own_v, own_active, own_x0, own_d, f, h, dt, mode, g_out);
+            M3 h;
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int j = 0; j < 3; ++j) {
+                    const int lo = i < j ? i : j, hi = i < j ? j : i;
+                    h.m[i][j] = a[SYM ? 3 + lo * (5 - lo) / 2 + hi : 3 + 3 * i + j];
+                }
+            if (own_live) finish_vertex(P, q, own_v, own_active, xp, own_d, f, h, dt, mode, g_out);
         }
     }
 }
 
-// Generic color pass for vertices with more than 256 element items: one
+// Generic color pass for vertices with more than 256 element items (or neighbours): one
 // vertex per work-group, the CSR walked in chunks of 256 items, same
 // canonical summation order; contacts from the per-particle lists.
 __global__ __launch_bounds__(kBlock) void k_solve_generic(KParams P, float* __restrict__ q, int slow_base, float dt,
@@ -1174,7 +1232,7 @@ __global__ __launch_bounds__(kBlock) void k_solve_generic(KParams P, float* __re
     const int v = P.color_particles[P.slow_pos[slow_base + blockIdx.x]];
     if (P.w_active && P.w_active[P.p_world[v]] == 0) return;  // frozen world (uniform)
     const bool active = particle_active(P, v);
-    const float dtr = 1.0f / (dt * dt);
+    const float dtr = P.dtr;
     if (t == 0) {
         int nt = 0, ne = 0, nk = 0, bt = 0, be = 0, bk = 0;
         if (active) {
@@ -1217,25 +1275,39 @@ __global__ __launch_bounds__(kBlock) void k_solve_generic(KParams P, float* __re
                 const float* mat = P.tri_mat + 5 * tri;
                 if (mat[0] > 0.0f || mat[1] > 0.0f) {
                     const int* ti = P.tri_idx + 3 * tri;
-                    eval_membrane(ld3(q, ti[0]), ld3(q, ti[1]), ld3(q, ti[2]), P.q_prev, ti[0], ti[1], ti[2],
-                                  P.tri_pose + 4 * tri, P.tri_area[tri], mat[0], mat[1], mat[2], dt, slot, fe, he);
+                    const float* D = P.tri_pose + 4 * tri;
+                    eval_membrane(ld3(q, ti[0]), ld3(q, ti[1]), ld3(q, ti[2]),
+                                  [&](int i) { return ld3(P.q_prev, ti[i]); }, D[0], D[1], D[2], D[3],
+                                  P.tri_area[tri], mat[0], lame_sum(mat[0], mat[1]), rest_ratio(mat[0], mat[1]),
+                                  mat[2], P.inv_dt, slot, fe, he);
                 }
             } else if (k < s_cnt[0] + s_cnt[1]) {
                 int base = s_beg[1] + 2 * (k - s_cnt[0]);
                 int ed = P.adj_edge[base], slot = P.adj_edge[base + 1];
                 float ke = P.edge_bend[2 * ed];
-                if (ke > 0.0f) {
-                    const int* ei = P.edge_idx + 4 * ed;
-                    eval_bending(q, P.q_prev, ei[0], ei[1], ei[2], ei[3], P.edge_rest_angle[ed], P.edge_rest_len[ed],
-                                 ke, P.edge_bend[2 * ed + 1], dt, slot, fe, he);
+                const int* ei = P.edge_idx + 4 * ed;
+                if (ke > 0.0f && ei[0] != -1 && ei[1] != -1) {
+                    const float kd = P.edge_bend[2 * ed + 1], len = P.edge_rest_len[ed];
+                    eval_bending(ld3(q, ei[0]), ld3(q, ei[1]), ld3(q, ei[2]), ld3(q, ei[3]),
+                                 [&](int i) { return ld3(P.q_prev, ei[i]); }, P.edge_rest_angle[ed], ke * len,
+                                 kd * len, kd > 0.0f, P.inv_dt, slot, fe, he);
                 }
             } else {
                 int base = s_beg[2] + 2 * (k - s_cnt[0] - s_cnt[1]);
                 int tet = P.adj_tet[base], slot = P.adj_tet[base + 1];
                 const float* mat = P.tet_mat + 3 * tet;
-                if (mat[0] > 0.0f || mat[1] > 0.0f)
-                    eval_tet(q, P.q_prev, P.tet_idx + 4 * tet, P.tet_pose + 9 * tet, mat[0], mat[1], mat[2], dt, slot,
-                             fe, he);
+                if (mat[0] > 0.0f || mat[1] > 0.0f) {
+                    const int* ti = P.tet_idx + 4 * tet;
+                    const float* dm = P.tet_pose + 9 * tet;
+                    M3 Dm;
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+#pragma unroll
+                        for (int j = 0; j < 3; ++j) Dm.m[i][j] = dm[3 * i + j];
+                    eval_tet(ld3(q, ti[0]), ld3(q, ti[1]), ld3(q, ti[2]), ld3(q, ti[3]),
+                             [&](int i) { return ld3(P.q_prev, ti[i]); }, Dm, 1.0f / (mdet(Dm) * 6.0f), mat[0],
+                             lame_sum(mat[0], mat[1]), rest_ratio(mat[0], mat[1]), mat[2], P.inv_dt, slot, fe, he);
+                }
             }
             store_row(s_item + t * kComp, fe, he);
         }
@@ -2212,11 +2284,13 @@ struct VbdContext {
     // pass layout on the device
     int* lay_batch = nullptr;
     int* lay_vert = nullptr;
+    int* lay_item = nullptr;
+    int* lay_list = nullptr;
     int* lay_tri = nullptr;
-    int* lay_edge = nullptr;
-    int* lay_edge_meta = nullptr;
+    int* lay_hinge_damp = nullptr;
     int* lay_tet = nullptr;
-    int* lay_tet_meta = nullptr;
+    vbd_layout::PassShape shape;  // lane ranges and strides of the uploaded layout
+    int variant = 0;              // k_solve_fast's element kinds (PassKinds)
     int* lay_slow = nullptr;
     int* lay_spr = nullptr;
     int* lay_pre = nullptr;
@@ -2280,8 +2354,8 @@ std::string h2d(T** dst, const std::vector<T>& src) {
 }
 
 void free_layout(VbdContext* c) {
-    for (int** p : {&c->lay_batch, &c->lay_vert, &c->lay_tri, &c->lay_edge, &c->lay_edge_meta, &c->lay_tet,
-                    &c->lay_tet_meta, &c->lay_slow, &c->bat_cinfo, &c->bat_coff, &c->lay_spr, &c->lay_pre,
+    for (int** p : {&c->lay_batch, &c->lay_vert, &c->lay_item, &c->lay_list, &c->lay_tri, &c->lay_hinge_damp,
+                    &c->lay_tet, &c->lay_slow, &c->bat_cinfo, &c->bat_coff, &c->lay_spr, &c->lay_pre,
                     &c->lay_slow_spr_off, &c->lay_slow_spr, &c->batch_list}) {
         hipFree(*p);
         *p = nullptr;
@@ -2364,18 +2438,18 @@ int32_t build_layout(VbdContext* c) {
     err = vbd_layout::build_pass_layout(hm, L, c->block, c->block / kComp, c->aligned != 0);
     if (!err.empty()) return fail(VBD_ERR_ARG, "vbd_create: " + err);
     const std::pair<int**, std::vector<int32_t>*> arrays[] = {
-        {&c->lay_batch, &L.batch_blk}, {&c->lay_vert, &L.vert_rec}, {&c->lay_tri, &L.tri_rec},
-        {&c->lay_edge, &L.edge_rec}, {&c->lay_edge_meta, &L.edge_meta}, {&c->lay_tet, &L.tet_rec},
-        {&c->lay_tet_meta, &L.tet_meta}, {&c->lay_slow, &L.slow_pos}, {&c->lay_spr, &L.spr_rec},
+        {&c->lay_batch, &L.batch_blk}, {&c->lay_vert, &L.vert_rec}, {&c->lay_item, &L.item_rec},
+        {&c->lay_list, &L.list}, {&c->lay_tri, &L.tri_rec}, {&c->lay_hinge_damp, &L.hinge_damp},
+        {&c->lay_tet, &L.tet_rec}, {&c->lay_slow, &L.slow_pos}, {&c->lay_spr, &L.spr_rec},
         {&c->lay_pre, &L.pre_item}, {&c->lay_slow_spr_off, &L.slow_spr_off}, {&c->lay_slow_spr, &L.slow_spr}};
     std::vector<size_t> sizes;
     for (const auto& pr : arrays) sizes.push_back(pr.second->size());
     // A rebuild whose layout has the same shape (array sizes, per-color batch / generic / pre-row
-    // ranges, batch width) -- the case of material or rest-data edits -- rewrites the existing
+    // ranges, batch width, lane ranges) -- the case of material or rest-data edits -- rewrites the existing
     // device buffers, so every pointer and launch shape a captured graph holds stays valid.
     const bool in_place = c->lay_batch != nullptr && sizes == c->lay_sizes && L.fast_color_off == c->fast_color_off &&
                           L.slow_color_off == c->slow_color_off && L.pre_color_off == c->pre_color_off &&
-                          L.max_v == c->max_v && L.blk_words == c->blk_words;
+                          L.max_v == c->max_v && L.blk_words == c->blk_words && L.shape == c->shape;
     if (in_place) {
         for (const auto& pr : arrays) {
             if (pr.second->empty()) continue;
@@ -2447,11 +2521,30 @@ int32_t build_layout(VbdContext* c) {
     k.bat_cinfo = c->bat_cinfo;
     k.bat_coff = c->bat_coff;
     k.vert_rec = c->lay_vert;
+    k.item_rec = c->lay_item;
+    k.list = c->lay_list;
     k.tri_rec = c->lay_tri;
-    k.edge_rec = c->lay_edge;
-    k.edge_meta = c->lay_edge_meta;
+    k.hinge_damp = reinterpret_cast<const float*>(c->lay_hinge_damp);
     k.tet_rec = c->lay_tet;
-    k.tet_meta = c->lay_tet_meta;
+    c->shape = L.shape;
+    k.tri_hi = L.shape.tri.hi;
+    k.hinge_lo = L.shape.hinge.lo;
+    k.hinge_hi = L.shape.hinge.hi;
+    k.tet_lo = L.shape.tet.lo;
+    k.tet_hi = L.shape.tet.hi;
+    k.spr_lo = L.shape.spring.lo;
+    k.spr_hi = L.shape.spring.hi;
+    k.list_stride = L.shape.list_stride;
+    k.hinge_damped = L.shape.hinge_damped ? 1 : 0;
+    k.prev = L.shape.prev ? 1 : 0;
+    {
+        const bool cloth = L.shape.tri.count() + L.shape.hinge.count() > 0;
+        const bool tet = L.shape.tet.count() > 0, spring = L.shape.spring.count() > 0;
+        if (c->params.self_contact || (tet && (cloth || spring)))
+            c->variant = kAllKinds;
+        else
+            c->variant = tet ? kTetKinds : (spring ? kClothSpringKinds : kClothKinds);
+    }
     k.slow_pos = c->lay_slow;
     k.has_spring = m->spring_count > 0;
     k.spring_idx = m->spring_indices;
@@ -2463,7 +2556,6 @@ int32_t build_layout(VbdContext* c) {
     k.spr_rows = c->spr_rows;
     k.slow_spr_off = c->lay_slow_spr_off;
     k.slow_spr = c->lay_slow_spr;
-    k.aligned = c->aligned;
     return VBD_OK;
 }
 
@@ -2735,6 +2827,28 @@ std::string noalloc_scratch(int32_t** out) {
     return std::string();
 }
 
+template <int BLOCK, int WAVES, bool FORCE_ONLY>
+void launch_kinds(VbdContext* c, hipStream_t s, int b0, int nb, float* q, float dt, int mode, float* g) {
+    const dim3 grid(nb), block(BLOCK);
+    switch (c->variant) {
+    case kClothKinds:
+        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, kClothKinds, FORCE_ONLY>), grid, block, 0, s, q, b0, nb, dt,
+                           mode, g, c->kp);
+        break;
+    case kClothSpringKinds:
+        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, kClothSpringKinds, FORCE_ONLY>), grid, block, 0, s, q, b0, nb,
+                           dt, mode, g, c->kp);
+        break;
+    case kTetKinds:
+        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, kTetKinds, FORCE_ONLY>), grid, block, 0, s, q, b0, nb, dt,
+                           mode, g, c->kp);
+        break;
+    default:
+        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, kAllKinds, FORCE_ONLY>), grid, block, 0, s, q, b0, nb, dt,
+                           mode, g, c->kp);
+    }
+}
+
 // Soft contacts in pair order from per-tile hit counts (count, scan of the tile counts, write).
 int32_t launch_collide_tiles(const ColParams& cp, hipStream_t s, const float* q, float margin, int* tiles_dev,
                              const VbdContactsOut& out) {
@@ -2894,7 +3008,24 @@ int32_t vbd_create(const VbdModelDesc* m, const VbdSolverParams* prm, VbdContext
     k.friction_epsilon = prm->friction_epsilon;
     k.fp64_ill = prm->fp64_ill_conditioned;
     k.write_q = 1;
-    int32_t rc = build_layout(c);
+    // Cloth starts with 192-lane work-groups and wave-aligned items: a regular mesh fills one wave with triangles,
+    // one with the hinges opposite its vertices and one with those on them, ten vertices a batch (pass of a
+    // 256x256 cloth 8.7 us, 9.5 us with 256 packed lanes; of a 32x32 one 4.3 and 5.2 us).  A mesh with vertices too
+    // large for that shape, tets (16.3 us either way for 128 cubes) and springs (a fourth range) start with 256
+    // packed lanes.
+    int32_t rc = VBD_OK;
+    bool narrow = m->tri_count > 0 && m->tet_count == 0 && m->spring_count == 0;
+    if (narrow) {
+        c->block = 192;
+        c->aligned = 1;
+        rc = build_layout(c);
+        narrow = c->slow_color_off.empty() || c->slow_color_off.back() == 0;
+    }
+    if (rc == VBD_OK && !narrow) {
+        c->block = 256;
+        c->aligned = 0;
+        rc = build_layout(c);
+    }
     if (rc == VBD_OK && prm->self_contact) rc = setup_self(c, m, prm);
     if (rc) {
         std::string msg = g_last_error;
@@ -3124,31 +3255,33 @@ int32_t vbd_forward(VbdContext* c, void* stream, float* q, const float* qd, cons
 }
 
 namespace {
+// the launch's dt, inverted once here instead of on every lane (same IEEE division)
+void set_dt(VbdContext* c, float dt) {
+    c->kp.inv_dt = 1.0f / dt;
+    c->kp.dtr = 1.0f / (dt * dt);
+}
+
 // mode 0 solves; mode 1 writes the assembled force g: by the force-only instantiations when
 // force_only (the residual), else by the solving kernels themselves (the autotuner times those)
 int32_t launch_fast(VbdContext* c, hipStream_t s, int b0, int nb, float* q, float dt, int mode, float* g,
                     bool force_only = false) {
     if (mode == 1 && force_only) {
-        if (c->block == 128) {
-            hipLaunchKernelGGL((k_solve_fast<128, 1, true>), dim3(nb), dim3(128), 0, s, c->kp, q, b0, nb, dt, mode, g);
-        } else if (c->block == 192) {
-            hipLaunchKernelGGL((k_solve_fast<192, 1, true>), dim3(nb), dim3(192), 0, s, c->kp, q, b0, nb, dt, mode, g);
-        } else {
-            hipLaunchKernelGGL((k_solve_fast<256, 1, true>), dim3(nb), dim3(256), 0, s, c->kp, q, b0, nb, dt, mode, g);
-        }
-        VBD_LAUNCH_CHECK("k_solve_fast");
-        return VBD_OK;
-    }
-    if (c->block == 128) {
-        hipLaunchKernelGGL((k_solve_fast<128, 1>), dim3(nb), dim3(128), 0, s, c->kp, q, b0, nb, dt, mode, g);
+        if (c->block == 128)
+            launch_kinds<128, 1, true>(c, s, b0, nb, q, dt, mode, g);
+        else if (c->block == 192)
+            launch_kinds<192, 1, true>(c, s, b0, nb, q, dt, mode, g);
+        else
+            launch_kinds<256, 1, true>(c, s, b0, nb, q, dt, mode, g);
+    } else if (c->block == 128) {
+        launch_kinds<128, 1, false>(c, s, b0, nb, q, dt, mode, g);
     } else if (c->block == 192 && c->waves == 7) {
-        hipLaunchKernelGGL((k_solve_fast<192, 7>), dim3(nb), dim3(192), 0, s, c->kp, q, b0, nb, dt, mode, g);
+        launch_kinds<192, 7, false>(c, s, b0, nb, q, dt, mode, g);
     } else if (c->block == 192) {
-        hipLaunchKernelGGL((k_solve_fast<192, 1>), dim3(nb), dim3(192), 0, s, c->kp, q, b0, nb, dt, mode, g);
+        launch_kinds<192, 1, false>(c, s, b0, nb, q, dt, mode, g);
     } else if (c->waves == 7) {
-        hipLaunchKernelGGL((k_solve_fast<256, 7>), dim3(nb), dim3(256), 0, s, c->kp, q, b0, nb, dt, mode, g);
+        launch_kinds<256, 7, false>(c, s, b0, nb, q, dt, mode, g);
     } else {
-        hipLaunchKernelGGL((k_solve_fast<256, 1>), dim3(nb), dim3(256), 0, s, c->kp, q, b0, nb, dt, mode, g);
+        launch_kinds<256, 1, false>(c, s, b0, nb, q, dt, mode, g);
     }
     VBD_LAUNCH_CHECK("k_solve_fast");
     return VBD_OK;
@@ -3169,6 +3302,7 @@ int32_t launch_contact_rows(VbdContext* c, hipStream_t s, int p_lo, int p_hi, co
 }
 
 int32_t launch_color(VbdContext* c, hipStream_t s, int color, float* q, float dt, int mode, float* g) {
+    set_dt(c, dt);
     int32_t rc0 = launch_spring_rows(c, s, c->pre_color_off[color], c->pre_color_off[color + 1], q, dt);
     if (rc0) return rc0;
     rc0 = launch_contact_rows(c, s, c->color_offsets[color], c->color_offsets[color + 1], q, dt);
@@ -3197,6 +3331,7 @@ int32_t launch_color(VbdContext* c, hipStream_t s, int color, float* q, float dt
 // The force residual assembled by the color-pass kernels' force-only instantiations (one launch
 // over every batch) and, for vertices with more than 256 items, the generic kernel.
 int32_t residual_by_passes(VbdContext* c, hipStream_t s, const float* q, float dt, float* g) {
+    set_dt(c, dt);
     int32_t rc0 = launch_spring_rows(c, s, 0, c->pre_color_off.back(), q, dt);
     if (rc0) return rc0;
     rc0 = launch_contact_rows(c, s, 0, c->model.particle_count, q, dt);

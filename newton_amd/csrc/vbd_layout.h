@@ -3,19 +3,35 @@
 // For every color, the color's vertices (in color-group order) are cut into
 // batches: runs of at most max_v consecutive vertices whose element counts sum
 // to at most cap (the work-group shape: 256 lanes -> cap 256, max_v 21; 128
-// lanes -> cap 128, max_v 10).  A batch is one workgroup.  Its element
-// contributions are stored as packed records in evaluation order -- all
-// triangle items of the batch, then all bending-edge items, then all tet
-// items -- each carrying the canonical row (the position of that contribution
-// in its vertex's serial sum: the vertex's triangles in CSR order, then its
-// edges, then its tets) and the vertex's local slot in the element.
+// lanes -> cap 128, max_v 10) and whose elements touch at most cap distinct
+// vertices.  A batch is one workgroup, and lane t evaluates item t: all
+// triangle items of the batch, then all bending-edge items (first those whose
+// vertex lies opposite the hinge edge, then those on it: the two run different
+// code), then all tet items, then the springs, each carrying the canonical row (the position of that
+// contribution in its vertex's serial sum: the vertex's triangles in CSR order,
+// then its edges, then its tets) and the vertex's local slot in the element.
+//
+// Storage is by fixed slots, so a lane finds its item, and its share of the
+// batch's vertex list, from the batch number alone, in the same round trip as
+// the batch header: item t of batch b is item_rec[b * cap + t]; the wider part
+// of a triangle (tet, spring) record sits in an array with one slot for each
+// lane that holds that kind in any batch ([tri_lo, tri_hi) and so on).  Slots
+// that a batch does not use are never read.  Items name their vertices by 8-bit
+// slots of the batch's vertex list (the batch's own vertices first), whose
+// positions the work-group stages in LDS: a hinge item is 16 bytes, and a
+// position is gathered once per batch instead of once per element.
+//
+// Values of an element that no step changes are evaluated here once, in single
+// precision and the kernels' expression order: lambda + mu, the rest ratio
+// alpha = 1 + mu / (lambda + mu), a tet's rest volume, stiffness * rest length.
 //
 // Elements the reference's solve skips are left out: triangles and tets with
 // mu <= 0 and lambda <= 0, edges with ke <= 0 (particle_vbd_kernels.py:2636,
 // :2658, :2679), and boundary hinges (o0 or o1 == -1), whose contribution is
 // an exact zero (:682-683).  Inactive particles (flag bit 0 clear or mass 0)
-// get no items.  A vertex with more than cap items goes to the "slow"
-// list, handled by the generic kernel that walks the CSR in chunks.
+// get no items.  A vertex with more than cap items, or whose elements touch
+// more than list_cap(cap) vertices, goes to the "slow" list, handled by the generic
+// kernel that walks the CSR in chunks.
 //
 // Springs (particle_vbd_kernels.py:1733-1783) join the batch as items of their
 // own: each active endpoint of a spring gets one item, in spring-index order
@@ -26,8 +42,11 @@
 // ("pre items") and the pass item only points at its row.
 #pragma once
 
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <string>
 #include <vector>
 
 namespace vbd_layout {
@@ -36,17 +55,27 @@ constexpr int kLayoutCap = 256;  // static items (rows) per batch of the 256-lan
 constexpr int kLayoutMaxV = 21;  // vertices per batch of the 256-lane shape (12 component lanes each)
 
 // record widths in 32-bit words
-constexpr int kTriWords = 12;   // i0 i1 i2 meta | D00 D01 D10 D11 | area mu lambda kd
-constexpr int kEdgeWords = 8;   // o0 o1 v0 v1 | rest_angle rest_length ke kd      (+ edge_meta)
-constexpr int kTetWords = 16;   // i0 i1 i2 i3 | Dm^-1 (9) | mu lambda kd         (+ tet_meta)
-constexpr int kSpringWords = 8; // v0 v1 (row | endpoint << 16) pre_row | rest ke kd 0
-constexpr int kBatchWords = 12; // vbegin nv tri_begin ntri edge_begin nedge tet_begin ntet spr_begin nspr 0 0
-constexpr int kVertWords = 4;   // v row_start nrows (local | active << 16 | nsprings << 17)
+constexpr int kItemWords = 4;    // vertex slots (4 x 8 bits) | item_meta | two words by kind:
+                                 //   triangle: area -   hinge: rest_angle ke*rest_length
+                                 //   tet: mu lambda+mu  spring: pre_row rest_length
+constexpr int kTriWords = 8;     // D00 D01 D10 D11 | mu lambda+mu alpha kd
+constexpr int kTetWords = 12;    // Dm^-1 (9) rest_volume alpha kd
+constexpr int kSpringWords = 2;  // ke kd
+constexpr int kBatchWords = 4;   // vbegin nv static_rows 0
+constexpr int kVertWords = 4;    // v row_start nrows (local | active << 16 | nsprings << 17)
+// Distinct vertices of a batch: its own and their elements' others (a regular cloth's batch has 7 to 9 for each
+// of its own, so the lanes fill first); the work-group stages that many positions in LDS, and a smaller bound
+// lets more work-groups share a CU.
+constexpr int list_cap(int cap) { return cap <= 192 ? 128 : 192; }
 // batch block: header (kBatchWords) then max_v vertex records (unused ones zero),
 // fixed size so a workgroup reads its header and vertex records in one round trip
 inline int block_words(int max_v) { return kBatchWords + max_v * kVertWords; }  // a multiple of 4 words
 
-inline int32_t meta(int row, int slot) { return (int32_t)(row | (slot << 16)); }
+enum ItemKind { kNone = 0, kTri = 1, kHinge = 2, kTet = 3, kSpring = 5 };
+// row (9 bits) | slot in the element << 9 (2 bits) | damped << 11 | kind << 12
+inline int32_t item_meta(int row, int slot, bool damped, int kind) {
+    return (int32_t)(row | (slot << 9) | ((damped ? 1 : 0) << 11) | (kind << 12));
+}
 
 struct HostModel {
     int N = 0, T = 0, E = 0, K = 0;
@@ -63,15 +92,47 @@ struct HostModel {
     std::vector<float> spring_rest, spring_ke, spring_kd;
 };
 
+// Lanes [lo, hi) that hold one kind of item in any batch (empty when lo == hi).
+struct LaneRange {
+    int lo = 0, hi = 0;
+    int count() const { return hi - lo; }
+    void cover(int b, int e) {
+        if (e <= b) return;
+        if (hi == lo) {
+            lo = b;
+            hi = e;
+        } else {
+            lo = std::min(lo, b);
+            hi = std::max(hi, e);
+        }
+    }
+    bool operator==(const LaneRange& o) const { return lo == o.lo && hi == o.hi; }
+};
+
+// What a launch is given besides the arrays; equal shapes may be exchanged under a captured graph.
+struct PassShape {
+    LaneRange tri, hinge, tet, spring;
+    int list_stride = 0;       // entries of a batch's vertex list
+    bool hinge_damped = false; // some hinge has kd > 0 (hinge_damp is read)
+    bool prev = false;         // some item reads previous positions (damping, springs)
+    bool operator==(const PassShape& o) const {
+        return tri == o.tri && hinge == o.hinge && tet == o.tet && spring == o.spring &&
+               list_stride == o.list_stride && hinge_damped == o.hinge_damped && prev == o.prev;
+    }
+};
+
 struct PassLayout {
     std::vector<int32_t> fast_color_off;  // [C+1] into batch records
     std::vector<int32_t> slow_color_off;  // [C+1] into slow_pos
     std::vector<int32_t> batch_blk;       // [B * block_words(max_v)]: header + vertex records
     int cap = kLayoutCap, max_v = kLayoutMaxV, blk_words = block_words(kLayoutMaxV);
+    PassShape shape;
     std::vector<int32_t> vert_rec;        // [N * kVertWords], indexed by color position
-    std::vector<int32_t> tri_rec, edge_rec, edge_meta, tet_rec, tet_meta;
+    std::vector<int32_t> item_rec;        // [B * cap * kItemWords]
+    std::vector<int32_t> list;            // [B * list_stride] vertex list of each batch, its first again past its end
+    std::vector<int32_t> tri_rec, tet_rec, spr_rec;  // [B * range.count() * words]
+    std::vector<int32_t> hinge_damp;      // [B * hinge.count()] kd * rest_length (float bits)
     std::vector<int32_t> slow_pos;        // color positions of oversized vertices
-    std::vector<int32_t> spr_rec;         // [*, kSpringWords] spring items of the batches
     std::vector<int32_t> pre_item;        // [P, 2] (spring, endpoint) of same-color spring items
     std::vector<int32_t> pre_color_off;   // [C+1] into pre_item
     std::vector<int32_t> slow_spr_off;    // [slow + 1] into slow_spr
@@ -85,10 +146,23 @@ inline int32_t fbits(float f) {
     return i;
 }
 
-// Builds the layout; returns an empty string or an error message.
+// lambda + mu and the rest ratio alpha of a stable Neo-Hookean element (particle_vbd_kernels.py:76-292, :502-632)
+inline float lame_sum(float mu, float lambda) { return lambda + mu; }
+inline float rest_ratio(float mu, float lambda) {
+    const float l_nh = lame_sum(mu, lambda);
+    const float l_safe = (l_nh < 0.0f ? -1.0f : 1.0f) * std::fmax(std::fabs(l_nh), 1.0e-6f);
+    return 1.0f + mu / l_safe;
+}
+// 1 / (6 det Dm^-1), determinant as row0 . (row1 x row2)
+inline float rest_volume(const float* m) {
+    const float cx = m[4] * m[8] - m[5] * m[7], cy = m[5] * m[6] - m[3] * m[8], cz = m[3] * m[7] - m[4] * m[6];
+    return 1.0f / ((m[0] * cx + m[1] * cy + m[2] * cz) * 6.0f);
+}
+
 // Lanes an item range takes when ranges start on wave (64-lane) boundaries.
 inline int wave_align(int n) { return (n + 63) & ~63; }
 
+// Builds the layout; returns an empty string or an error message.
 // aligned: each kind's items start on a wave boundary of the work-group (a wave then evaluates one
 // kind only); the batch's lane budget counts the padded ranges.
 inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap = kLayoutCap,
@@ -128,16 +202,19 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
         for (int p = off[v]; p < off[v + 1]; p += 2) c += ok[vals[p]] ? 1 : 0;
         return c;
     };
-    std::vector<int32_t> ntri((size_t)N, 0), nedge((size_t)N, 0), ntet((size_t)N, 0), nspr((size_t)N, 0);
+    // hinges by the vertex's place: opposite the edge (slots 0, 1) or on it (slots 2, 3)
+    std::vector<int32_t> ntri((size_t)N, 0), nopp((size_t)N, 0), nedge((size_t)N, 0), ntet((size_t)N, 0), nspr((size_t)N, 0);
     for (int v = 0; v < N; ++v) {
         if (!active[v]) continue;
         if (m.T > 0) ntri[v] = count_ok(m.adj_tri, m.adj_tri_off, tri_ok, v);
-        if (m.E > 0) nedge[v] = count_ok(m.adj_edge, m.adj_edge_off, edge_ok, v);
+        if (m.E > 0) {
+            nedge[v] = count_ok(m.adj_edge, m.adj_edge_off, edge_ok, v);
+            for (int p = m.adj_edge_off[v]; p < m.adj_edge_off[v + 1]; p += 2)
+                nopp[v] += edge_ok[m.adj_edge[p]] && m.adj_edge[p + 1] < 2;
+        }
         if (m.K > 0) ntet[v] = count_ok(m.adj_tet, m.adj_tet_off, tet_ok, v);
         nspr[v] = vs_off[v + 1] - vs_off[v];
     }
-    auto nitems = [&](int v) { return ntri[v] + nedge[v] + ntet[v] + nspr[v]; };
-
     L = PassLayout();
     L.cap = cap;
     L.max_v = max_v;
@@ -164,18 +241,76 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
         }
     }
     L.pre_color_off[C] = (int32_t)(L.pre_item.size() / 2);
-    std::vector<int> rows;
+    // fn(kind, element, slot, vertices of the element, their count) over v's items in canonical order
+    auto for_items = [&](int v, auto&& fn) {
+        if (!active[v]) return;
+        if (m.T > 0)
+            for (int p = m.adj_tri_off[v]; p < m.adj_tri_off[v + 1]; p += 2)
+                if (tri_ok[m.adj_tri[p]]) fn(kTri, m.adj_tri[p], m.adj_tri[p + 1], &m.tri_idx[3 * (size_t)m.adj_tri[p]], 3);
+        if (m.E > 0)
+            for (int p = m.adj_edge_off[v]; p < m.adj_edge_off[v + 1]; p += 2)
+                if (edge_ok[m.adj_edge[p]])
+                    fn(kHinge, m.adj_edge[p], m.adj_edge[p + 1], &m.edge_idx[4 * (size_t)m.adj_edge[p]], 4);
+        if (m.K > 0)
+            for (int p = m.adj_tet_off[v]; p < m.adj_tet_off[v + 1]; p += 2)
+                if (tet_ok[m.adj_tet[p]]) fn(kTet, m.adj_tet[p], m.adj_tet[p + 1], &m.tet_idx[4 * (size_t)m.adj_tet[p]], 4);
+        for (int p = vs_off[v]; p < vs_off[v + 1]; ++p)
+            fn(kSpring, p, vs_item[p] & 1, &m.spring_idx[2 * (size_t)(vs_item[p] >> 1)], 2);
+    };
+
+    // lane ranges of a batch: triangles, opposite hinges, edge hinges, tets, springs
+    constexpr int kLanes = 5;
+
+    // ---- the batches: greedy runs of a color's vertices that fit one work-group
+    struct Batch {
+        int vb, nv;
+        int n[kLanes];     // items of each lane range
+        int list_begin;    // into L.list while the runs are found
+        int list_count;
+    };
+    std::vector<Batch> batches;
+    std::vector<int32_t> lists;                       // vertex lists, one after another
+    std::vector<int32_t> stamp((size_t)N, -1), slot_of((size_t)N, 0);
+    PassShape& sh = L.shape;
+    auto align = [&](int n) { return aligned ? wave_align(n) : n; };
     for (int c = 0; c < C; ++c) {
-        L.fast_color_off[c] = (int32_t)(L.batch_blk.size() / L.blk_words);
+        L.fast_color_off[c] = (int32_t)batches.size();
         L.slow_color_off[c] = (int32_t)L.slow_pos.size();
         int k = m.color_off[c];
         const int kend = m.color_off[c + 1];
         while (k < kend) {
-            int v0 = m.color_particles[k];
-            int items0 = nitems(v0);
-            const int lanes0 = wave_align(ntri[v0]) + wave_align(nedge[v0]) + wave_align(ntet[v0]) +
-                               wave_align(nspr[v0]);
-            if (items0 > cap || (aligned && lanes0 > cap)) {  // oversized vertex: generic kernel
+            const int id = (int)batches.size();
+            Batch b{};
+            b.vb = k;
+            b.list_begin = (int)lists.size();
+            std::vector<int32_t> seen;  // distinct vertices so far (own and neighbours)
+            auto meet = [&](int v) {
+                if (stamp[v] == id) return;
+                stamp[v] = id;
+                seen.push_back(v);
+            };
+            while (k < kend && b.nv < max_v) {
+                const int v = m.color_particles[k];
+                const int add[kLanes] = {ntri[v], nopp[v], nedge[v] - nopp[v], ntet[v], nspr[v]};
+                int lanes = 0;
+                for (int i = 0; i < kLanes; ++i) lanes += align(b.n[i] + add[i]);
+                if (lanes > cap) break;
+                const size_t before = seen.size();
+                meet(v);
+                for_items(v, [&](int, int, int, const int32_t* e, int n) {
+                    for (int i = 0; i < n; ++i) meet(e[i]);
+                });
+                if ((int)seen.size() > list_cap(cap)) {
+                    for (size_t i = before; i < seen.size(); ++i) stamp[seen[i]] = -1;
+                    seen.resize(before);
+                    break;
+                }
+                for (int i = 0; i < kLanes; ++i) b.n[i] += add[i];
+                ++b.nv;
+                ++k;
+            }
+            if (b.nv == 0) {  // oversized vertex: generic kernel
+                const int v0 = m.color_particles[k];
                 L.slow_pos.push_back(k);
                 if (active[v0])
                     for (int p = vs_off[v0]; p < vs_off[v0 + 1]; ++p) {
@@ -186,139 +321,112 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
                 ++k;
                 continue;
             }
-            // greedy run of vertices that fit one workgroup
-            int vb = k, nv = 0, items = 0, kt = 0, ke = 0, kk = 0, ks = 0;
-            while (k < kend && nv < max_v) {
-                int v = m.color_particles[k];
-                int it = nitems(v);
-                if (it > cap || items + it > cap) break;
-                if (aligned && active[v]) {
-                    const int lanes = wave_align(kt + ntri[v]) + wave_align(ke + nedge[v]) +
-                                      wave_align(kk + ntet[v]) + wave_align(ks + nspr[v]);
-                    if (lanes > cap) break;
-                }
-                if (active[v]) {
-                    kt += ntri[v];
-                    ke += nedge[v];
-                    kk += ntet[v];
-                    ks += nspr[v];
-                }
-                items += it;
-                ++nv;
-                ++k;
+            // the batch's own vertices first, then the others in the order they were met
+            for (int v : seen) slot_of[v] = -1;
+            for (int s = 0; s < b.nv; ++s) {
+                lists.push_back(m.color_particles[b.vb + s]);
+                slot_of[m.color_particles[b.vb + s]] = s;
             }
-            // canonical rows and vertex records
-            rows.assign((size_t)nv, 0);
-            int acc = 0;
-            for (int s = 0; s < nv; ++s) {
-                int v = m.color_particles[vb + s];
-                rows[s] = acc;
-                int nr = ntri[v] + nedge[v] + ntet[v];
-                int32_t* vr = &L.vert_rec[(size_t)(vb + s) * kVertWords];
-                vr[0] = v;
-                vr[1] = acc;
-                vr[2] = nr;
-                vr[3] = s | ((active[v] ? 1 : 0) << 16) | (nspr[v] << 17);
-                acc += nr + nspr[v];
+            for (int v : seen)
+                if (slot_of[v] < 0) lists.push_back(v);
+            b.list_count = (int)lists.size() - b.list_begin;
+            sh.list_stride = std::max(sh.list_stride, b.list_count);
+            int at = 0;
+            LaneRange* ranges[kLanes] = {&sh.tri, &sh.hinge, &sh.hinge, &sh.tet, &sh.spring};
+            for (int i = 0; i < kLanes; ++i) {
+                ranges[i]->cover(at, at + b.n[i]);
+                at += align(b.n[i]);
             }
-            int32_t rec[kBatchWords];
-            rec[0] = vb;
-            rec[1] = nv;
-            rec[2] = (int32_t)(L.tri_rec.size() / kTriWords);
-            for (int s = 0; s < nv; ++s) {
-                int v = m.color_particles[vb + s];
-                if (!active[v] || m.T == 0) continue;
-                int j = 0;
-                for (int p = m.adj_tri_off[v]; p < m.adj_tri_off[v + 1]; p += 2) {
-                    int t = m.adj_tri[p], slot = m.adj_tri[p + 1];
-                    if (!tri_ok[t]) continue;
-                    int32_t r[kTriWords];
-                    r[0] = m.tri_idx[3 * t];
-                    r[1] = m.tri_idx[3 * t + 1];
-                    r[2] = m.tri_idx[3 * t + 2];
-                    r[3] = meta(rows[s] + j, slot);
-                    for (int q = 0; q < 4; ++q) r[4 + q] = fbits(m.tri_pose[4 * t + q]);
-                    r[8] = fbits(m.tri_area[t]);
-                    r[9] = fbits(m.tri_mat[5 * t]);
-                    r[10] = fbits(m.tri_mat[5 * t + 1]);
-                    r[11] = fbits(m.tri_mat[5 * t + 2]);
-                    L.tri_rec.insert(L.tri_rec.end(), r, r + kTriWords);
-                    ++j;
-                }
-            }
-            rec[3] = (int32_t)(L.tri_rec.size() / kTriWords) - rec[2];
-            rec[4] = (int32_t)L.edge_meta.size();
-            for (int s = 0; s < nv; ++s) {
-                int v = m.color_particles[vb + s];
-                if (!active[v] || m.E == 0) continue;
-                int j = 0;
-                for (int p = m.adj_edge_off[v]; p < m.adj_edge_off[v + 1]; p += 2) {
-                    int e = m.adj_edge[p], slot = m.adj_edge[p + 1];
-                    if (!edge_ok[e]) continue;
-                    int32_t r[kEdgeWords];
-                    for (int q = 0; q < 4; ++q) r[q] = m.edge_idx[4 * e + q];
-                    r[4] = fbits(m.edge_rest[e]);
-                    r[5] = fbits(m.edge_len[e]);
-                    r[6] = fbits(m.edge_bend[2 * e]);
-                    r[7] = fbits(m.edge_bend[2 * e + 1]);
-                    L.edge_rec.insert(L.edge_rec.end(), r, r + kEdgeWords);
-                    L.edge_meta.push_back(meta(rows[s] + ntri[v] + j, slot));
-                    ++j;
-                }
-            }
-            rec[5] = (int32_t)L.edge_meta.size() - rec[4];
-            rec[6] = (int32_t)L.tet_meta.size();
-            for (int s = 0; s < nv; ++s) {
-                int v = m.color_particles[vb + s];
-                if (!active[v] || m.K == 0) continue;
-                int j = 0;
-                for (int p = m.adj_tet_off[v]; p < m.adj_tet_off[v + 1]; p += 2) {
-                    int t = m.adj_tet[p], slot = m.adj_tet[p + 1];
-                    if (!tet_ok[t]) continue;
-                    int32_t r[kTetWords];
-                    for (int q = 0; q < 4; ++q) r[q] = m.tet_idx[4 * t + q];
-                    for (int q = 0; q < 9; ++q) r[4 + q] = fbits(m.tet_pose[9 * t + q]);
-                    r[13] = fbits(m.tet_mat[3 * t]);
-                    r[14] = fbits(m.tet_mat[3 * t + 1]);
-                    r[15] = fbits(m.tet_mat[3 * t + 2]);
-                    L.tet_rec.insert(L.tet_rec.end(), r, r + kTetWords);
-                    L.tet_meta.push_back(meta(rows[s] + ntri[v] + nedge[v] + j, slot));
-                    ++j;
-                }
-            }
-            rec[7] = (int32_t)L.tet_meta.size() - rec[6];
-            rec[8] = (int32_t)(L.spr_rec.size() / kSpringWords);
-            for (int s = 0; s < nv; ++s) {
-                int v = m.color_particles[vb + s];
-                if (!active[v]) continue;
-                const int row0 = rows[s] + ntri[v] + nedge[v] + ntet[v];
-                for (int p = vs_off[v]; p < vs_off[v + 1]; ++p) {
-                    const int sp = vs_item[p] >> 1, end = vs_item[p] & 1;
-                    int32_t r[kSpringWords];
-                    r[0] = m.spring_idx[2 * sp];
-                    r[1] = m.spring_idx[2 * sp + 1];
-                    r[2] = meta(row0 + (p - vs_off[v]), end);
-                    r[3] = pre_row[p];
-                    r[4] = fbits(m.spring_rest[sp]);
-                    r[5] = fbits(m.spring_ke[sp]);
-                    r[6] = fbits(m.spring_kd[sp]);
-                    r[7] = 0;
-                    L.spr_rec.insert(L.spr_rec.end(), r, r + kSpringWords);
-                }
-            }
-            rec[9] = (int32_t)(L.spr_rec.size() / kSpringWords) - rec[8];
-            rec[10] = 0;
-            rec[11] = 0;
-            L.fast_items += rec[3] + rec[5] + rec[7] + rec[9];
-            const size_t at = L.batch_blk.size();
-            L.batch_blk.resize(at + L.blk_words, 0);
-            std::memcpy(&L.batch_blk[at], rec, sizeof(rec));
-            std::memcpy(&L.batch_blk[at + kBatchWords], &L.vert_rec[(size_t)vb * kVertWords],
-                        sizeof(int32_t) * kVertWords * (size_t)nv);
+            batches.push_back(b);
         }
     }
-    L.fast_color_off[C] = (int32_t)(L.batch_blk.size() / L.blk_words);
+    L.fast_color_off[C] = (int32_t)batches.size();
     L.slow_color_off[C] = (int32_t)L.slow_pos.size();
+
+    // ---- the records
+    const size_t B = batches.size();
+    sh.list_stride = (sh.list_stride + 3) & ~3;
+    L.batch_blk.assign(B * (size_t)L.blk_words, 0);
+    L.item_rec.assign(B * (size_t)cap * kItemWords, 0);
+    L.list.assign(B * (size_t)sh.list_stride, 0);
+    L.tri_rec.assign(B * (size_t)sh.tri.count() * kTriWords, 0);
+    L.tet_rec.assign(B * (size_t)sh.tet.count() * kTetWords, 0);
+    L.spr_rec.assign(B * (size_t)sh.spring.count() * kSpringWords, 0);
+    L.hinge_damp.assign(B * (size_t)sh.hinge.count(), 0);
+    for (size_t bi = 0; bi < B; ++bi) {
+        const Batch& b = batches[bi];
+        const int32_t* list = &lists[(size_t)b.list_begin];
+        std::memcpy(&L.list[bi * (size_t)sh.list_stride], list, sizeof(int32_t) * (size_t)b.list_count);
+        for (int i = b.list_count; i < sh.list_stride; ++i) L.list[bi * (size_t)sh.list_stride + i] = list[0];
+        for (int i = 0; i < b.list_count; ++i) slot_of[list[i]] = i;
+        int lane[kLanes];
+        for (int i = 0, at = 0; i < kLanes; at += align(b.n[i++])) lane[i] = at;
+        int32_t* head = &L.batch_blk[bi * (size_t)L.blk_words];
+        int row = 0;
+        for (int s = 0; s < b.nv; ++s) {
+            const int v = m.color_particles[b.vb + s];
+            const int nr = ntri[v] + nedge[v] + ntet[v];
+            int32_t* vr = &L.vert_rec[(size_t)(b.vb + s) * kVertWords];
+            vr[0] = v;
+            vr[1] = row;
+            vr[2] = nr;
+            vr[3] = s | ((active[v] ? 1 : 0) << 16) | (nspr[v] << 17);
+            std::memcpy(head + kBatchWords + s * kVertWords, vr, sizeof(int32_t) * kVertWords);
+            for_items(v, [&](int kind, int e, int slot, const int32_t* who, int n) {
+                const int which = kind == kTri ? 0 : (kind == kHinge ? 1 + (slot >> 1) : (kind == kTet ? 3 : 4));
+                const int t = lane[which]++;
+                int32_t* r = &L.item_rec[(bi * (size_t)cap + t) * kItemWords];
+                uint32_t slots = 0;
+                for (int i = 0; i < n; ++i) slots |= (uint32_t)slot_of[who[i]] << (8 * i);
+                r[0] = (int32_t)slots;
+                bool damped = false;
+                if (kind == kTri) {
+                    const float* mat = &m.tri_mat[5 * (size_t)e];
+                    int32_t* w = &L.tri_rec[(bi * (size_t)sh.tri.count() + (t - sh.tri.lo)) * kTriWords];
+                    for (int q = 0; q < 4; ++q) w[q] = fbits(m.tri_pose[4 * (size_t)e + q]);
+                    w[4] = fbits(mat[0]);
+                    w[5] = fbits(lame_sum(mat[0], mat[1]));
+                    w[6] = fbits(rest_ratio(mat[0], mat[1]));
+                    w[7] = fbits(mat[2]);
+                    r[2] = fbits(m.tri_area[e]);
+                    damped = mat[2] > 0.0f;
+                } else if (kind == kHinge) {
+                    const float* bend = &m.edge_bend[2 * (size_t)e];
+                    r[2] = fbits(m.edge_rest[e]);
+                    r[3] = fbits(bend[0] * m.edge_len[e]);
+                    damped = bend[1] > 0.0f;
+                    if (damped) sh.hinge_damped = true;
+                    L.hinge_damp[bi * (size_t)sh.hinge.count() + (t - sh.hinge.lo)] = fbits(bend[1] * m.edge_len[e]);
+                } else if (kind == kTet) {
+                    const float* mat = &m.tet_mat[3 * (size_t)e];
+                    const float* dm = &m.tet_pose[9 * (size_t)e];
+                    int32_t* w = &L.tet_rec[(bi * (size_t)sh.tet.count() + (t - sh.tet.lo)) * kTetWords];
+                    for (int q = 0; q < 9; ++q) w[q] = fbits(dm[q]);
+                    w[9] = fbits(rest_volume(dm));
+                    w[10] = fbits(rest_ratio(mat[0], mat[1]));
+                    w[11] = fbits(mat[2]);
+                    r[2] = fbits(mat[0]);
+                    r[3] = fbits(lame_sum(mat[0], mat[1]));
+                    damped = mat[2] > 0.0f;
+                } else {  // e indexes vs_item
+                    const int sp = vs_item[e] >> 1;
+                    int32_t* w = &L.spr_rec[(bi * (size_t)sh.spring.count() + (t - sh.spring.lo)) * kSpringWords];
+                    w[0] = fbits(m.spring_ke[sp]);
+                    w[1] = fbits(m.spring_kd[sp]);
+                    r[2] = pre_row[e];
+                    r[3] = fbits(m.spring_rest[sp]);
+                    damped = true;  // a spring always reads its endpoints' previous positions
+                }
+                if (damped) sh.prev = true;
+                r[1] = item_meta(row, slot, damped, kind);
+                ++row;
+            });
+        }
+        head[0] = b.vb;
+        head[1] = b.nv;
+        head[2] = row;
+        L.fast_items += row;
+    }
     return std::string();
 }
 

@@ -1,0 +1,76 @@
+"""The color-pass layout (newton_amd/csrc/vbd_layout.h) on the CPU: every vertex in one batch or on the generic
+path, every item's vertices found through the batch's vertex list, rows in canonical order, slots in range."""
+
+import ctypes
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from newton_amd import ModelBuilder, scenes
+from newton_amd.solvers.solver_vbd import color_layout
+
+HERE = Path(__file__).resolve().parent
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    so = tmp_path_factory.mktemp("layout") / "layout_check.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", str(so), str(HERE / "layout_check.cpp")],
+                   check=True)
+    return ctypes.CDLL(str(so)).check_layout
+
+
+def _fan(segments):
+    """A fan whose centre has `segments` triangles and twice as many hinges and neighbours."""
+    b = ModelBuilder(up_axis="Y")
+    a = 2.0 * np.pi * np.arange(segments) / segments
+    verts = [(0.0, 0.0, 0.0)] + [(r * np.cos(x), 0.0, r * np.sin(x)) for r in (0.5, 1.0) for x in a]
+    tris = []
+    for i in range(segments):
+        j = (i + 1) % segments
+        tris += [0, 1 + i, 1 + j, 1 + i, 1 + segments + i, 1 + j]
+    b.add_cloth_mesh(pos=(0.0, 0.0, 0.0), rot=(0.0, 0.0, 0.0, 1.0), scale=1.0, vel=(0.0, 0.0, 0.0), vertices=verts,
+                     indices=tris, density=0.1, tri_ke=1.0e3, tri_ka=1.0e3, tri_kd=1.0e-3, edge_ke=0.1, edge_kd=0.0)
+    b.color(include_bending=True)
+    return b.finalize("cpu")
+
+
+MODELS = {
+    "strip": lambda: scenes.cloth_strip_pinned("cpu")[0],
+    "cloth_17": lambda: scenes.cloth_hanging("cpu", verts_per_side=17)[0],
+    "springs": lambda: scenes.cloth_drop_on_sphere("cpu", verts_per_side=13, springs=True)[0],
+    "rope": lambda: scenes.bead_rope_light("cpu")[0],
+    "cube": lambda: scenes.soft_cube("cpu", cells=4)[0],
+    "worlds": lambda: scenes.cloth_batched("cpu", worlds=3, side_min=5, side_max=12)[0],
+    "fan_40": lambda: _fan(40),    # 120 items, 81 vertices: every packed shape holds it
+    "fan_80": lambda: _fan(80),    # 240 items, 161 vertices: only the widest shape holds it
+    "fan_120": lambda: _fan(120),  # generic path
+}
+
+
+@pytest.mark.parametrize("name", sorted(MODELS))
+@pytest.mark.parametrize("block,aligned", [(256, 0), (256, 1), (192, 0), (192, 1), (128, 0), (128, 1)])
+def test_layout(check, name, block, aligned):
+    m = MODELS[name]()
+    adj = m.soft_mesh_adjacency
+    co, cp = color_layout(m)
+
+    def arr(x, dtype):
+        x = x.cpu().numpy() if hasattr(x, "cpu") else x
+        return np.ascontiguousarray(np.zeros(1) if x is None else x, dtype=dtype).reshape(-1)
+
+    f, i = np.float32, np.int32
+    keep = [arr(m.particle_mass, f), arr(m.particle_flags, i), arr(m.tri_indices, i), arr(m.tri_materials, f),
+            arr(m.edge_indices, i), arr(m.edge_bending_properties, f), arr(m.tet_indices, i), arr(m.tet_materials, f),
+            arr(adj.v_adj_tris_offsets, i), arr(adj.v_adj_tris, i), arr(adj.v_adj_edges_offsets, i),
+            arr(adj.v_adj_edges, i), arr(adj.v_adj_tets_offsets, i), arr(adj.v_adj_tets, i),
+            arr(m.spring_indices if m.spring_count else None, i), co, cp]
+    stats = (ctypes.c_longlong * 4)()
+    rc = check(m.particle_count, m.tri_count, m.edge_count, m.tet_count, int(m.spring_count), len(co) - 1,
+               *[a.ctypes.data_as(ctypes.c_void_p) for a in keep], block, block // 12, aligned, stats)
+    assert rc == 0, f"layout_check.cpp:{rc}"
+    assert stats[0] + stats[1] > 0
+    if name == "fan_120":
+        assert stats[1] >= 1
