@@ -198,6 +198,55 @@ __device__ __forceinline__ float portable_atan2f(float y, float x) {
 }
 
 // ---------------------------------------------------------------------------
+// Square roots, reciprocals and quotients that share their work, with the bits of IEEE sqrt and division.
+//
+// An element divides several numbers by one length.  An IEEE division is 11 instructions (one of them a
+// quarter-rate reciprocal) and an IEEE square root 14, and a hinge has 13 and 3 of them: a third of its
+// instructions.  Here a length costs one v_rsq_f32 and Newton steps that give sqrt(d) and RN(1 / sqrt(d)), and
+// each quotient four more instructions (P. W. Markstein, "Computation of elementary functions on the IBM RISC
+// System/6000 processor", IBM J. Res. Dev. 34 (1990)).
+//  * root: g = d * rsq(d) and h = rsq(d) / 2, one coupled step, one correction.  Compared with IEEE sqrt for
+//    every float of [2^-100, 2^100], and 1 / root with IEEE division: the same bits.
+//  * quotient: with y = RN(1 / b) and yl = (1 - b y) y the first guess fma(a, y, a yl) is the rounded quotient
+//    unless a / b lies within 2^-23 ulp of a midpoint; there the remainder r = a - b q is exact and q + r y is
+//    within m_b 2^-26 ulp of a / b (m_b in [1, 2) the significand of b), while a quotient of two floats is no
+//    closer to a midpoint than 2^-24 / m_b ulp: the last rounding is that of a / b.
+// Callers check the ranges first (no intermediate over- or underflows within them) and take the IEEE operations
+// outside; a zero keeps its sign.
+// ---------------------------------------------------------------------------
+struct Root {
+    float s, y;  // RN(sqrt(d)), RN(1 / s)
+};
+__device__ __forceinline__ Root root_and_inverse(float d) {
+    const float t = __builtin_amdgcn_rsqf(d);
+    float g = d * t, h = 0.5f * t;
+    const float e = __builtin_fmaf(-h, g, 0.5f);
+    g = __builtin_fmaf(g, e, g);
+    h = __builtin_fmaf(h, e, h);
+    const float s = __builtin_fmaf(__builtin_fmaf(-g, g, d), h, g);
+    const float y0 = h + h, e0 = __builtin_fmaf(-s, y0, 1.0f);
+    float y = __builtin_fmaf(__builtin_fmaf(e0, e0, e0), y0, y0);
+    // 1 / s of a significand of all ones lies 2^-48 above a midpoint, which the sum above hits exactly
+    y = __uint_as_float(__float_as_uint(y) + ((__float_as_uint(s) << 9) == 0xfffffe00u ? 1u : 0u));
+    return Root{s, y};
+}
+// the low part of 1 / b beside y = RN(1 / b)
+__device__ __forceinline__ float inverse_low(float b, float y) { return __builtin_fmaf(-b, y, 1.0f) * y; }
+__device__ __forceinline__ float quotient(float a, float b, float y, float yl) {
+    const float q = __builtin_fmaf(a, y, a * yl);
+    return copysignf(__builtin_fmaf(__builtin_fmaf(-b, q, a), y, q), a);  // b > 0
+}
+__device__ __forceinline__ V3 quotients(V3 a, float b, float y, float yl) {
+    return v3(quotient(a.x, b, y, yl), quotient(a.y, b, y, yl), quotient(a.z, b, y, yl));
+}
+// |a| with zero counted as larger than everything, as an ordered integer: min3(...) >= tiny_key(2^-60) means
+// that every component is zero or at least 2^-60
+__device__ __forceinline__ unsigned size_key(float a) { return (__float_as_uint(a) << 1) - 1u; }
+__device__ __forceinline__ unsigned size_key(V3 a) { return min(min(size_key(a.x), size_key(a.y)), size_key(a.z)); }
+constexpr unsigned kTinyKey = ((127u - 60u) << 24) - 1u;   // size_key(2^-60)
+constexpr unsigned kSmallKey = ((127u - 30u) << 24) - 1u;  // size_key(2^-30): squares are above 2^-60
+
+// ---------------------------------------------------------------------------
 // element force / Hessian contributions for one (vertex, element) pair
 // ---------------------------------------------------------------------------
 
@@ -224,17 +273,24 @@ __device__ __forceinline__ void eval_membrane(V3 X0, V3 X1, V3 X2, Prev prev, fl
     float f0f0 = dot(f0, f0), f1f1 = dot(f1, f1), f0f1 = dot(f0, f1);
     float Jsq = f0f0 * f1f1 - f0f1 * f0f1;
     Jsq = fmaxf(Jsq, 1.0e-20f);
-    float Js = sqrtf(Jsq);
-    float invJ = 1.0f / Js;
+    float Js, invJ;
+    if (Jsq <= 0x1p100f) {  // Jsq >= 1e-20
+        const Root r = root_and_inverse(Jsq);
+        Js = r.s;
+        invJ = r.y;
+    } else {
+        Js = sqrtf(Jsq);
+        invJ = 1.0f / Js;
+    }
     float mu_nh = mu;
     V3 g0 = scl(sub(scl(f0, f1f1), scl(f1, f0f1)), invJ);
     V3 g1 = scl(sub(scl(f1, f0f0), scl(f0, f0f1)), invJ);
     float s = l_nh * (Js - alpha);
     V3 P0 = add(scl(f0, mu_nh), scl(g0, s));
     V3 P1 = add(scl(f1, mu_nh), scl(g1, s));
-    float m0 = (float)(v_order == 0), m1 = (float)(v_order == 1), m2 = (float)(v_order == 2);
-    float df0 = D00 * (m1 - m0) + D10 * (m2 - m0);
-    float df1 = D01 * (m1 - m0) + D11 * (m2 - m0);
+    // D00 (m1 - m0) + D10 (m2 - m0) with the slot's 0/1 masks m: the other products add signed zeros only
+    float df0 = v_order == 0 ? -(D00 + D10) : (v_order == 1 ? D00 : D10);
+    float df1 = v_order == 0 ? -(D01 + D11) : (v_order == 1 ? D01 : D11);
     V3 force = neg(add(scl(P0, df0), scl(P1, df1)));
     float s_clamp = fmaxf(0.0f, s);
     float r = s_clamp * invJ;
@@ -281,23 +337,23 @@ __device__ __forceinline__ void eval_membrane(V3 X0, V3 X1, V3 X2, Prev prev, fl
         for (int j = 0; j < 3; ++j) h_out.m[i][j] = area * hess.m[i][j];
 }
 
-// ((1/len) * (I - n n^T)) * (sign * skew(v)), where sign*skew(v) == skew(sign*v)
-__device__ __forceinline__ M3 nvd_skew(float len, V3 nh, V3 v) {
-    float s = 1.0f / len;
+// ((1/len) * (I - n n^T)) * (sign * skew(v)), where sign*skew(v) == skew(sign*v); inv_len = 1/len
+__device__ __forceinline__ M3 nvd_skew(float inv_len, V3 nh, V3 v) {
     M3 P;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) P.m[i][j] = s * ((i == j ? 1.0f : 0.0f) - comp(nh, i) * comp(nh, j));
+        for (int j = 0; j < 3; ++j) P.m[i][j] = inv_len * ((i == j ? 1.0f : 0.0f) - comp(nh, i) * comp(nh, j));
     return mul_skew_right(P, v);
 }
 
-// Dihedral-angle bending, particle_vbd_kernels.py:635-816.  Only the solved
-// vertex's angle derivative is formed, in one branch-free form for all four
-// slots: with s1, s2 the vectors whose skew matrices enter dn1/dx and dn2/dx
-// (zero where the reference uses a zero matrix, :730-741) the reference's
-// products are reproduced term for term; the terms it adds for the other
-// slots, and its 0/1 mask selection, contribute signed zeros only.
+// Dihedral-angle bending, particle_vbd_kernels.py:635-816.  Only the solved vertex's angle derivative is formed.
+// A vertex opposite the hinge edge (slots 0, 1) moves one of the two normals, a vertex on the edge (slots 2, 3)
+// both: the reference's products are reproduced term for term; the terms it adds for the other slots, its zero
+// matrices (:730-741) and its 0/1 mask selection contribute signed zeros only, and a sign factored out of a
+// product or a sum changes no other bit.  The pass layout puts slots 0, 1 and slots 2, 3 into lanes of their own,
+// so in a wave-aligned layout a wave runs one of the two forms (548 -> 380 and 470 vector instructions a hinge,
+// with the shared square roots and reciprocals above: pass of 512 cloth worlds 60.7 -> 52.0 us).
 // k = ke * rest_length and kdl = kd * rest_length come from the caller.
 template <typename Prev>
 __device__ __forceinline__ void eval_bending(V3 x0, V3 x1, V3 x2, V3 x3, Prev prev, float rest_angle, float k,
@@ -307,35 +363,65 @@ __device__ __forceinline__ void eval_bending(V3 x0, V3 x1, V3 x2, V3 x3, Prev pr
     const float eps = 1.0e-6f;
     V3 x02 = sub(x2, x0), x03 = sub(x3, x0), x13 = sub(x3, x1), x12 = sub(x2, x1), e = sub(x3, x2);
     V3 n1 = cross(x02, x03), n2 = cross(x13, x12);
-    float n1n = length(n1), n2n = length(n2), en = length(e);
-    if (n1n < eps || n2n < eps || en < eps) return;
-    V3 n1h = divs(n1, n1n), n2h = divs(n2, n2n), eh = divs(e, en);
+    const float d1 = dot(n1, n1), d2 = dot(n2, n2), de = dot(e, e);
+    float n1n, n2n, en, inv1, inv2;
+    V3 n1h, n2h, eh;
+    const float dmin = fminf(fminf(d1, d2), de), dmax = fmaxf(fmaxf(d1, d2), de);
+    if (dmin >= 0x1p-60f && dmax <= 0x1p60f &&
+        min(min(size_key(n1), size_key(n2)), size_key(e)) >= kTinyKey) {
+        const Root r1 = root_and_inverse(d1), r2 = root_and_inverse(d2), re = root_and_inverse(de);
+        n1n = r1.s;
+        n2n = r2.s;
+        en = re.s;
+        if (n1n < eps || n2n < eps || en < eps) return;
+        inv1 = r1.y;
+        inv2 = r2.y;
+        n1h = quotients(n1, n1n, inv1, inverse_low(n1n, inv1));
+        n2h = quotients(n2, n2n, inv2, inverse_low(n2n, inv2));
+        eh = quotients(e, en, re.y, inverse_low(en, re.y));
+    } else {
+        n1n = sqrtf(d1);
+        n2n = sqrtf(d2);
+        en = sqrtf(de);
+        if (n1n < eps || n2n < eps || en < eps) return;
+        inv1 = 1.0f / n1n;
+        inv2 = 1.0f / n2n;
+        n1h = divs(n1, n1n);
+        n2h = divs(n2, n2n);
+        eh = divs(e, en);
+    }
     float sin_t = dot(cross(n1h, n2h), eh);
     float cos_t = dot(n1h, n2h);
     float theta = portable_atan2f(sin_t, cos_t);
     float dE = k * (theta - rest_angle);
-    // per-component selects (the compiler turns selects of whole vectors into branches)
-    const bool o0 = v_order == 0, o1 = v_order == 1, o2 = v_order == 2;
-    const V3 m03 = neg(x03), me = neg(e), m12 = neg(x12);
-    V3 s1, s2;
-    s1.x = o0 ? e.x : (o1 ? 0.0f : (o2 ? m03.x : x02.x));
-    s1.y = o0 ? e.y : (o1 ? 0.0f : (o2 ? m03.y : x02.y));
-    s1.z = o0 ? e.z : (o1 ? 0.0f : (o2 ? m03.z : x02.z));
-    s2.x = o0 ? 0.0f : (o1 ? me.x : (o2 ? x13.x : m12.x));
-    s2.y = o0 ? 0.0f : (o1 ? me.y : (o2 ? x13.y : m12.y));
-    s2.z = o0 ? 0.0f : (o1 ? me.z : (o2 ? x13.z : m12.z));
-    M3 dn1 = nvd_skew(n1n, n1h, s1);
-    M3 dn2 = nvd_skew(n2n, n2h, s2);
-    M3 a = mul_skew_left(n1h, dn2);
-    M3 b = mul_skew_left(n2h, dn1);
-    M3 Mm;
+    V3 dth;
+    if (v_order < 2) {
+        // slot 0: dn1 = nvd(n1, e), dsin = -(n2h x dn1)^T eh, dcos = dn1^T n2h; slot 1: dn2 = nvd(n2, -e),
+        // dsin = (n1h x dn2)^T eh, dcos = dn2^T n1h
+        const bool o0 = v_order == 0;
+        const V3 nh = v3(o0 ? n1h.x : n2h.x, o0 ? n1h.y : n2h.y, o0 ? n1h.z : n2h.z);
+        const V3 oh = v3(o0 ? n2h.x : n1h.x, o0 ? n2h.y : n1h.y, o0 ? n2h.z : n1h.z);
+        const M3 dn = nvd_skew(o0 ? inv1 : inv2, nh, e);
+        const V3 ds = mtvec(mul_skew_left(oh, dn), eh);
+        dth = sub(scl(ds, -cos_t), scl(mtvec(dn, oh), o0 ? sin_t : -sin_t));
+    } else {
+        // per-component selects (the compiler turns selects of whole vectors into branches)
+        const bool o2 = v_order == 2;
+        const V3 s1 = v3(o2 ? -x03.x : x02.x, o2 ? -x03.y : x02.y, o2 ? -x03.z : x02.z);
+        const V3 s2 = v3(o2 ? x13.x : -x12.x, o2 ? x13.y : -x12.y, o2 ? x13.z : -x12.z);
+        const M3 dn1 = nvd_skew(inv1, n1h, s1);
+        const M3 dn2 = nvd_skew(inv2, n2h, s2);
+        const M3 a = mul_skew_left(n1h, dn2);
+        const M3 b = mul_skew_left(n2h, dn1);
+        M3 Mm;
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
+        for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) Mm.m[i][j] = a.m[i][j] - b.m[i][j];
-    V3 dsin = mtvec(Mm, eh);
-    V3 dcos = add(mtvec(dn1, n2h), mtvec(dn2, n1h));
-    V3 dth = sub(scl(dsin, cos_t), scl(dcos, sin_t));
+            for (int j = 0; j < 3; ++j) Mm.m[i][j] = a.m[i][j] - b.m[i][j];
+        const V3 dsin = mtvec(Mm, eh);
+        const V3 dcos = add(mtvec(dn1, n2h), mtvec(dn2, n1h));
+        dth = sub(scl(dsin, cos_t), scl(dcos, sin_t));
+    }
     V3 bf = scl(dth, -dE);
     M3 bh;
 #pragma unroll
@@ -811,20 +897,46 @@ __global__ __launch_bounds__(256) void k_contact_rows(KParams P, const float* __
 __device__ __forceinline__ void eval_spring(V3 x0, V3 x1, V3 a0, V3 a1, float rest, float ke, float kd, float dt,
                                             int endpoint, V3& f, M3& h) {
     const V3 diff = sub(x0, x1);
-    const float len = fmaxf(length(diff), 1.0e-8f);
-    const V3 base = scl(diff, ke * (rest - len) / len);
     const M3 nd = outer(diff, diff);
-    const float lsq = len * len, rl = rest / len;
+    const float d2 = dot(diff, diff);
+    float len = sqrtf(d2);
+    float num = ke * (rest - len);
+    float pull, rl;
+    V3 dir;
+    M3 nq;  // nd / len^2
+    if (d2 >= 0x1p-40f && d2 <= 0x1p40f && size_key(diff) >= kSmallKey &&
+        min(size_key(rest), size_key(num)) >= kTinyKey && fabsf(rest) <= 0x1p40f && fabsf(num) <= 0x1p60f) {
+        // 13 quotients by len and len^2 (len > 1e-8)
+        const float y = 1.0f / len, yl = inverse_low(len, y);
+        const float lsq = len * len, y2 = 1.0f / lsq, yl2 = inverse_low(lsq, y2);
+        pull = quotient(num, len, y, yl);
+        rl = quotient(rest, len, y, yl);
+        dir = quotients(diff, len, y, yl);
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) nq.m[i][j] = quotient(nd.m[i][j], lsq, y2, yl2);
+    } else {
+        len = fmaxf(len, 1.0e-8f);
+        const float lsq = len * len;
+        pull = ke * (rest - len) / len;
+        rl = rest / len;
+        dir = divs(diff, len);
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) nq.m[i][j] = nd.m[i][j] / lsq;
+    }
+    const V3 base = scl(diff, pull);
     M3 hs;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             const float id = i == j ? 1.0f : 0.0f;
-            const float inner = id - nd.m[i][j] / lsq;
+            const float inner = id - nq.m[i][j];
             hs.m[i][j] = ke * (id - rl * inner);
         }
-    const V3 dir = divs(diff, len);
     const float len_a = fmaxf(length(sub(a0, a1)), 1.0e-8f);
     const float dlen = len - len_a;
     const float kdt = kd / dt;
@@ -930,8 +1042,8 @@ __device__ __forceinline__ float add_rows_in_order(float ca, const float* __rest
 //   c  the vertex's lane solves the 3x3 block and writes displacement and position
 // Bound: vector instructions and the waits of one work-group's chain.  The items are read coalesced from fixed
 // slots and the positions once per batch, no load waits for another's branch, and six to seven waves a SIMD cover
-// what waits are left: 936 k cloth vertices in 512 worlds, 60.7 us a pass (65.2 us with element records found through
-// the header and positions gathered per element), 256x256 cloth 8.7 us (10.9).
+// what waits are left: 936 k cloth vertices in 512 worlds, 52.0 us a pass (65.2 us with element records found through
+// the header and positions gathered per element), 256x256 cloth 7.6 us (10.9).
 constexpr int kBatchHdr = vbd_layout::kBatchWords;
 
 // Element kinds a pass holds.  Every contribution of a cloth pass (triangles, hinges, springs, contacts with
@@ -3010,7 +3122,7 @@ int32_t vbd_create(const VbdModelDesc* m, const VbdSolverParams* prm, VbdContext
     k.write_q = 1;
     // Cloth starts with 192-lane work-groups and wave-aligned items: a regular mesh fills one wave with triangles,
     // one with the hinges opposite its vertices and one with those on them, ten vertices a batch (pass of a
-    // 256x256 cloth 8.7 us, 9.5 us with 256 packed lanes; of a 32x32 one 4.3 and 5.2 us).  A mesh with vertices too
+    // 256x256 cloth 7.6 us, 8.6 us with 256 packed lanes; of a 32x32 one 4.3 and 5.0 us).  A mesh with vertices too
     // large for that shape, tets (16.3 us either way for 128 cubes) and springs (a fourth range) start with 256
     // packed lanes.
     int32_t rc = VBD_OK;

@@ -220,6 +220,36 @@ def test_condition_screen_bitexact(cuda_device, mass):
     assert np.array_equal(q_gpu, q_ref) and np.array_equal(qd_gpu, qd_ref)
 
 
+@pytest.mark.parametrize("scene", ["strip", "springs"])
+@pytest.mark.parametrize("case", ["flat", "tiny_parts", "shrunk", "stretched", "far_out"])
+def test_shared_quotient_ranges_bitexact(cuda_device, scene, case):
+    """Square roots and quotients that share a reciprocal, at the edges of their ranges: exact zeros (an axis-aligned
+    flat sheet), components below 2^-60 beside ordinary ones, and lengths under and over the ranges, where the IEEE
+    operations take over."""
+    import torch
+
+    from newton_amd import scenes
+
+    if scene == "strip":
+        model, state, info = scenes.cloth_strip_pinned(cuda_device)
+    else:
+        model, state, info = scenes.cloth_drop_on_sphere(cuda_device, verts_per_side=9, springs=True)
+    q = model.particle_q.clone()
+    rng = np.random.default_rng(5)
+    q[:, 1] = q[0, 1]
+    if case == "tiny_parts":
+        q[:, 1] = torch.as_tensor(rng.choice([0.0, -0.0, 1.0e-22, -3.0e-20, 2.0e-19, 1.0e-9], q.shape[0]))
+    elif case != "flat":
+        q *= {"shrunk": 1.0e-7, "stretched": 3.0e3, "far_out": 1.0e7}[case]
+        q += torch.as_tensor(rng.normal(0.0, 0.01, q.shape), device=q.device) * q.abs().max()
+    state.particle_q.copy_(q)
+    q0, qd0 = initial(state)
+    q_gpu, qd_gpu, _ = gpu_run(model, state, info, 1)
+    q_ref, qd_ref, _ = oracle_run(model, q0, qd0, info, 1)
+    np.testing.assert_array_equal(q_gpu.view(np.uint32), q_ref.view(np.uint32))
+    np.testing.assert_array_equal(qd_gpu, qd_ref)
+
+
 def test_penalty_ramp_bitexact(cuda_device):
     """rigid_avbd_beta > 0 exercises the per-iteration penalty update (rigid_vbd_kernels.py:4861-4926)."""
     model, state, info = _scene("strip", cuda_device)
