@@ -376,29 +376,30 @@ __global__ __launch_bounds__(kBlock) void k_forward(int n, const uint16_t* __res
     }
 }
 
-// ---- inference: weights resident in LDS, 16x16x32 BF16 MFMA ------------------------
+// ---- inference: weights resident in LDS, activations in registers, 16x16x32 BF16 MFMA ---------
 // k_forward re-reads every weight tile from L2 for each 16 rows (about 6 KB per row), which bounds
 // it far below the matrix cores.  The inference kernel keeps all four BF16 weight matrices in LDS
-// (92 KB, loaded once per work-group), runs one 512-lane work-group per CU over 128-row groups
-// (8 waves x 16 rows), and uses gfx950's v_mfma_f32_16x16x32_bf16 (A: lane = row l % 16, k =
-// 8 (l / 16) .. + 7 of the 32-wide k step; B: lane = column l % 16, same k; C: lane holds rows
+// (84 KB, loaded once per work-group) and uses gfx950's v_mfma_f32_16x16x32_bf16 (A: lane = row l % 16,
+// k = 8 (l / 16) .. + 7 of the 32-wide k step; B: lane = column l % 16, same k; C: lane holds rows
 // 4 (l / 16) .. + 3 of column l % 16).  Each layer is computed transposed, Z^T = W^T H^T: the weight
-// tile is the A operand and the activation rows the B operand, so a lane ends with four
-// consecutive output columns of one row and writes them to LDS as one 8-byte store.  Layer 1's k
-// runs to 64 with the columns past 48 zero.  SiLU uses the hardware exp2 and reciprocal (the
-// activations are rounded to BF16 right after).
+// tile is the A operand and the activation rows the B operand, so a lane ends with four consecutive
+// output columns of one row in each of eight tiles.  The sum over k may take k in any order, as long as
+// both operands take the same: with lane (li, lq) carrying k = 32 kt + 4 lq .. + 3 and 32 kt + 16 + 4 lq
+// .. + 3, a lane's own columns of tiles 2 kt and 2 kt + 1 are its B operand of the next layer.  So the
+// activations never leave their lane -- no LDS, no shuffle, no barrier -- and the weights lie in LDS in
+// that order, one 16-byte read per lane and tile, without bank conflicts.  A wave carries one or two
+// groups of 16 rows.  SiLU uses the hardware exp2 and reciprocal (the
+// activations are rounded to BF16 right after); the biases are the accumulators' first values.
+// Bound: the 384 SiLUs a row, two quarter-rate instructions each (about 85 us per million rows, 120 with the
+// multiplies); without the barriers of an LDS exchange the other waves' products fill in beside them:
+// 1,048,576 rows 118.5 us, 690 TFLOP/s (215 us with activations exchanged through LDS), 16,384 rows 9.2 us (17.7).
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int kK1 = 64;                 // layer-1 k padded to two 32-wide steps
-constexpr int kS1 = kK1 + 8;            // LDS row strides (BF16 elements; 16-byte skew)
-constexpr int kSH = kHid + 8;
-constexpr int kInfWaves = 8;
-constexpr int kInfBlock = 64 * kInfWaves;
-constexpr int kInfRows = 16 * kInfWaves;  // rows per work-group iteration
-constexpr int kLdsW1 = kHid * kS1;
-constexpr int kLdsW = kHid * kSH;
-constexpr int kLdsW4 = kOutP * kSH;
-constexpr int kLdsH = kInfWaves * 16 * kSH;
+constexpr int kFrag1 = 0;                      // layer 1: k to 64 (zero past 48), then eight tiles of 16 columns
+constexpr int kFrag2 = kFrag1 + 2 * 8 * 64;    // layers 2 and 3: four k steps
+constexpr int kFrag3 = kFrag2 + 4 * 8 * 64;
+constexpr int kFrag4 = kFrag3 + 4 * 8 * 64;    // layer 4: one tile
+constexpr int kFrags = kFrag4 + 4 * 64;        // 16-byte fragments, (k step, tile, lane)
 
 __device__ inline floatx4 mfma32(bf16x8 a, bf16x8 b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -421,91 +422,116 @@ __device__ inline uint32_t pack_bf16x2(float a, float b) {
     return u;
 }
 
-// bias + SiLU of the wave's tile (lane: row li, columns 16 nt + 4 lq .. + 3) into its LDS rows
-__device__ inline void infer_epilogue(const floatx4 (&acc)[8], const float* __restrict__ bias, uint16_t* h, int li,
-                                      int lq) {
+// fragment f of the weights: lane (li, lq) of tile nt and k step kt of its layer
+__device__ inline uint4 weight_fragment(const uint16_t* __restrict__ pk, int f) {
+    const int lane = f & 63, li = lane & 15, lq = lane >> 4;
+    if (f < kFrag2) {
+        const int nt = (f >> 6) & 7, k = ((f >> 9) & 1) * 32 + lq * 8;
+        if (k >= kIn) return make_uint4(0u, 0u, 0u, 0u);
+        return *reinterpret_cast<const uint4*>(pk + pWt1 + (nt * 16 + li) * kIn + k);
+    }
+    const bool last = f >= kFrag4;
+    const int at = f - (last ? kFrag4 : (f >= kFrag3 ? kFrag3 : kFrag2));
+    const int nt = last ? 0 : (at >> 6) & 7, kt = last ? at >> 6 : at >> 9;
+    const uint16_t* row = pk + (last ? pWt4 : (f >= kFrag3 ? pWt3 : pWt2)) + (nt * 16 + li) * kHid + kt * 32 + lq * 4;
+    const uint2 lo = *reinterpret_cast<const uint2*>(row), hi = *reinterpret_cast<const uint2*>(row + 16);
+    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+}
+
+// one layer of the wave's S row groups: accumulators from the biases, then the k steps
+template <int S, int KSTEPS>
+__device__ inline void infer_layer(const uint4* w, const float4* bias, const bf16x8 (&b)[S][KSTEPS], int lane,
+                                   floatx4 (&acc)[S][8]) {
+    asm volatile("" ::: "memory");  // the weights stay in LDS: hoisted out of the row loop they would fill every register
 #pragma unroll
     for (int nt = 0; nt < 8; ++nt) {
-        const int j = nt * 16 + lq * 4;
-        const uint32_t lo = pack_bf16x2(silu_fast(acc[nt][0] + bias[j]), silu_fast(acc[nt][1] + bias[j + 1]));
-        const uint32_t hi = pack_bf16x2(silu_fast(acc[nt][2] + bias[j + 2]), silu_fast(acc[nt][3] + bias[j + 3]));
-        *reinterpret_cast<uint2*>(h + li * kSH + j) = make_uint2(lo, hi);
+        const float4 v = bias[nt * 4 + (lane >> 4)];
+#pragma unroll
+        for (int s = 0; s < S; ++s) acc[s][nt] = floatx4{v.x, v.y, v.z, v.w};
     }
+#pragma unroll
+    for (int kt = 0; kt < KSTEPS; ++kt)
+#pragma unroll
+        for (int nt = 0; nt < 8; ++nt) {
+            const bf16x8 a = __builtin_bit_cast(bf16x8, w[(kt * 8 + nt) * 64 + lane]);
+#pragma unroll
+            for (int s = 0; s < S; ++s) acc[s][nt] = mfma32(a, b[s][kt], acc[s][nt]);
+        }
 }
 
-template <int KSTEPS, int STRIDE>
-__device__ inline void infer_layer(const uint16_t* h_rows, const uint16_t* w, int li, int lq, floatx4 (&acc)[8]) {
+// SiLU of the accumulators into the next layer's operands, lane by lane
+template <int S>
+__device__ inline void infer_silu(const floatx4 (&acc)[S][8], bf16x8 (&b)[S][4]) {
 #pragma unroll
-    for (int nt = 0; nt < 8; ++nt) acc[nt] = zero4();
+    for (int s = 0; s < S; ++s)
 #pragma unroll
-    for (int kt = 0; kt < KSTEPS; ++kt) {
-        const bf16x8 hb = ld8(h_rows + li * kSH + kt * 32 + lq * 8);
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt)
-            acc[nt] = mfma32(ld8(w + (nt * 16 + li) * STRIDE + kt * 32 + lq * 8), hb, acc[nt]);
-    }
+        for (int kt = 0; kt < 4; ++kt) {
+            const floatx4 lo = acc[s][2 * kt], hi = acc[s][2 * kt + 1];
+            const uint4 u = make_uint4(pack_bf16x2(silu_fast(lo[0]), silu_fast(lo[1])),
+                                       pack_bf16x2(silu_fast(lo[2]), silu_fast(lo[3])),
+                                       pack_bf16x2(silu_fast(hi[0]), silu_fast(hi[1])),
+                                       pack_bf16x2(silu_fast(hi[2]), silu_fast(hi[3])));
+            b[s][kt] = __builtin_bit_cast(bf16x8, u);
+        }
 }
 
-__global__ __launch_bounds__(kInfBlock) void k_infer(int n, const uint16_t* __restrict__ feat,
-                                                    const uint16_t* __restrict__ pk, const float* __restrict__ prm,
-                                                    float* __restrict__ out) {
-    __shared__ __align__(16) uint16_t s_w1[kLdsW1];
-    __shared__ __align__(16) uint16_t s_w2[kLdsW];
-    __shared__ __align__(16) uint16_t s_w3[kLdsW];
-    __shared__ __align__(16) uint16_t s_w4[kLdsW4];
-    __shared__ __align__(16) uint16_t s_h[kLdsH];
-    for (int e = threadIdx.x; e < kLdsW1; e += kInfBlock) {
-        const int r = e / kS1, k = e % kS1;
-        s_w1[e] = k < kIn ? pk[pWt1 + r * kIn + k] : (uint16_t)0;
-    }
-    for (int e = threadIdx.x; e < kLdsW; e += kInfBlock) {
-        const int r = e / kSH, k = e % kSH;
-        s_w2[e] = k < kHid ? pk[pWt2 + r * kHid + k] : (uint16_t)0;
-        s_w3[e] = k < kHid ? pk[pWt3 + r * kHid + k] : (uint16_t)0;
-    }
-    for (int e = threadIdx.x; e < kLdsW4; e += kInfBlock) {
-        const int r = e / kSH, k = e % kSH;
-        s_w4[e] = k < kHid ? pk[pWt4 + r * kHid + k] : (uint16_t)0;
-    }
+// WAVES a work-group, S groups of 16 rows a wave
+template <int WAVES, int S>
+__global__ __launch_bounds__(64 * WAVES) void k_infer(int n, const uint16_t* __restrict__ feat,
+                                                      const uint16_t* __restrict__ pk, const float* __restrict__ prm,
+                                                      float* __restrict__ out) {
+    __shared__ uint4 s_w[kFrags];
+    __shared__ float4 s_b[3][kHid / 4];
+    for (int f = threadIdx.x; f < kFrags; f += 64 * WAVES) s_w[f] = weight_fragment(pk, f);
+    for (int e = threadIdx.x; e < 3 * kHid; e += 64 * WAVES)
+        reinterpret_cast<float*>(s_b)[e] = prm[(e < kHid ? ob1 : (e < 2 * kHid ? ob2 - kHid : ob3 - 2 * kHid)) + e];
     __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lq = lane >> 4;
-    uint16_t* H = s_h + wave * 16 * kSH;
-    floatx4 acc[8];
-    // every wave runs the same number of iterations (the barriers below are work-group wide)
-    for (int base = blockIdx.x * kInfRows; base < n; base += gridDim.x * kInfRows) {
-        const int r = base + wave * 16 + li;  // the row this lane carries
-        // layer 1: the B operand straight from the feature rows (48 BF16 each); k >= 48 and rows >= n
-        // read as 0
+    const int lane = threadIdx.x & 63, li = lane & 15, lq = lane >> 4;
+    const float b40 = prm[ob4], b41 = prm[ob4 + 1], b42 = prm[ob4 + 2];
+    constexpr int ROWS = 16 * S;
+    const long groups = ((long)n + ROWS - 1) / ROWS;
+    for (long g = (long)blockIdx.x * WAVES + (threadIdx.x >> 6); g < groups; g += (long)gridDim.x * WAVES) {
+        floatx4 acc[S][8];
+        bf16x8 b[S][4];
+        {
+            // layer 1: the B operand straight from the feature rows (48 BF16 each); k >= 48 and rows >= n
+            // read as 0
+            bf16x8 f[S][2] = {};
 #pragma unroll
-        for (int nt = 0; nt < 8; ++nt) acc[nt] = zero4();
-#pragma unroll
-        for (int kt = 0; kt < kK1 / 32; ++kt) {
-            const int k0 = kt * 32 + lq * 8;
-            bf16x8 fb = {};
-            if (r < n && k0 < kIn) fb = ld8(feat + (size_t)r * kIn + k0);
-#pragma unroll
-            for (int nt = 0; nt < 8; ++nt) acc[nt] = mfma32(ld8(s_w1 + (nt * 16 + li) * kS1 + k0), fb, acc[nt]);
+            for (int s = 0; s < S; ++s) {
+                const long r = g * ROWS + s * 16 + li;
+                if (r < n) {
+                    f[s][0] = ld8(feat + r * kIn + lq * 8);
+                    if (lq < 2) f[s][1] = ld8(feat + r * kIn + 32 + lq * 8);
+                }
+            }
+            infer_layer<S, 2>(s_w + kFrag1, s_b[0], f, lane, acc);
         }
-        infer_epilogue(acc, prm + ob1, H, li, lq);
-        __syncthreads();
-        infer_layer<kHid / 32, kSH>(H, s_w2, li, lq, acc);
-        __syncthreads();
-        infer_epilogue(acc, prm + ob2, H, li, lq);
-        __syncthreads();
-        infer_layer<kHid / 32, kSH>(H, s_w3, li, lq, acc);
-        __syncthreads();
-        infer_epilogue(acc, prm + ob3, H, li, lq);
-        __syncthreads();
-        floatx4 o = zero4();
+        infer_silu<S>(acc, b);
+        infer_layer<S, 4>(s_w + kFrag2, s_b[1], b, lane, acc);
+        infer_silu<S>(acc, b);
+        infer_layer<S, 4>(s_w + kFrag3, s_b[2], b, lane, acc);
+        infer_silu<S>(acc, b);
+        floatx4 o[S];
 #pragma unroll
-        for (int kt = 0; kt < kHid / 32; ++kt)
-            o = mfma32(ld8(s_w4 + li * kSH + kt * 32 + lq * 8), ld8(H + li * kSH + kt * 32 + lq * 8), o);
-        // lane (li, lq = 0) holds outputs 0..3 of row r; the first three are the network's
-        if (lq == 0 && r < n) {
+        for (int s = 0; s < S; ++s) o[s] = zero4();
 #pragma unroll
-            for (int c = 0; c < kOut; ++c) out[(size_t)r * kOut + c] = o[c] + prm[ob4 + c];
+        for (int kt = 0; kt < 4; ++kt) {
+            const bf16x8 a = __builtin_bit_cast(bf16x8, s_w[kFrag4 + kt * 64 + lane]);
+#pragma unroll
+            for (int s = 0; s < S; ++s) o[s] = mfma32(a, b[s][kt], o[s]);
         }
-        __syncthreads();  // H is rewritten by the next group's first epilogue
+        // lane (li, lq = 0) holds outputs 0..3 of its row; the first three are the network's
+        if (lq == 0)
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                const long r = g * ROWS + s * 16 + li;
+                if (r < n) {
+                    out[r * kOut] = o[s][0] + b40;
+                    out[r * kOut + 1] = o[s][1] + b41;
+                    out[r * kOut + 2] = o[s][2] + b42;
+                }
+            }
     }
 }
 
@@ -766,8 +792,21 @@ int32_t vbd_ws_forward(void* stream, int32_t n, const uint16_t* feat, const uint
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
                                                  hipSuccess || cus <= 0)
         cus = 256;
-    const int grid = std::min(blocks_for(n, kInfRows), cus);
-    hipLaunchKernelGGL(k_infer, dim3(grid), dim3(kInfBlock), 0, (hipStream_t)stream, n, feat, packed, params, out);
+    // One work-group per CU (its weights fill half the LDS), with as few waves as give every group of 16 rows its
+    // own: a short call pays for loading the weights and one chain of layers (16,384 rows: 4 waves 9.2 us, 8 waves
+    // 9.7, 16 waves 12.3).  32 rows a wave read the weights half as often but leave more of the last round idle: they
+    // win from about four rounds on (400,000 rows 56.3 us against 61.9, 1,048,576 rows 122.8 against 118.5).
+    hipStream_t s = (hipStream_t)stream;
+    const int g16 = blocks_for(n, 16), g32 = blocks_for(n, 32);
+    if (g16 <= 4 * cus)
+        hipLaunchKernelGGL((k_infer<4, 1>), dim3(blocks_for(g16, 4)), dim3(256), 0, s, n, feat, packed, params, out);
+    else if (g16 <= 8 * cus)
+        hipLaunchKernelGGL((k_infer<8, 1>), dim3(blocks_for(g16, 8)), dim3(512), 0, s, n, feat, packed, params, out);
+    else if (g32 < 4 * 16 * cus)
+        hipLaunchKernelGGL((k_infer<16, 1>), dim3(std::min(blocks_for(g16, 16), cus)), dim3(1024), 0, s, n, feat,
+                           packed, params, out);
+    else
+        hipLaunchKernelGGL((k_infer<16, 2>), dim3(cus), dim3(1024), 0, s, n, feat, packed, params, out);
     WS_LAUNCH_CHECK("k_infer");
     return 0;
 }

@@ -47,6 +47,26 @@ def test_forward_matches_oracle(cuda_device):
         assert np.linalg.norm(got - ref) <= 5e-3 * np.linalg.norm(ref), n
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 16384, 16385, 32769, 70001, 524288, 540001])
+def test_forward_row_ranges(cuda_device, n):
+    """Every launch shape of the inference kernel at its first and last sizes: each row's output is that of a call
+    with the row in another place, up to the order of a matrix instruction's sums (FP32 accumulation)."""
+    import torch
+
+    from newton_amd.warmstart import WarmStartMLP
+
+    mlp = WarmStartMLP(cuda_device, seed=3)
+    g = torch.Generator(device=cuda_device).manual_seed(n)
+    x = torch.randn((n, 48), generator=g, device=cuda_device).to(torch.bfloat16).view(torch.int16)
+    out = torch.full((n + 64, 3), 7.0, device=cuda_device)
+    mlp.forward(x, out)
+    assert bool((out[n:] == 7.0).all())  # nothing past the last row
+    pick = torch.unique(torch.cat([torch.arange(min(n, 40)), torch.arange(max(n - 40, 0), n),
+                                   torch.randint(0, n, (200,))])).to(cuda_device)
+    ref = mlp.forward(x[pick].contiguous())
+    np.testing.assert_array_equal(out[pick].cpu().numpy(), ref.cpu().numpy())
+
+
 def test_packed_weights_are_bf16_of_params(cuda_device):
     import torch
 
