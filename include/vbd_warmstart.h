@@ -79,6 +79,21 @@ int32_t vbd_ws_backward(void* stream, int32_t n, const uint16_t* feat, const flo
 int32_t vbd_ws_reduce(void* stream, int32_t n, const float* partial_grad, const float* partial_loss, float* grad,
                       float* loss);
 
+/* The three pieces above in two kernels that keep H, Z and the weight-gradient sums on the chip.
+ * partial_grad [vbd_ws_gradient_parts(n), n_params] and partial_loss [parts] are scratch; grad and
+ * loss (may be NULL) as vbd_ws_reduce gives them, up to the order of FP32 sums over rows (fixed for
+ * a given n and device). */
+int32_t vbd_ws_gradient_parts(int32_t n);
+int32_t vbd_ws_gradient(void* stream, int32_t n, const uint16_t* feat, const float* target, const float* row_weight,
+                        const uint16_t* packed, const float* params, float* partial_grad, float* partial_loss,
+                        float* grad, float* loss);
+
+/* vbd_ws_gradient, then vbd_ws_adam and vbd_ws_pack of the new parameters, in the same two kernels. */
+int32_t vbd_ws_train_step(void* stream, int32_t n, const uint16_t* feat, const float* target, const float* row_weight,
+                          uint16_t* packed, float* params, float* partial_grad, float* partial_loss, float* grad,
+                          float* loss, float* m, float* v, float lr, float beta1, float beta2, float eps,
+                          int32_t step);
+
 /* Adam (FP32): m, v, params updated in place; step is the 1-based step count. */
 int32_t vbd_ws_adam(void* stream, float* params, const float* grad, float* m, float* v, float lr, float beta1,
                     float beta2, float eps, int32_t step);

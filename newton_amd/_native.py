@@ -260,6 +260,12 @@ WS_EXPORTS = {
         [c_void_p, c_int32, c_u16p, c_void_p, c_void_p, c_u16p, c_void_p, c_u16p, c_void_p, c_void_p, c_void_p],
     ),
     "vbd_ws_reduce": (c_int32, [c_void_p, c_int32, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "vbd_ws_gradient_parts": (c_int32, [c_int32]),
+    "vbd_ws_gradient": (c_int32, [c_void_p, c_int32, c_u16p, c_void_p, c_void_p, c_u16p, c_void_p, c_void_p, c_void_p,
+                                  c_void_p, c_void_p]),
+    "vbd_ws_train_step": (c_int32, [c_void_p, c_int32, c_u16p, c_void_p, c_void_p, c_u16p, c_void_p, c_void_p, c_void_p,
+                                    c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_float, c_float, c_float,
+                                    c_int32]),
     "vbd_ws_adam": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_float, c_float, c_float,
                               c_int32]),
 }

@@ -126,10 +126,8 @@ class WarmStartMLP:
         if n <= self._train_cap:
             return
         cap = max(n, 2 * self._train_cap)
-        parts = -(-cap // self.rows_per_wg)
-        self._out = torch.empty((cap, N_OUT), dtype=torch.float32, device=self.device)
-        self._h = torch.empty((cap, 3, N_HIDDEN), dtype=torch.int16, device=self.device)
-        self._z = torch.empty((cap, 3, N_HIDDEN), dtype=torch.float32, device=self.device)
+        with torch.cuda.device(self.device):
+            parts = int(_native.ws_lib().vbd_ws_gradient_parts(cap))
         self._pgrad = torch.empty((parts, self.n_params), dtype=torch.float32, device=self.device)
         self._ploss = torch.empty(parts, dtype=torch.float32, device=self.device)
         self._train_cap = cap
@@ -140,30 +138,28 @@ class WarmStartMLP:
         if n <= 0:
             raise ValueError("empty training batch")
         self._ensure_train_buffers(n)
-        lib = _native.ws_lib()
-        s = self._s()
-        _native.ws_check(lib.vbd_ws_forward_train(s, n, feat.data_ptr(), self.packed.data_ptr(),
-                                                  self.params.data_ptr(), self._out.data_ptr(), self._h.data_ptr(),
-                                                  self._z.data_ptr()), "vbd_ws_forward_train")
-        _native.ws_check(lib.vbd_ws_backward(s, n, feat.data_ptr(), target.data_ptr(),
-                                             None if row_weight is None else row_weight.data_ptr(),
-                                             self.packed.data_ptr(), self._out.data_ptr(), self._h.data_ptr(),
-                                             self._z.data_ptr(), self._pgrad.data_ptr(), self._ploss.data_ptr()),
-                         "vbd_ws_backward")
-        _native.ws_check(lib.vbd_ws_reduce(s, n, self._pgrad.data_ptr(), self._ploss.data_ptr(),
-                                           self.grad.data_ptr(), self.loss.data_ptr()), "vbd_ws_reduce")
+        _native.ws_check(_native.ws_lib().vbd_ws_gradient(self._s(), n, feat.data_ptr(), target.data_ptr(),
+                                                          None if row_weight is None else row_weight.data_ptr(),
+                                                          self.packed.data_ptr(), self.params.data_ptr(),
+                                                          self._pgrad.data_ptr(), self._ploss.data_ptr(),
+                                                          self.grad.data_ptr(), self.loss.data_ptr()),
+                         "vbd_ws_gradient")
         return self.loss, self.grad
 
     def train_step(self, feat, target, row_weight=None, lr: float = 1e-3, beta1: float = 0.9, beta2: float = 0.999,
                    eps: float = 1e-8) -> torch.Tensor:
         """One Adam step on the weighted MSE; returns the loss before the step (device [1])."""
-        loss, _ = self.gradient(feat, target, row_weight)
+        n = feat.shape[0]
+        if n <= 0:
+            raise ValueError("empty training batch")
+        self._ensure_train_buffers(n)
         self.step_count += 1
-        _native.ws_check(_native.ws_lib().vbd_ws_adam(self._s(), self.params.data_ptr(), self.grad.data_ptr(),
-                                                      self.m.data_ptr(), self.v.data_ptr(), float(lr), float(beta1),
-                                                      float(beta2), float(eps), self.step_count), "vbd_ws_adam")
-        self.pack()
-        return loss
+        _native.ws_check(_native.ws_lib().vbd_ws_train_step(
+            self._s(), n, feat.data_ptr(), target.data_ptr(), None if row_weight is None else row_weight.data_ptr(),
+            self.packed.data_ptr(), self.params.data_ptr(), self._pgrad.data_ptr(), self._ploss.data_ptr(),
+            self.grad.data_ptr(), self.loss.data_ptr(), self.m.data_ptr(), self.v.data_ptr(), float(lr), float(beta1),
+            float(beta2), float(eps), self.step_count), "vbd_ws_train_step")
+        return self.loss
 
 
 class LearnedWarmStart:

@@ -119,6 +119,49 @@ def test_gradient_matches_oracle(cuda_device, n, weighted):
         assert rel <= 2e-2 and cos >= 0.999, (name, rel, cos)
 
 
+@pytest.mark.parametrize("n", [1, 63, 65, 16384, 16385, 40001])
+def test_gradient_equals_its_pieces(cuda_device, n):
+    """The one-kernel gradient against forward_train, backward and reduce (row blocks short, one per CU, and several
+    per CU).  Both round activations and dZ to BF16 at the same points; FP32 sums in another order move a value by
+    1e-6 of itself, which flips the BF16 rounding (2^-8) of about one in a thousand."""
+    import ctypes
+
+    import torch
+
+    from newton_amd import _native
+    from newton_amd.warmstart import WarmStartMLP
+
+    mlp = WarmStartMLP(cuda_device, seed=6)
+    g = torch.Generator(device=cuda_device).manual_seed(n)
+    x = torch.randn((n, 48), generator=g, device=cuda_device).to(torch.bfloat16).view(torch.int16)
+    t = torch.randn((n, 3), generator=g, device=cuda_device)
+    w = torch.rand(n, generator=g, device=cuda_device)
+    loss, grad = (v.clone() for v in mlp.gradient(x, t, w))
+    parts = -(-n // mlp.rows_per_wg)
+    f32 = dict(dtype=torch.float32, device=cuda_device)
+    out, z = torch.empty((n, 3), **f32), torch.empty((n, 3, 128), **f32)
+    h = torch.empty((n, 3, 128), dtype=torch.int16, device=cuda_device)
+    pg, pl = torch.empty((parts, mlp.n_params), **f32), torch.empty(parts, **f32)
+    ref, ref_loss = torch.empty(mlp.n_params, **f32), torch.empty(1, **f32)
+    lib, s = _native.ws_lib(), torch.cuda.current_stream(cuda_device).cuda_stream
+    P = [a.data_ptr() for a in (x, t, w, mlp.packed, mlp.params, out, h, z, pg, pl, ref, ref_loss)]
+    _native.ws_check(lib.vbd_ws_forward_train(s, n, P[0], P[3], P[4], P[5], P[6], P[7]), "forward_train")
+    _native.ws_check(lib.vbd_ws_backward(s, n, P[0], P[1], P[2], P[3], P[5], P[6], P[7], P[8], P[9]), "backward")
+    _native.ws_check(lib.vbd_ws_reduce(s, n, P[8], P[9], P[10], P[11]), "reduce")
+    assert abs(loss.item() - ref_loss.item()) <= 1e-3 * abs(ref_loss.item())
+    assert float((grad - ref).norm()) <= 4e-3 * float(ref.norm())
+    # a training step is this gradient, then Adam and the packed weights
+    p0, m0, v0 = mlp.params.clone(), mlp.m.clone(), mlp.v.clone()
+    mlp.train_step(x, t, w, lr=3e-3)
+    assert bool((mlp.grad == grad).all())
+    lib.vbd_ws_adam(s, p0.data_ptr(), grad.data_ptr(), m0.data_ptr(), v0.data_ptr(), ctypes.c_float(3e-3),
+                    ctypes.c_float(0.9), ctypes.c_float(0.999), ctypes.c_float(1e-8), 1)
+    packed = torch.empty_like(mlp.packed)
+    lib.vbd_ws_pack(s, p0.data_ptr(), packed.data_ptr())
+    for a, b in ((mlp.params, p0), (mlp.m, m0), (mlp.v, v0), (mlp.packed, packed)):
+        assert bool((a == b).all())
+
+
 def test_adam_matches_oracle(cuda_device):
     import torch
 
