@@ -116,6 +116,28 @@ __device__ inline bf16x4 ld4_strided(const uint16_t* p, int stride) {
 
 __device__ inline floatx4 zero4() { return floatx4{0.0f, 0.0f, 0.0f, 0.0f}; }
 
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// two floats -> two BF16 (round to nearest even) in one v_cvt_pk_bf16_f32
+__device__ inline uint32_t pack_bf16x2(float a, float b) {
+    const bf16x2 p = __builtin_convertvector((floatx2){a, b}, bf16x2);
+    uint32_t u;
+    __builtin_memcpy(&u, &p, 4);
+    return u;
+}
+
+// Work-group -> block of particles such that each XCD (work-group i runs on XCD i % 8) takes one contiguous run of
+// blocks: its L2 then holds the neighbours its particles share, instead of every L2 reading the whole field.
+__device__ inline int xcd_block(int bid, int nb) {
+    const int xcd = bid & 7, q = nb >> 3, r = nb & 7;
+    return xcd * q + (xcd < r ? xcd : r) + (bid >> 3);
+}
+
+
+// neighbours whose indexes, and then values, are loaded together (a triangle mesh has six)
+constexpr int kRing = 6;
+
 // ---- features ----------------------------------------------------------------
 // Columns (a = (y - x0) / s_disp, c = corr / s_corr, over 1-ring neighbours j):
 //  0-2 a          3-5 c          6-8 mean(a_j) - a    9-11 mean(c_j) - c
@@ -125,13 +147,16 @@ __device__ inline floatx4 zero4() { return floatx4{0.0f, 0.0f, 0.0f, 0.0f}; }
 //  37 mass / mean mass   38 area / mean area   39 pinned fraction of neighbours   40 degree / 6
 //  41-43 mean(y_j - y_i) / s_len   44-46 sum over pinned j of (x0_j - x0_i) / (degree * s_len)   47 1
 // A particle without neighbours gets its own values for the neighbour statistics.
+// Bound: gathers and vector instructions (8 divisions and square roots a neighbour): 1,048,576 particles 78 us
+// (116 us with one neighbour's loads at a time and rows stored by their lanes).
 __global__ __launch_bounds__(kFeatBlock) void k_features(int n, const int* __restrict__ nbr_off,
                                                         const int* __restrict__ nbr, const float* __restrict__ x0,
                                                         const float* __restrict__ y, const float* __restrict__ corr,
                                                         const float* __restrict__ acc, const float* __restrict__ mass,
                                                         const float* __restrict__ area, float dt,
                                                         const float* __restrict__ scales, uint16_t* __restrict__ out) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ uint2 s_rows[kFeatBlock * (kIn / 4)];
+    const int i = xcd_block(blockIdx.x, gridDim.x) * kFeatBlock + threadIdx.x;
     if (i >= n) return;
     const float sd = scales[0], sc = scales[1], sl = scales[2], mm = scales[3], ma = scales[4];
     float xi[3], yi[3], a[3], c[3];
@@ -150,46 +175,65 @@ __global__ __launch_bounds__(kFeatBlock) void k_features(int n, const int* __res
         mxa[k] = mna[k] = a[k];
         mxc[k] = mnc[k] = c[k];
     }
-    for (int jj = j0; jj < j1; ++jj) {
-        int j = nbr[jj];
-        float aj[3], cj[3], dx[3];
-        for (int k = 0; k < 3; ++k) {
-            float xj = x0[3 * j + k];
-            aj[k] = (y[3 * j + k] - xj) / sd;
-            cj[k] = corr ? corr[3 * j + k] / sc : 0.0f;
-            dx[k] = xj - xi[k];
-            sdy[k] += y[3 * j + k] - yi[k];
-        }
-        float len = sqrtf(dx[0] * dx[0] + dx[1] * dx[1] + dx[2] * dx[2]) / sl;
-        float ac = sqrtf(cj[0] * cj[0] + cj[1] * cj[1] + cj[2] * cj[2]);
-        if (jj == j0) {
+    for (int jc = j0; jc < j1; jc += kRing / 2) {
+        // three neighbours' values are loaded together
+        int js[kRing / 2];
+        float xs[kRing / 2][3], ys[kRing / 2][3], cs[kRing / 2][3] = {}, ms[kRing / 2];
+#pragma unroll
+        for (int u = 0; u < kRing / 2; ++u) js[u] = nbr[min(jc + u, j1 - 1)];
+#pragma unroll
+        for (int u = 0; u < kRing / 2; ++u) {
+            ms[u] = mass[js[u]];
+#pragma unroll
             for (int k = 0; k < 3; ++k) {
-                mxa[k] = mna[k] = aj[k];
-                mxc[k] = mnc[k] = cj[k];
+                xs[u][k] = x0[3 * js[u] + k];
+                ys[u][k] = y[3 * js[u] + k];
+                if (corr) cs[u][k] = corr[3 * js[u] + k];
             }
-            mxl = mnl = len;
-            mxabsc = ac;
-        } else {
+        }
+#pragma unroll
+        for (int u = 0; u < kRing / 2; ++u) {
+            const int jj = jc + u;
+            if (jj >= j1) break;
+            float aj[3], cj[3], dx[3];
             for (int k = 0; k < 3; ++k) {
-                mxa[k] = fmaxf(mxa[k], aj[k]);
-                mna[k] = fminf(mna[k], aj[k]);
-                mxc[k] = fmaxf(mxc[k], cj[k]);
-                mnc[k] = fminf(mnc[k], cj[k]);
+                float xj = xs[u][k];
+                aj[k] = (ys[u][k] - xj) / sd;
+                cj[k] = corr ? cs[u][k] / sc : 0.0f;
+                dx[k] = xj - xi[k];
+                sdy[k] += ys[u][k] - yi[k];
             }
-            mxl = fmaxf(mxl, len);
-            mnl = fminf(mnl, len);
-            mxabsc = fmaxf(mxabsc, ac);
-        }
-        for (int k = 0; k < 3; ++k) {
-            sa[k] += aj[k];
-            sc3[k] += cj[k];
-            sdx[k] += dx[k];
-        }
-        slen += len;
-        sabsc += ac;
-        if (mass[j] == 0.0f) {
-            ++npin;
-            for (int k = 0; k < 3; ++k) spin[k] += dx[k];
+            float len = sqrtf(dx[0] * dx[0] + dx[1] * dx[1] + dx[2] * dx[2]) / sl;
+            float ac = sqrtf(cj[0] * cj[0] + cj[1] * cj[1] + cj[2] * cj[2]);
+            if (jj == j0) {
+                for (int k = 0; k < 3; ++k) {
+                    mxa[k] = mna[k] = aj[k];
+                    mxc[k] = mnc[k] = cj[k];
+                }
+                mxl = mnl = len;
+                mxabsc = ac;
+            } else {
+                for (int k = 0; k < 3; ++k) {
+                    mxa[k] = fmaxf(mxa[k], aj[k]);
+                    mna[k] = fminf(mna[k], aj[k]);
+                    mxc[k] = fmaxf(mxc[k], cj[k]);
+                    mnc[k] = fminf(mnc[k], cj[k]);
+                }
+                mxl = fmaxf(mxl, len);
+                mnl = fminf(mnl, len);
+                mxabsc = fmaxf(mxabsc, ac);
+            }
+            for (int k = 0; k < 3; ++k) {
+                sa[k] += aj[k];
+                sc3[k] += cj[k];
+                sdx[k] += dx[k];
+            }
+            slen += len;
+            sabsc += ac;
+            if (ms[u] == 0.0f) {
+                ++npin;
+                for (int k = 0; k < 3; ++k) spin[k] += dx[k];
+            }
         }
     }
     float f[kIn];
@@ -222,15 +266,19 @@ __global__ __launch_bounds__(kFeatBlock) void k_features(int n, const int* __res
     f[39] = (float)npin * inv;
     f[40] = (float)deg / 6.0f;
     f[47] = 1.0f;
-    uint16_t* o = out + (size_t)i * kIn;
-    for (int k = 0; k < kIn; k += 4) {
-        bf16x4 v;
-        v[0] = (short)f2bf(f[k]);
-        v[1] = (short)f2bf(f[k + 1]);
-        v[2] = (short)f2bf(f[k + 2]);
-        v[3] = (short)f2bf(f[k + 3]);
-        *reinterpret_cast<bf16x4*>(o + k) = v;
-    }
+    // rows leave through LDS: a lane's 96 bytes would be twelve 8-byte stores 96 bytes from the next lane's, the
+    // wave's rows together are contiguous
+    constexpr int kRowWords = kIn / 4;  // 8 bytes each
+    uint2* const rows = s_rows + (threadIdx.x >> 6) * 64 * kRowWords;
+#pragma unroll
+    for (int k = 0; k < kIn; k += 4)
+        rows[(threadIdx.x & 63) * kRowWords + k / 4] = make_uint2(pack_bf16x2(f[k], f[k + 1]),
+                                                                  pack_bf16x2(f[k + 2], f[k + 3]));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int first = i - (int)(threadIdx.x & 63), count = min(64, n - first);  // the wave's rows, one a lane
+    uint2* const dst = reinterpret_cast<uint2*>(out + (size_t)first * kIn);
+    for (int e = threadIdx.x & 63; e < count * kRowWords; e += count) dst[e] = rows[e];
 }
 
 // ---- weight packing ------------------------------------------------------------
@@ -241,28 +289,63 @@ __global__ __launch_bounds__(kFeatBlock) void k_features(int n, const int* __res
 // of a predicted correction fast and its smooth ones slowly.
 constexpr int kSmoothMaxWidth = 12;
 
+// W > 0: the width at compile time (3 and 6: one and two fields); 0: width at run time.
+// Bound: memory.  Six index loads and then six gathers are in flight at a time (one dependent pair after another
+// before), and an XCD's particles share its L2: 1,048,576 particles of width 3 13.5 us a sweep, 4.7 TB/s (26.4 us).
+template <int W>
 __global__ __launch_bounds__(256) void k_smooth(int n, int width, const int* __restrict__ nbr_off,
                                                 const int* __restrict__ nbr, const float* __restrict__ active,
                                                 const float* __restrict__ in, float* __restrict__ out) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
     if (i >= n) return;
+    constexpr int MAX = W > 0 ? W : kSmoothMaxWidth;
+    if (W > 0) width = W;
+    const int b = nbr_off[i], e = nbr_off[i + 1];
+    const float act = active[i];
+    float acc[MAX];
+    const float* vi = in + (size_t)width * i;
+#pragma unroll
+    for (int c = 0; c < MAX; ++c)
+        if (W > 0 || c < width) acc[c] = vi[c];
     float* o = out + (size_t)width * i;
-    if (active[i] == 0.0f) {
-        for (int c = 0; c < width; ++c) o[c] = 0.0f;
+    if (act == 0.0f) {
+#pragma unroll
+        for (int c = 0; c < MAX; ++c)
+            if (W > 0 || c < width) o[c] = 0.0f;
         return;
     }
-    float acc[kSmoothMaxWidth];
-    const float* vi = in + (size_t)width * i;
-    for (int c = 0; c < width; ++c) acc[c] = vi[c];
-    const int b = nbr_off[i], e = nbr_off[i + 1];
-    for (int k = b; k < e; ++k) {
-        const int j = nbr[k];
-        const float w = active[j];
-        const float* vj = in + (size_t)width * j;
-        for (int c = 0; c < width; ++c) acc[c] += w * vj[c];
+    if constexpr (W > 0) {
+        for (int k = b; k < e; k += kRing) {
+            int j[kRing];
+            float w[kRing], v[kRing][MAX];
+#pragma unroll
+            for (int u = 0; u < kRing; ++u) j[u] = nbr[min(k + u, e - 1)];
+#pragma unroll
+            for (int u = 0; u < kRing; ++u) {
+                w[u] = active[j[u]];
+#pragma unroll
+                for (int c = 0; c < MAX; ++c) v[u][c] = in[(size_t)W * j[u] + c];
+            }
+#pragma unroll
+            for (int u = 0; u < kRing; ++u)
+                if (k + u < e)
+#pragma unroll
+                    for (int c = 0; c < MAX; ++c) acc[c] += w[u] * v[u][c];
+        }
+    } else {
+        for (int k = b; k < e; ++k) {
+            const int j = nbr[k];
+            const float w = active[j];
+            const float* vj = in + (size_t)width * j;
+#pragma unroll
+            for (int c = 0; c < MAX; ++c)
+                if (c < width) acc[c] += w * vj[c];
+        }
     }
     const float inv = 1.0f / (float)(1 + e - b);
-    for (int c = 0; c < width; ++c) o[c] = acc[c] * inv;
+#pragma unroll
+    for (int c = 0; c < MAX; ++c)
+        if (W > 0 || c < width) o[c] = acc[c] * inv;
 }
 
 __global__ void k_pack(const float* __restrict__ prm, uint16_t* __restrict__ pk) {
@@ -409,17 +492,6 @@ __device__ inline bf16x8 ld8(const uint16_t* p) { return *reinterpret_cast<const
 
 __device__ inline float silu_fast(float z) {
     return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
-}
-
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// two floats -> two BF16 (round to nearest even) in one v_cvt_pk_bf16_f32
-__device__ inline uint32_t pack_bf16x2(float a, float b) {
-    const bf16x2 p = __builtin_convertvector((floatx2){a, b}, bf16x2);
-    uint32_t u;
-    __builtin_memcpy(&u, &p, 4);
-    return u;
 }
 
 // fragment f of the weights: lane (li, lq) of tile nt and k step kt of its layer
@@ -1164,8 +1236,13 @@ int32_t vbd_ws_smooth(void* stream, int32_t n, int32_t width, const int32_t* nbr
     float* src = v;
     float* dst = tmp;
     for (int k = 0; k < sweeps; ++k) {
-        hipLaunchKernelGGL(k_smooth, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, width, nbr_off, nbr, active, src,
-                           dst);
+        const dim3 grid(blocks_for(n, 256)), block(256);
+        if (width == 3)
+            hipLaunchKernelGGL(k_smooth<3>, grid, block, 0, s, n, width, nbr_off, nbr, active, src, dst);
+        else if (width == 6)
+            hipLaunchKernelGGL(k_smooth<6>, grid, block, 0, s, n, width, nbr_off, nbr, active, src, dst);
+        else
+            hipLaunchKernelGGL(k_smooth<0>, grid, block, 0, s, n, width, nbr_off, nbr, active, src, dst);
         WS_LAUNCH_CHECK("k_smooth");
         float* t = src;
         src = dst;

@@ -291,6 +291,8 @@ class LearnedWarmStart:
         learned = self.corr + delta
         if not self.offer_reuse:
             return self._y + self.smooth(learned)
+        if self.smooth_sweeps == 0:
+            return [self._y + self.corr, self._y + learned]
         both = self.smooth(torch.cat([self.corr, learned], dim=1))  # one set of sweeps for both fields
         return [self._y + both[:, :3], self._y + both[:, 3:]]
 

@@ -353,3 +353,52 @@ def test_smooth_matches_oracle(cuda_device):
     torch.cuda.synchronize()
     ref = mo.smooth(ws.nbr_off.cpu().numpy(), ws.nbr.cpu().numpy(), ws._act.cpu().numpy()[:, 0], v, 64)
     np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 255, 257, 2049, 5003])
+@pytest.mark.parametrize("width", [3, 6, 5])
+def test_smooth_and_features_on_irregular_rings(cuda_device, n, width):
+    """Rings of 0 to 20 neighbours (more than are loaded together), some particles inactive, sizes around the
+    work-group's and the wave's: the low-pass bit for bit, and feature rows that do not depend on their place."""
+    import torch
+
+    from newton_amd import _native
+    from newton_amd.sim.collide import current_stream_handle
+
+    rng = np.random.default_rng(n + width)
+    deg = rng.integers(0, 21, n) if n > 1 else np.zeros(1, np.int64)
+    off = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    nbr = rng.integers(0, n, max(int(off[-1]), 1)).astype(np.int32)
+    act = (rng.random(n) > 0.1).astype(np.float32)
+    v = rng.normal(0, 1, (n, width)).astype(np.float32)
+    lib, s = _native.ws_lib(), current_stream_handle(cuda_device)
+    up = lambda a: torch.as_tensor(a, device=cuda_device)  # noqa: E731
+    d_off, d_nbr, d_act, d_v = up(off), up(nbr), up(act), up(v.copy())
+    tmp = torch.empty_like(d_v)
+    _native.ws_check(lib.vbd_ws_smooth(s, n, width, d_off.data_ptr(), d_nbr.data_ptr(), d_act.data_ptr(), 3,
+                                       d_v.data_ptr(), tmp.data_ptr()), "smooth")
+    np.testing.assert_array_equal(d_v.cpu().numpy(), mo.smooth(off, nbr, act, v, 3))
+
+    x0, y, c = (up(rng.normal(0, 1, (n, 3)).astype(np.float32)) for _ in range(3))
+    mass, area = up(act * 2.0), up(rng.random(n).astype(np.float32) + 0.1)
+    scales = up(np.array([0.1, 0.01, 0.5, 1.0, 0.3], np.float32))
+
+    def features(off_, nbr_, count, x0_, y_, c_, mass_, area_):
+        out = torch.full((count + 8, 48), 77, dtype=torch.int16, device=cuda_device)
+        _native.ws_check(lib.vbd_ws_features(s, count, off_.data_ptr(), nbr_.data_ptr(), x0_.data_ptr(),
+                                             y_.data_ptr(), c_.data_ptr(), None, mass_.data_ptr(), area_.data_ptr(),
+                                             1.0 / 600.0, scales.data_ptr(), out.data_ptr()), "features")
+        assert bool((out[count:] == 77).all())
+        return out[:count]
+
+    got = features(d_off, d_nbr, n, x0, y, c, mass, area)
+    # the same particles, each alone at the end of a larger set: renumber by a rotation
+    k = max(n // 3, 1)
+    perm = torch.roll(torch.arange(n), k)
+    order = perm.numpy()
+    inv = np.argsort(order)
+    deg2 = deg[order]
+    off2 = np.concatenate([[0], np.cumsum(deg2)]).astype(np.int32)
+    nbr2 = np.concatenate([inv[nbr[off[p]:off[p + 1]]] for p in order] + [np.zeros(1, np.int64)]).astype(np.int32)
+    again = features(up(off2), up(nbr2), n, *(a[perm.to(cuda_device)].contiguous() for a in (x0, y, c, mass, area)))
+    assert bool((again == got[perm.to(cuda_device)]).all())
