@@ -2785,6 +2785,7 @@ int32_t setup_self(VbdContext* c, const VbdModelDesc* m, const VbdSolverParams* 
         (e = sc_malloc(c, &S.it_off, (size_t)N + 1)) != hipSuccess || (e = sc_malloc(c, &S.it_cur, (size_t)N)) != hipSuccess ||
         (e = sc_malloc(c, &S.ee_n, (size_t)N)) != hipSuccess ||
         (e = sc_malloc(c, &S.items, (size_t)it_cap)) != hipSuccess ||
+        (e = sc_malloc(c, &S.it_who, (size_t)it_cap)) != hipSuccess ||
         (e = sc_malloc(c, &S.rows, (size_t)it_cap * 12)) != hipSuccess ||
         (e = sc_malloc(c, &S.pos_cd, 3 * (size_t)N)) != hipSuccess || (e = sc_malloc(c, &S.trunc, (size_t)N)) != hipSuccess ||
         (e = sc_malloc(c, &S.coll, (size_t)nslots)) != hipSuccess || (e = sc_malloc(c, &S.ncoll, 1)) != hipSuccess)
@@ -2884,6 +2885,8 @@ int32_t self_detect(VbdContext* c, hipStream_t s, const float* q) {
     VBD_LAUNCH_CHECK("k_sc_items_vt");
     hipLaunchKernelGGL(k_sc_items_sort, dim3(blocks_for(N, 256)), dim3(256), 0, s, S);
     VBD_LAUNCH_CHECK("k_sc_items_sort");
+    hipLaunchKernelGGL(k_sc_items_who, dim3(kSelfGrid), dim3(256), 0, s, S);
+    VBD_LAUNCH_CHECK("k_sc_items_who");
     // compact collision list for the truncation
     hipLaunchKernelGGL(k_sc_collect, dim3((int)std::max(1L, (nslots + 256L * kCollectPer - 1) / (256L * kCollectPer))),
                        dim3(256), 0, s, S);

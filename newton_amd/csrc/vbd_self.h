@@ -74,13 +74,46 @@ struct SelfParams {
     const int* adj_edge;         // per-particle (edge, slot) CSR, ascending edge ids
     const int* adj_edge_off;     // [N+1]
     int2* items;                 // [it_cap] (key, role)
+    int4* it_who;                // [it_cap] the item's four vertices, with role and kind (sc_pack_who)
     float* rows;                 // [it_cap * 12]
     // displacement base and truncation
     float* pos_cd;               // [N,3]
     int* trunc;                  // [N] float bits
-    int* coll;                   // [E*ee_cap + N*vt_cap] recorded collision slots (any order)
+    int4* coll;                  // [E*ee_cap + N*vt_cap] recorded collisions (any order): their vertices (sc_pack_who)
     int* ncoll;                  // [1]
 };
+
+// A contact's vertices as the per-color kernels read them, resolved once per detection (slot -> list -> primitive ->
+// vertices were three dependent loads in every row and truncation): edge-edge (e1.v0, e1.v1, e2.v0, e2.v1),
+// vertex-triangle (p, t0, t1, t2). The sign bits hold the kind (x: vertex-triangle) and the item's role (y + 2 z).
+__device__ __forceinline__ int4 sc_pack_who(int4 w, int kind, int role) {
+    w.x |= kind << 31;
+    w.y |= (role & 1) << 31;
+    w.z |= (role >> 1) << 31;
+    return w;
+}
+__device__ __forceinline__ int4 sc_unpack_who(int4 w, int& kind, int& role) {
+    kind = (int)((unsigned)w.x >> 31);
+    role = (int)(((unsigned)w.y >> 31) | ((unsigned)w.z >> 31) << 1);
+    w.x &= INT_MAX;
+    w.y &= INT_MAX;
+    w.z &= INT_MAX;
+    return w;
+}
+// vertices of the contact in list slot i (edge-edge slots first)
+__device__ __forceinline__ int4 sc_slot_vertices(const SelfParams& S, long i, int& kind) {
+    const long nee = (long)S.E * S.ee_cap;
+    if (i < nee) {
+        const int* a = S.edge_idx + 4 * (int)(i / S.ee_cap);
+        const int* b = S.edge_idx + 4 * S.ee_list[i];
+        kind = 0;
+        return make_int4(a[2], a[3], b[2], b[3]);
+    }
+    const long j = i - nee;
+    const int* t = S.tri_idx + 3 * S.vt_list[j];
+    kind = 1;
+    return make_int4((int)(j / S.vt_cap), t[0], t[1], t[2]);
+}
 
 constexpr int kSelfGrid = 2048;  // work-groups of the self-contact grid-stride kernels (a contact-rich pass has a few hundred thousand items: one per lane)
 
@@ -912,45 +945,42 @@ __global__ __launch_bounds__(256) void k_sc_items_sort(SelfParams S) {
     }
 }
 
-// rows of the items of color positions [pos0, pos1) at the positions q (the pass start) and
-// anchors q_prev; the item range is read on the device (grid-stride)
-__device__ void sc_row(const SelfParams& S, const float* __restrict__ q, const float* __restrict__ q_prev, int j,
-                       float dt);
-
-__global__ void k_sc_rows(SelfParams S, const float* __restrict__ q, const float* __restrict__ q_prev, int pos0,
-                          int pos1, float dt) {
-    const int j0 = S.it_off[pos0], j1 = S.it_off[pos1];
-    for (int j = j0 + blockIdx.x * blockDim.x + threadIdx.x; j < j1; j += gridDim.x * blockDim.x)
-        sc_row(S, q, q_prev, j, dt);
+// the vertices of every item, once the items of all color positions are in order
+__global__ void k_sc_items_who(SelfParams S) {
+    const int n = S.it_off[S.N];
+    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
+        const int2 it = S.items[j];
+        int kind;
+        const int4 w = sc_slot_vertices(S, it.x, kind);
+        S.it_who[j] = sc_pack_who(w, kind, it.y);
+    }
 }
 
-__device__ void sc_row(const SelfParams& S, const float* __restrict__ q, const float* __restrict__ q_prev, int j,
-                       float dt) {
-    const int2 it = S.items[j];
-    const long nee = (long)S.E * S.ee_cap;
-    V3 f = v3(0.0f, 0.0f, 0.0f);
-    M3 h = mzero();
-    bool has;
-    if (it.x < nee) {
-        const int e1 = it.x / S.ee_cap;
-        const int e2 = S.ee_list[it.x];
-        const int* a = S.edge_idx + 4 * e1;
-        const int* b = S.edge_idx + 4 * e2;
-        has = sc_ee_role(ld3(q, a[2]), ld3(q, a[3]), ld3(q, b[2]), ld3(q, b[3]), ld3(q_prev, a[2]), ld3(q_prev, a[3]),
-                         ld3(q_prev, b[2]), ld3(q_prev, b[3]), S.radius, S.ke, S.kd, S.mu, S.friction_eps, dt,
-                         S.par_eps, it.y, f, h);
-    } else {
-        const long jj = it.x - nee;
-        const int p = (int)(jj / S.vt_cap);
-        const int* t = S.tri_idx + 3 * S.vt_list[jj];
-        has = sc_vt_role(ld3(q, t[0]), ld3(q, t[1]), ld3(q, t[2]), ld3(q, p), ld3(q_prev, t[0]), ld3(q_prev, t[1]),
-                         ld3(q_prev, t[2]), ld3(q_prev, p), S.radius, S.ke, S.kd, S.mu, S.friction_eps, dt, it.y, f, h);
+// rows of the items of color positions [pos0, pos1) at the positions q (the pass start) and
+// anchors q_prev; the item range is read on the device (grid-stride)
+__global__ __launch_bounds__(256) void k_sc_rows(SelfParams S, const float* __restrict__ q,
+                                                 const float* __restrict__ q_prev, int pos0, int pos1, float dt) {
+    const int j0 = S.it_off[pos0], j1 = S.it_off[pos1];
+    for (int j = j0 + blockIdx.x * blockDim.x + threadIdx.x; j < j1; j += gridDim.x * blockDim.x) {
+        int kind, role;
+        const int4 w = sc_unpack_who(S.it_who[j], kind, role);
+        const V3 x0 = ld3(q, w.x), x1 = ld3(q, w.y), x2 = ld3(q, w.z), x3 = ld3(q, w.w);
+        const V3 a0 = ld3(q_prev, w.x), a1 = ld3(q_prev, w.y), a2 = ld3(q_prev, w.z), a3 = ld3(q_prev, w.w);
+        V3 f = v3(0.0f, 0.0f, 0.0f);
+        M3 h = mzero();
+        const bool has = kind == 0 ? sc_ee_role(x0, x1, x2, x3, a0, a1, a2, a3, S.radius, S.ke, S.kd, S.mu,
+                                                S.friction_eps, dt, S.par_eps, role, f, h)
+                                   : sc_vt_role(x1, x2, x3, x0, a1, a2, a3, a0, S.radius, S.ke, S.kd, S.mu,
+                                                S.friction_eps, dt, role, f, h);
+        if (!has) {
+            f = v3(0.0f, 0.0f, 0.0f);
+            h = mzero();
+        }
+        float4* o = reinterpret_cast<float4*>(S.rows) + 3 * (size_t)j;
+        o[0] = make_float4(f.x, f.y, f.z, h.m[0][0]);
+        o[1] = make_float4(h.m[0][1], h.m[0][2], h.m[1][0], h.m[1][1]);
+        o[2] = make_float4(h.m[1][2], h.m[2][0], h.m[2][1], h.m[2][2]);
     }
-    if (!has) {
-        f = v3(0.0f, 0.0f, 0.0f);
-        h = mzero();
-    }
-    store_row(S.rows + 12 * (size_t)j, f, h);
 }
 
 // ---------------------------------------------------------------------------
@@ -1003,57 +1033,37 @@ __global__ __launch_bounds__(256) void k_sc_collect(SelfParams S) {
     __syncthreads();
     int w = s_base + s_cnt[t] - mine;
     for (int k = 0; k < kCollectPer; ++k)
-        if ((rec >> k) & 1u) S.coll[w++] = (int)(b0 + (long)k * 256 + t);
+        if ((rec >> k) & 1u) {
+            int kind;
+            const int4 who = sc_slot_vertices(S, b0 + (long)k * 256 + t, kind);
+            S.coll[w++] = sc_pack_who(who, kind, 0);
+        }
 }
 
-__device__ void sc_trunc_one(const SelfParams& S, const float* __restrict__ disp, long i);
-
-__global__ void k_sc_trunc_collisions(SelfParams S, const float* __restrict__ disp) {
-    const int n = S.ncoll[0];
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x)
-        sc_trunc_one(S, disp, S.coll[c]);
-}
-
-__device__ void sc_trunc_one(const SelfParams& S, const float* __restrict__ disp, long i) {
-    const long nee = (long)S.E * S.ee_cap;
-    int who[4];
-    int kind;
-    if (i < nee) {
-        const int e1 = (int)(i / S.ee_cap);
-        const int* a = S.edge_idx + 4 * e1;
-        const int* b = S.edge_idx + 4 * S.ee_list[i];
-        who[0] = a[2];
-        who[1] = a[3];
-        who[2] = b[2];
-        who[3] = b[3];
-        kind = 0;
-    } else {
-        const long j = i - nee;
-        const int p = (int)(j / S.vt_cap);
-        const int* t = S.tri_idx + 3 * S.vt_list[j];
-        who[0] = p;
-        who[1] = t[0];
-        who[2] = t[1];
-        who[3] = t[2];
-        kind = 1;
-    }
-    V3 x[4], dx[4];
+__global__ __launch_bounds__(256) void k_sc_trunc_collisions(SelfParams S, const float* __restrict__ disp) {
+    const int count = S.ncoll[0];
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < count; c += gridDim.x * blockDim.x) {
+        int kind, role;
+        const int4 w = sc_unpack_who(S.coll[c], kind, role);
+        const int who[4] = {w.x, w.y, w.z, w.w};
+        V3 x[4], dx[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        x[r] = ld3(S.pos_cd, who[r]);
-        dx[r] = ld3(disp, who[r]);
-    }
-    bool dummy[4];
-    V3 n, d;
-    if (kind == 0)
-        sc_ee_plane(x[0], dx[0], x[1], dx[1], x[2], dx[2], x[3], dx[3], dummy, n, d);
-    else
-        sc_vt_plane(x[0], dx[0], x[1], dx[1], x[2], dx[2], x[3], dx[3], dummy, n, d);
+        for (int r = 0; r < 4; ++r) {
+            x[r] = ld3(S.pos_cd, who[r]);
+            dx[r] = ld3(disp, who[r]);
+        }
+        bool dummy[4];
+        V3 n, d;
+        if (kind == 0)
+            sc_ee_plane(x[0], dx[0], x[1], dx[1], x[2], dx[2], x[3], dx[3], dummy, n, d);
+        else
+            sc_vt_plane(x[0], dx[0], x[1], dx[1], x[2], dx[2], x[3], dx[3], dummy, n, d);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        if (dummy[r]) continue;
-        const float t = sc_trunc_t(x[r], dx[r], n, d, S.par_eps, S.relax);
-        atomicMin(S.trunc + who[r], __float_as_int(t));
+        for (int r = 0; r < 4; ++r) {
+            if (dummy[r]) continue;
+            const float t = sc_trunc_t(x[r], dx[r], n, d, S.par_eps, S.relax);
+            atomicMin(S.trunc + who[r], __float_as_int(t));
+        }
     }
 }
 
