@@ -2784,7 +2784,6 @@ int32_t setup_self(VbdContext* c, const VbdModelDesc* m, const VbdSolverParams* 
         (e = sc_malloc(c, &S.it_cnt, (size_t)N + 1)) != hipSuccess ||
         (e = sc_malloc(c, &S.it_off, (size_t)N + 1)) != hipSuccess || (e = sc_malloc(c, &S.it_cur, (size_t)N)) != hipSuccess ||
         (e = sc_malloc(c, &S.ee_n, (size_t)N)) != hipSuccess ||
-        (e = sc_malloc(c, &S.items, (size_t)it_cap)) != hipSuccess ||
         (e = sc_malloc(c, &S.it_who, (size_t)it_cap)) != hipSuccess ||
         (e = sc_malloc(c, &S.rows, (size_t)it_cap * 12)) != hipSuccess ||
         (e = sc_malloc(c, &S.pos_cd, 3 * (size_t)N)) != hipSuccess || (e = sc_malloc(c, &S.trunc, (size_t)N)) != hipSuccess ||
@@ -2831,7 +2830,6 @@ int32_t sc_scan(VbdContext* c, hipStream_t s, const int* in, int* out, int n) {
 int32_t self_detect(VbdContext* c, hipStream_t s, const float* q) {
     SelfParams& S = c->sp;
     const int N = S.N, T = S.T, E = S.E;
-    const long nslots = (long)E * S.ee_cap + (long)N * S.vt_cap;
     const int nb = S.nbucket;
     // one launch clears what this detection accumulates into (the bucket counts are already zero)
     FillList F{};
@@ -2844,23 +2842,23 @@ int32_t self_detect(VbdContext* c, hipStream_t s, const float* q) {
     add_fill(S.ext, 0, 2);
     add_fill(S.tri_min, vbd_layout::fbits(S.margin), T);
     add_fill(S.it_cnt, 0, N + 1);
-    add_fill(S.ee_n, 0, N);
+    add_fill(S.it_cur, 0, N);
     add_fill(S.ncoll, 0, 1);
     hipLaunchKernelGGL(k_fill_many, dim3(blocks_for(std::max(std::max(T, N + 1), 1), 256)), dim3(256), 0, s, F);
     VBD_LAUNCH_CHECK("k_fill_many");
-    const int np = std::max(std::max(T, E), 1);
+    const int np = std::max(std::max(T, E), N);
     hipLaunchKernelGGL(k_sc_extents, dim3(blocks_for(np, 256)), dim3(256), 0, s, S, q);
     VBD_LAUNCH_CHECK("k_sc_extents");
     for (int mode = 0; mode < 2; ++mode) {
         const int n = mode == 0 ? T : E;
         if (n > 0) {
-            hipLaunchKernelGGL(k_sc_grid_insert, dim3(blocks_for(n, 256)), dim3(256), 0, s, S, q, mode, 0);
+            hipLaunchKernelGGL(k_sc_grid_insert, dim3(blocks_for((long)n * kInsertLanes, 256)), dim3(256), 0, s, S, q, mode, 0);
             VBD_LAUNCH_CHECK("k_sc_grid_insert");
         }
         int32_t rc = sc_scan(c, s, S.g_count, S.g_off, nb + 1);
         if (rc) return rc;
         if (n > 0) {
-            hipLaunchKernelGGL(k_sc_grid_insert, dim3(blocks_for(n, 256)), dim3(256), 0, s, S, q, mode, 1);
+            hipLaunchKernelGGL(k_sc_grid_insert, dim3(blocks_for((long)n * kInsertLanes, 256)), dim3(256), 0, s, S, q, mode, 1);
             VBD_LAUNCH_CHECK("k_sc_grid_insert");
         }
         if (mode == 0) {
@@ -2871,29 +2869,18 @@ int32_t self_detect(VbdContext* c, hipStream_t s, const float* q) {
             VBD_LAUNCH_CHECK("k_sc_ee_query");
         }
     }
-    // item lists per color position
+    // item lists per color position (their vertex-triangle counts are the query's)
     hipLaunchKernelGGL(k_sc_items_count_ee, dim3(blocks_for(N, 256)), dim3(256), 0, s, S);
     VBD_LAUNCH_CHECK("k_sc_items_count_ee");
-    const int gv = (int)std::max(1L, ((long)N * S.vt_cap + 255) / 256);
-    hipLaunchKernelGGL(k_sc_items_count, dim3(gv), dim3(256), 0, s, S);
-    VBD_LAUNCH_CHECK("k_sc_items_count");
     int32_t rc = sc_scan(c, s, S.it_cnt, S.it_off, N + 1);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_sc_items_ee, dim3(blocks_for(N, 256)), dim3(256), 0, s, S);
-    VBD_LAUNCH_CHECK("k_sc_items_ee");
-    hipLaunchKernelGGL(k_sc_items_vt, dim3(gv), dim3(256), 0, s, S);
+    hipLaunchKernelGGL(k_sc_items_vt, dim3(blocks_for(16L * N, 256)), dim3(256), 0, s, S);
     VBD_LAUNCH_CHECK("k_sc_items_vt");
-    hipLaunchKernelGGL(k_sc_items_sort, dim3(blocks_for(N, 256)), dim3(256), 0, s, S);
-    VBD_LAUNCH_CHECK("k_sc_items_sort");
-    hipLaunchKernelGGL(k_sc_items_who, dim3(kSelfGrid), dim3(256), 0, s, S);
-    VBD_LAUNCH_CHECK("k_sc_items_who");
+    hipLaunchKernelGGL(k_sc_items_finish, dim3(blocks_for(N, kQPerBlock)), dim3(256), 0, s, S);
+    VBD_LAUNCH_CHECK("k_sc_items_finish");
     // compact collision list for the truncation
-    hipLaunchKernelGGL(k_sc_collect, dim3((int)std::max(1L, (nslots + 256L * kCollectPer - 1) / (256L * kCollectPer))),
-                       dim3(256), 0, s, S);
+    hipLaunchKernelGGL(k_sc_collect, dim3(blocks_for((long)E + N, 256)), dim3(256), 0, s, S);
     VBD_LAUNCH_CHECK("k_sc_collect");
-    // displacements are measured from the positions of the last detection
-    hipLaunchKernelGGL(k_sc_copy3, dim3(blocks_for(3L * N, 256)), dim3(256), 0, s, S.pos_cd, q, N);
-    VBD_LAUNCH_CHECK("k_sc_copy3");
     return VBD_OK;
 }
 
