@@ -726,8 +726,8 @@ struct KParams {
     float* inertia;
     float* disp;
     const float* mass;
-    float* crows;         // full-surface contexts: every packed entry's row (force 3 + Hessian 9), evaluated
-                          // by k_contact_rows at the pass start and read back in the serial sum
+    const int* cpack_ef;  // full-surface contexts, per packed entry of an edge/face record: {c0, c1, c2, corner}
+                          // {w0, w1, w2, 0}
     int list_stride;
     int tri_hi, hinge_lo, hinge_hi, tet_lo, tet_hi, spr_lo, spr_hi;  // lanes that hold each kind (tri_lo = 0)
     int hinge_damped;      // hinge_damp is read
@@ -788,7 +788,6 @@ struct KParams {
     const float* c_body_vel;
     const float* c_normal;
     const int* pos_coff;
-    const int* cpack_ef;  // per packed entry of an edge/face record: {c0, c1, c2, corner} {w0, w1, w2, 0}
     const float* shape_margin;
     int shape_count;
 };
@@ -872,24 +871,6 @@ __device__ __forceinline__ void eval_packed_contact(const KParams& P, const floa
                                                     V3& f, M3& h) {
     const float4* c4 = reinterpret_cast<const float4*>(P.cpack) + 4 * (size_t)rec;
     eval_contact_rec(P, q, rec, c4[0], c4[1], c4[2], c4[3], dt, f, h);
-}
-
-// The rows of every packed contact entry of the color positions [p_lo, p_hi) at the positions q of
-// the pass start (a grid-stride loop over the device-sized entry range): with full-surface contacts a
-// vertex can carry a dozen entries and a batch's entries outnumber its LDS rows, so they are evaluated
-// here, one lane each, and the pass sums the stored rows in order.  An entry's force depends on its
-// vertex and on corners of other colors only, none of which moves before the vertex is solved, so
-// the rows hold the values the pass would evaluate itself.
-constexpr int kContactRowsGrid = 1024;  // work-groups of its grid-stride loop
-__global__ __launch_bounds__(256) void k_contact_rows(KParams P, const float* __restrict__ q, int p_lo, int p_hi,
-                                                      float dt) {
-    const int j0 = P.pos_coff[p_lo], j1 = P.pos_coff[p_hi];
-    for (int j = j0 + (int)(blockIdx.x * blockDim.x + threadIdx.x); j < j1; j += (int)(gridDim.x * blockDim.x)) {
-        V3 f;
-        M3 h;
-        eval_packed_contact(P, q, j, dt, f, h);
-        store_row(P.crows + (size_t)kComp * j, f, h);
-    }
 }
 
 // evaluate_spring_force_and_hessian_both_vertices (particle_vbd_kernels.py:1685-1730), the
@@ -1051,6 +1032,11 @@ constexpr int kBatchHdr = vbd_layout::kBatchWords;
 // (more work-groups per CU) and fewer lanes in the sums.  Tet and self-contact Hessians are symmetric
 // only up to rounding.
 enum PassKinds { kClothKinds = 0, kClothSpringKinds = 1, kTetKinds = 2, kAllKinds = 3 };
+// Added to the kinds of a context whose contacts include edge/face records.  A pass evaluates those itself, their
+// corners read from memory and in parts when they outnumber the rows; a kernel of their rows before each pass took
+// 8.5 us of 27 (256x256 cloth, ten entries a vertex where it touches).  Kept apart from the other passes:
+// compiled into them it cost their occupancy (936 k cloth vertices 47.3 -> 55.2 us a pass).
+constexpr int kEdgeFace = 4;
 
 // component k of a row -> its place in {f (3), H row-major (9)}
 template <bool SYM>
@@ -1085,11 +1071,13 @@ __device__ __forceinline__ void put_row(float* __restrict__ row, V3 f, const M3&
 template <int BLOCK, int WAVES, int KINDS, bool FORCE_ONLY = false>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_solve_fast(
     float* __restrict__ q, int batch_base, int nb, float dt, int mode, float* __restrict__ g_out, KParams P) {
-    constexpr bool CLOTH = KINDS != kTetKinds;
-    constexpr bool TET = KINDS == kTetKinds || KINDS == kAllKinds;
-    constexpr bool SPRING = KINDS == kClothSpringKinds || KINDS == kAllKinds;
-    constexpr bool SELF = KINDS == kAllKinds;
-    constexpr bool SYM = KINDS == kClothKinds || KINDS == kClothSpringKinds;
+    constexpr int ELEMS = KINDS & ~kEdgeFace;
+    constexpr bool EF = (KINDS & kEdgeFace) != 0;
+    constexpr bool CLOTH = ELEMS != kTetKinds;
+    constexpr bool TET = ELEMS == kTetKinds || ELEMS == kAllKinds;
+    constexpr bool SPRING = ELEMS == kClothSpringKinds || ELEMS == kAllKinds;
+    constexpr bool SELF = ELEMS == kAllKinds;
+    constexpr bool SYM = ELEMS == kClothKinds || ELEMS == kClothSpringKinds;
     constexpr int NC = FORCE_ONLY ? 3 : (SYM ? 9 : 12);  // numbers per row
     constexpr int MAXV = BLOCK / kComp;
     constexpr int ROWS = BLOCK + 64;  // static items (<= BLOCK) + contacts evaluated in parallel
@@ -1162,7 +1150,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
         if (t < nv) live = own_live = P.w_active[P.p_world[vr.x]] != 0;
         if (!__syncthreads_or(live)) return;
     }
-    const bool par_contacts = !P.crows && nstatic + ncont <= ROWS;
+    const bool par_contacts = nstatic + ncont <= ROWS;
     const int npar = par_contacts ? ncont : 0;
 
     // ---- round trip 2
@@ -1213,20 +1201,25 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
         const float4 v = s_p[(item.x >> (8 * i)) & 0xff];
         return v3(v.x, v.y, v.z);
     };
-    // a packed contact of one of the batch's own vertices (edge/face records never get here: their
-    // contexts evaluate every entry in k_contact_rows)
-    auto contact = [&](float4 A, float4 B, float4 C, float4 D, V3& f, M3& h) {
-        const int l = __float_as_int(A.y) & 0xffff;
-        const float4 v = s_q[l], p = s_p[l];
-        eval_contact(v3(v.x, v.y, v.z), v3(p.x, p.y, p.z), v3(B.w, C.x, C.y), v3(C.z, C.w, D.x), v3(D.y, D.z, D.w),
-                     B.z, B.y, A.z, A.w, B.x, P.friction_epsilon, dt, f, h);
+    // the batch's packed contact k: its vertex's staged positions, or the corners of an edge/face record, which are of
+    // other colors (no pass moves them while this one reads them)
+    auto contact = [&](int k, V3& f, M3& h) {
+        const float4* c4 = reinterpret_cast<const float4*>(P.cpack) + 4 * (size_t)(cbeg + k);
+        const float4 A = c4[0], B = c4[1], C = c4[2], D = c4[3];
+        if constexpr (EF) {
+            eval_contact_rec(P, q, cbeg + k, A, B, C, D, dt, f, h);
+        } else {
+            const int l = __float_as_int(A.y) & 0xffff;
+            const float4 v = s_q[l], p = s_p[l];
+            eval_contact(v3(v.x, v.y, v.z), v3(p.x, p.y, p.z), v3(B.w, C.x, C.y), v3(C.z, C.w, D.x),
+                         v3(D.y, D.z, D.w), B.z, B.y, A.z, A.w, B.x, P.friction_epsilon, dt, f, h);
+        }
     };
     // contacts first, from the second wave on (the first has the batch's own vertices to look after)
     for (int k = t >= 64 ? t - 64 : t + BLOCK - 64; k < npar; k += BLOCK) {
-        const float4* c4 = reinterpret_cast<const float4*>(P.cpack) + 4 * (size_t)(cbeg + k);
         V3 fe;
         M3 he;
-        contact(c4[0], c4[1], c4[2], c4[3], fe, he);
+        contact(k, fe, he);
         put_row<SYM, FORCE_ONLY>(s_rows + (nstatic + k) * NC, fe, he);  // contact rows follow the static rows
     }
     if (kind != 0) {
@@ -1269,8 +1262,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
     // ---- phase b
     const int cs = t / NC;
     const int cc = t - cs * NC;
-    if (cs < nv) {
-        float acc = s_acc[t];
+    const bool sums = cs < nv;
+    float acc = 0.0f, ca = 0.0f;
+    if (sums) {
+        acc = s_acc[t];
         const int q0 = s_row[cs], q1 = q0 + s_nrow[cs];
         // the LDS reads of four rows are issued together; the additions stay serial, in row order
         int r = q0;
@@ -1284,28 +1279,47 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
         }
         for (; r < q1; ++r) acc = acc + s_rows[r * NC + cc];
         // contacts from zero -- their LDS rows, or, when they did not fit, evaluated here by each of
-        // the vertex's lanes (component cc kept) -- then the vertex's spring rows and
+        // the vertex's lanes (component cc kept; edge/face contexts below) -- then the vertex's spring rows and
         // self-contact rows continue that sum, which is added to the element sum
-        const int c0 = s_cb[cs], c1 = s_cb[cs + 1], fc12 = full_component<SYM>(cc);
-        float ca = 0.0f;
+        const int c0 = s_cb[cs], c1 = s_cb[cs + 1];
         if (par_contacts) {
             for (int r = c0; r < c1; ++r) ca = ca + s_rows[(nstatic + r) * NC + cc];
-        } else if (P.crows) {
-            ca = add_rows_in_order(ca, P.crows + (size_t)kComp * cbeg, c0, c1, fc12);
-        } else {
+        } else if constexpr (!EF) {
             for (int r = c0; r < c1; ++r) {
                 V3 fc;
                 M3 hc;
                 eval_packed_contact(P, q, cbeg + r, dt, fc, hc);
-                ca = ca + row_component(fc, hc, fc12);
+                ca = ca + row_component(fc, hc, full_component<SYM>(cc));
             }
         }
+    }
+    if constexpr (EF) {
+        if (!par_contacts) {
+            // a part at a time, over the rows already summed (spring rows are still needed)
+            const int base = SPRING ? nstatic : 0, room = ROWS - base;
+            for (int k0 = 0; k0 < ncont; k0 += room) {
+                const int k1 = min(k0 + room, ncont);
+                __syncthreads();
+                for (int k = k0 + t; k < k1; k += BLOCK) {
+                    V3 fe;
+                    M3 he;
+                    contact(k, fe, he);
+                    put_row<SYM, FORCE_ONLY>(s_rows + (base + k - k0) * NC, fe, he);
+                }
+                __syncthreads();
+                if (sums)
+                    for (int r = max(s_cb[cs], k0), re = min(s_cb[cs + 1], k1); r < re; ++r)
+                        ca = ca + s_rows[(base + r - k0) * NC + cc];
+            }
+        }
+    }
+    if (sums) {
         if constexpr (SPRING)
-            for (int r = q1, re = q1 + s_nspr[cs]; r < re; ++r) ca = ca + s_rows[r * NC + cc];
+            for (int r = s_row[cs] + s_nrow[cs], re = r + s_nspr[cs]; r < re; ++r) ca = ca + s_rows[r * NC + cc];
         if constexpr (SELF)
-            if (P.has_self) ca = add_rows_in_order(ca, P.so_rows, s_so[cs], s_so[cs + 1], fc12);
-        acc = acc + ca;
-        s_acc[t] = acc;
+            if (P.has_self)
+                ca = add_rows_in_order(ca, P.so_rows, s_so[cs], s_so[cs + 1], full_component<SYM>(cc));
+        s_acc[t] = acc + ca;
     }
     __syncthreads();
 
@@ -2379,7 +2393,6 @@ struct VbdContext {
     int* pos_coff = nullptr;    // [N+1]
     float* cpack = nullptr;     // [entry_cap * 16]
     int* cpack_ef = nullptr;    // [entry_cap * 8] corners and weights of edge/face entries (full surface only)
-    float* crows = nullptr;     // [entry_cap * 12] contact rows of a pass (full surface only)
     int* cid_to_pack = nullptr; // [cap * 3] packed entry of each (contact, corner), -1 when none
     float* g_tmp = nullptr;     // [N,3] residual scratch
     double* r_part = nullptr;   // residual partial sums, one per first-stage workgroup
@@ -2656,6 +2669,7 @@ int32_t build_layout(VbdContext* c) {
             c->variant = kAllKinds;
         else
             c->variant = tet ? kTetKinds : (spring ? kClothSpringKinds : kClothKinds);
+        if (c->params.soft_contact_full_surface) c->variant += kEdgeFace;
     }
     k.slow_pos = c->lay_slow;
     k.has_spring = m->spring_count > 0;
@@ -2933,21 +2947,20 @@ template <int BLOCK, int WAVES, bool FORCE_ONLY>
 void launch_kinds(VbdContext* c, hipStream_t s, int b0, int nb, float* q, float dt, int mode, float* g) {
     const dim3 grid(nb), block(BLOCK);
     switch (c->variant) {
-    case kClothKinds:
-        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, kClothKinds, FORCE_ONLY>), grid, block, 0, s, q, b0, nb, dt,
-                           mode, g, c->kp);
+#define PASS_OF_KINDS(K)                                                                                          \
+    case K:                                                                                                        \
+        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, K, FORCE_ONLY>), grid, block, 0, s, q, b0, nb, dt, mode, g, \
+                           c->kp);                                                                                 \
         break;
-    case kClothSpringKinds:
-        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, kClothSpringKinds, FORCE_ONLY>), grid, block, 0, s, q, b0, nb,
-                           dt, mode, g, c->kp);
-        break;
-    case kTetKinds:
-        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, kTetKinds, FORCE_ONLY>), grid, block, 0, s, q, b0, nb, dt,
-                           mode, g, c->kp);
-        break;
-    default:
-        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, kAllKinds, FORCE_ONLY>), grid, block, 0, s, q, b0, nb, dt,
-                           mode, g, c->kp);
+        PASS_OF_KINDS(kClothKinds)
+        PASS_OF_KINDS(kClothSpringKinds)
+        PASS_OF_KINDS(kTetKinds)
+        PASS_OF_KINDS(kAllKinds)
+        PASS_OF_KINDS(kClothKinds + kEdgeFace)
+        PASS_OF_KINDS(kClothSpringKinds + kEdgeFace)
+        PASS_OF_KINDS(kTetKinds + kEdgeFace)
+        PASS_OF_KINDS(kAllKinds + kEdgeFace)
+#undef PASS_OF_KINDS
     }
 }
 
@@ -3040,8 +3053,7 @@ int32_t vbd_create(const VbdModelDesc* m, const VbdSolverParams* prm, VbdContext
     if ((e = hipMalloc(&c->cpack, sizeof(float) * kContactWords * c->entry_cap)) != hipSuccess)
         return cleanup("hipMalloc", e);
     if (prm->soft_contact_full_surface &&
-        ((e = hipMalloc(&c->cpack_ef, sizeof(int) * 8 * c->entry_cap)) != hipSuccess ||
-         (e = hipMalloc(&c->crows, sizeof(float) * kComp * c->entry_cap)) != hipSuccess))
+        (e = hipMalloc(&c->cpack_ef, sizeof(int) * 8 * c->entry_cap)) != hipSuccess)
         return cleanup("hipMalloc", e);
     if ((e = hipMalloc(&c->g_tmp, sizeof(float) * 3 * (size_t)N)) != hipSuccess) return cleanup("hipMalloc", e);
     if ((e = hipMalloc(&c->r_part, sizeof(double) * (size_t)norm_parts(N))) != hipSuccess)
@@ -3104,7 +3116,6 @@ int32_t vbd_create(const VbdModelDesc* m, const VbdSolverParams* prm, VbdContext
     k.pos_coff = c->pos_coff;
     k.cpack = c->cpack;
     k.cpack_ef = c->cpack_ef;
-    k.crows = c->crows;
     k.shape_margin = m->shape_margin;
     k.shape_count = m->shape_count;
     k.friction_epsilon = prm->friction_epsilon;
@@ -3156,7 +3167,6 @@ int32_t vbd_destroy(VbdContext* c) {
     hipFree(c->c_state);
     hipFree(c->cpack);
     hipFree(c->cpack_ef);
-    hipFree(c->crows);
     hipFree(c->g_tmp);
     hipFree(c->r_part);
     hipFree(c->r_dev);
@@ -3396,18 +3406,9 @@ int32_t launch_spring_rows(VbdContext* c, hipStream_t s, int j0, int j1, const f
     return VBD_OK;
 }
 
-int32_t launch_contact_rows(VbdContext* c, hipStream_t s, int p_lo, int p_hi, const float* q, float dt) {
-    if (!c->crows || !c->have_contacts || p_hi <= p_lo) return VBD_OK;
-    hipLaunchKernelGGL(k_contact_rows, dim3(kContactRowsGrid), dim3(256), 0, s, c->kp, q, p_lo, p_hi, dt);
-    VBD_LAUNCH_CHECK("k_contact_rows");
-    return VBD_OK;
-}
-
 int32_t launch_color(VbdContext* c, hipStream_t s, int color, float* q, float dt, int mode, float* g) {
     set_dt(c, dt);
     int32_t rc0 = launch_spring_rows(c, s, c->pre_color_off[color], c->pre_color_off[color + 1], q, dt);
-    if (rc0) return rc0;
-    rc0 = launch_contact_rows(c, s, c->color_offsets[color], c->color_offsets[color + 1], q, dt);
     if (rc0) return rc0;
     if (c->self_on) {
         hipLaunchKernelGGL(k_sc_rows, dim3(kSelfGrid), dim3(256), 0, s, c->sp, q, c->kp.q_prev,
@@ -3435,8 +3436,6 @@ int32_t launch_color(VbdContext* c, hipStream_t s, int color, float* q, float dt
 int32_t residual_by_passes(VbdContext* c, hipStream_t s, const float* q, float dt, float* g) {
     set_dt(c, dt);
     int32_t rc0 = launch_spring_rows(c, s, 0, c->pre_color_off.back(), q, dt);
-    if (rc0) return rc0;
-    rc0 = launch_contact_rows(c, s, 0, c->model.particle_count, q, dt);
     if (rc0) return rc0;
     if (c->self_on) {
         hipLaunchKernelGGL(k_sc_rows, dim3(kSelfGrid), dim3(256), 0, s, c->sp, q, c->kp.q_prev, 0,

@@ -1,5 +1,5 @@
 // Cloth self-contact on the GPU (SolverVBD particle_enable_self_contact).
-// Included by vbd_hip.hip after the vector helpers and store_row.
+// Included by vbd_hip.hip after the vector helpers.
 //
 // Reference: newton/_src/solvers/vbd/particle_vbd_kernels.py (K), solver_vbd.py (S),
 // newton/_src/geometry/kernels.py (G), newton/_src/math/__init__.py (M).
