@@ -265,3 +265,56 @@ def test_noalloc_full_surface_matches_allocating_entry_point(cuda_device):
     for name in ("soft_contact_indices", "soft_contact_barycentric", "soft_contact_body_pos", "soft_contact_normal",
                  "soft_contact_shape"):
         assert torch.equal(getattr(got, name)[:n], getattr(ref, name)[:n]), name
+
+
+@pytest.mark.parametrize("extra", ["cloth", "springs", "tets"])
+def test_full_surface_entries_beyond_the_pass_rows_bitexact(cuda_device, extra):
+    """A small cloth inside the margin of six spheres: dozens of entries a vertex, several times the rows of a
+    color pass's work-group, which sums them in parts; springs keep their rows meanwhile."""
+    import torch
+
+    from newton_amd import CollisionPipeline, ModelBuilder
+    from newton_amd.solvers import SolverVBD
+
+    b = ModelBuilder(up_axis="Y", gravity=-9.81)
+    for k in range(6):
+        b.add_shape_sphere(-1, xform=((0.01 * k, -0.5 + 0.001 * k, 0.004 * k), (0.0, 0.0, 0.0, 1.0)), radius=0.5,
+                           cfg=ModelBuilder.ShapeConfig(ke=1.0e3, kd=1.0, mu=0.2 + 0.1 * k))
+    b.add_cloth_grid(pos=(-0.04, 0.012, 0.04), rot=_quat((1.0, 0.0, 0.0), -math.pi / 2), vel=(0.1, -0.3, 0.0),
+                     dim_x=7, dim_y=7, cell_x=0.012, cell_y=0.012, mass=0.01, tri_ke=1.0e3, tri_ka=1.0e3,
+                     tri_kd=1.0e-4, edge_ke=0.5, particle_radius=0.01)
+    if extra == "springs":
+        for i in range(20, 40):
+            b.add_spring(i, i + 2, 50.0, 0.01)
+    if extra == "tets":
+        b.add_soft_grid(pos=(0.1, 0.01, 0.0), rot=(0.0, 0.0, 0.0, 1.0), vel=(0.0, 0.0, 0.0), dim_x=2, dim_y=2,
+                        dim_z=2, cell_x=0.02, cell_y=0.02, cell_z=0.02, density=100.0, k_mu=1.0e3, k_lambda=1.0e3,
+                        k_damp=1.0e-3)
+    b.color()
+    model = b.finalize(cuda_device)
+    model.soft_contact_ke, model.soft_contact_kd, model.soft_contact_mu = 1.0e3, 1.0, 0.3
+    q0, qd0 = model.particle_q.cpu().numpy().copy(), model.particle_qd.cpu().numpy().copy()
+    margin, dt, substeps, iters = 0.02, 1.0 / 600.0, 3, 3
+    pipe = CollisionPipeline(model, soft_contact_margin=margin, enable_rigid_soft_full_surface_contact=True)
+    contacts = pipe.contacts()
+    solver = SolverVBD(model, iterations=iters)
+    s0, s1 = model.state(), model.state()
+    for _ in range(substeps):
+        s0.clear_forces()
+        pipe.collide(s0, contacts)
+        solver.step(s0, s1, None, contacts, dt)
+        s0, s1 = s1, s0
+    torch.cuda.synchronize()
+    om = _full_oracle(model, pipe)
+    prm = oracle.params(iters)
+    q, qd = q0.astype(np.float32), qd0.astype(np.float32)
+    for _ in range(substeps):
+        c = oracle.Contacts(pipe.soft_contact_max)
+        n = oracle.create_soft_contacts(om, q, margin, c)
+        entries = np.bincount(c.indices[:n][c.indices[:n] >= 0], minlength=model.particle_count)[:64]
+        _, q, qd = oracle.step(om, prm, q, qd, None, c, dt)
+    # nine or more of these vertices share a batch and its at most 320 rows
+    assert np.sort(entries)[-32:].min() * 9 > 320
+    assert np.isfinite(q).all()
+    np.testing.assert_array_equal(s0.particle_q.cpu().numpy(), q)
+    np.testing.assert_array_equal(s0.particle_qd.cpu().numpy(), qd)

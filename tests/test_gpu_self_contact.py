@@ -238,3 +238,64 @@ def test_graph_capture_replay_matches_oracle(cuda_device):
     for k in range(6):
         _, q, qd = oracle.step(om, prm, q, qd, None, None, dt)
         np.testing.assert_array_equal(replays[k], q)
+
+
+def test_stacked_fans_bitexact(cuda_device):
+    """Seven fans of 24 triangles within one margin: hubs with more edges than a query has lanes, buckets of many
+    loads, more matches than a query's list holds, more vertex-triangle items at a hub than are sorted by rank."""
+    import torch
+
+    from newton_amd import ModelBuilder
+    from newton_amd.solvers import SolverVBD
+
+    blades, fans = 24, 7
+    ang = 2.0 * math.pi * np.arange(blades) / blades
+    rim = np.stack([0.01 * np.cos(ang), np.zeros(blades), 0.01 * np.sin(ang)], axis=1)
+    verts = np.concatenate([np.zeros((1, 3)), rim]).astype(np.float32)
+    tris = np.array([[0, 1 + i, 1 + (i + 1) % blades] for i in range(blades)]).reshape(-1)
+    b = ModelBuilder(up_axis="Y", gravity=0.0)
+    for k in range(fans):
+        b.add_cloth_mesh(pos=(0.0003 * k, 0.002 * k, 0.0002 * k), rot=(0.0, 0.0, 0.0, 1.0), scale=1.0,
+                         vel=(0.0, -0.2 * k, 0.0), vertices=[tuple(v) for v in verts], indices=tris.tolist(),
+                         density=10.0, tri_ke=1e2, tri_ka=1e2, tri_kd=1e-4, edge_ke=0.01, edge_kd=1e-4)
+    b.color(include_bending=True)
+    model = b.finalize(cuda_device)
+    model.soft_contact_ke, model.soft_contact_kd, model.soft_contact_mu = 1.0e2, 0.1, 0.3
+    kw = dict(particle_self_contact_radius=0.004, particle_self_contact_margin=0.025,
+              particle_vertex_contact_buffer_size=32, particle_edge_contact_buffer_size=24)
+    rng = np.random.default_rng(11)
+    q0 = (model.particle_q.cpu().numpy() + rng.normal(0, 2e-4, (model.particle_count, 3))).astype(np.float32)
+    qd0 = model.particle_qd.cpu().numpy()
+    solver = SolverVBD(model, iterations=3, particle_enable_self_contact=True, **kw)
+    s0, s1 = model.state(), model.state()
+    s0.particle_q.copy_(torch.from_numpy(q0))
+    solver.collision_detection(s0)
+    info = {k: v.cpu().numpy() for k, v in solver.collision_info().items()}
+    assert not solver.self_contact_overflow()
+    om = oracle.OracleModel(model)
+    sc = _oracle_self(model, kw)
+    oracle.self_detect(om, sc, q0)
+    assert sc.vt_count.max() > 128 and sc.ee_count.max() > 128
+    items = np.zeros(model.particle_count, int)  # vertex-triangle items of each vertex
+    tri = model.tri_indices.cpu().numpy().reshape(-1, 3)
+    for v in range(model.particle_count):
+        kept = sc.vt_list[v][sc.vt_list[v] >= 0]
+        items[v] += len(kept)
+        np.add.at(items, tri[kept].reshape(-1), 1)
+    assert items.max() > 64
+    for name, ref in (("vertex_colliding_triangles_count", sc.vt_count), ("vertex_colliding_triangles", sc.vt_list),
+                      ("edge_colliding_edges_count", sc.ee_count), ("edge_colliding_edges", sc.ee_list)):
+        np.testing.assert_array_equal(info[name], ref, err_msg=name)
+    dt = 1.0 / 1200.0
+    for _ in range(2):
+        s0.clear_forces()
+        solver.step(s0, s1, None, None, dt)
+        s0, s1 = s1, s0
+    torch.cuda.synchronize()
+    q, qd = q0, qd0
+    prm = oracle.params(3, self_contact=_oracle_self(model, kw))
+    for _ in range(2):
+        _, q, qd = oracle.step(om, prm, q, qd, None, None, dt)
+    assert np.isfinite(q).all()
+    np.testing.assert_array_equal(s0.particle_q.cpu().numpy(), q)
+    np.testing.assert_array_equal(s0.particle_qd.cpu().numpy(), qd)
