@@ -1037,6 +1037,10 @@ enum PassKinds { kClothKinds = 0, kClothSpringKinds = 1, kTetKinds = 2, kAllKind
 // 8.5 us of 27 (256x256 cloth, ten entries a vertex where it touches).  Kept apart from the other passes:
 // compiled into them it cost their occupancy (936 k cloth vertices 47.3 -> 55.2 us a pass).
 constexpr int kEdgeFace = 4;
+// Added for self-contact, whose rows k_sc_rows evaluates (contacts crowd in a few batches: evaluated in the pass, it
+// took 39 us instead of 12 and 11 of the rows kernel).  Without springs and tets the pass needs no scratch memory:
+// 12.4 -> 11.3 us (two sheets of 128x128).
+constexpr int kSelfRows = 8;
 
 // component k of a row -> its place in {f (3), H row-major (9)}
 template <bool SYM>
@@ -1071,13 +1075,13 @@ __device__ __forceinline__ void put_row(float* __restrict__ row, V3 f, const M3&
 template <int BLOCK, int WAVES, int KINDS, bool FORCE_ONLY = false>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_solve_fast(
     float* __restrict__ q, int batch_base, int nb, float dt, int mode, float* __restrict__ g_out, KParams P) {
-    constexpr int ELEMS = KINDS & ~kEdgeFace;
+    constexpr int ELEMS = KINDS & 3;
     constexpr bool EF = (KINDS & kEdgeFace) != 0;
     constexpr bool CLOTH = ELEMS != kTetKinds;
     constexpr bool TET = ELEMS == kTetKinds || ELEMS == kAllKinds;
     constexpr bool SPRING = ELEMS == kClothSpringKinds || ELEMS == kAllKinds;
-    constexpr bool SELF = ELEMS == kAllKinds;
-    constexpr bool SYM = ELEMS == kClothKinds || ELEMS == kClothSpringKinds;
+    constexpr bool SELF = (KINDS & kSelfRows) != 0;
+    constexpr bool SYM = !SELF && (ELEMS == kClothKinds || ELEMS == kClothSpringKinds);
     constexpr int NC = FORCE_ONLY ? 3 : (SYM ? 9 : 12);  // numbers per row
     constexpr int MAXV = BLOCK / kComp;
     constexpr int ROWS = BLOCK + 64;  // static items (<= BLOCK) + contacts evaluated in parallel
@@ -1164,7 +1168,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
     const V3 own_d = ld3(P.disp, own_v);
     int so = 0;
     if constexpr (SELF)  // self-contact row bounds of the batch's color positions (consecutive positions)
-        if (P.has_self) so = P.so_off[v_begin + min(t, nv)];
+        so = P.so_off[v_begin + min(t, nv)];
     if (t < nv) {  // the list starts with the batch's own vertices: id == own_v
         float* a = s_acc + t * NC;
         a[0] = (m * (y.x - x.x)) * P.dtr;
@@ -1316,9 +1320,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
     if (sums) {
         if constexpr (SPRING)
             for (int r = s_row[cs] + s_nrow[cs], re = r + s_nspr[cs]; r < re; ++r) ca = ca + s_rows[r * NC + cc];
-        if constexpr (SELF)
-            if (P.has_self)
-                ca = add_rows_in_order(ca, P.so_rows, s_so[cs], s_so[cs + 1], full_component<SYM>(cc));
+        if constexpr (SELF) ca = add_rows_in_order(ca, P.so_rows, s_so[cs], s_so[cs + 1], full_component<SYM>(cc));
         s_acc[t] = acc + ca;
     }
     __syncthreads();
@@ -2665,11 +2667,12 @@ int32_t build_layout(VbdContext* c) {
     {
         const bool cloth = L.shape.tri.count() + L.shape.hinge.count() > 0;
         const bool tet = L.shape.tet.count() > 0, spring = L.shape.spring.count() > 0;
-        if (c->params.self_contact || (tet && (cloth || spring)))
+        if ((tet && (cloth || spring)) || (c->params.self_contact && (tet || spring)))
             c->variant = kAllKinds;
         else
             c->variant = tet ? kTetKinds : (spring ? kClothSpringKinds : kClothKinds);
         if (c->params.soft_contact_full_surface) c->variant += kEdgeFace;
+        if (c->params.self_contact) c->variant += kSelfRows;
     }
     k.slow_pos = c->lay_slow;
     k.has_spring = m->spring_count > 0;
@@ -2960,6 +2963,10 @@ void launch_kinds(VbdContext* c, hipStream_t s, int b0, int nb, float* q, float 
         PASS_OF_KINDS(kClothSpringKinds + kEdgeFace)
         PASS_OF_KINDS(kTetKinds + kEdgeFace)
         PASS_OF_KINDS(kAllKinds + kEdgeFace)
+        PASS_OF_KINDS(kClothKinds + kSelfRows)
+        PASS_OF_KINDS(kAllKinds + kSelfRows)
+        PASS_OF_KINDS(kClothKinds + kSelfRows + kEdgeFace)
+        PASS_OF_KINDS(kAllKinds + kSelfRows + kEdgeFace)
 #undef PASS_OF_KINDS
     }
 }
