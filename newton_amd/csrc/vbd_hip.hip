@@ -1033,9 +1033,9 @@ constexpr int kBatchHdr = vbd_layout::kBatchWords;
 // only up to rounding.
 enum PassKinds { kClothKinds = 0, kClothSpringKinds = 1, kTetKinds = 2, kAllKinds = 3 };
 // Added to the kinds of a context whose contacts include edge/face records.  A pass evaluates those itself, their
-// corners read from memory and in parts when they outnumber the rows; a kernel of their rows before each pass took
-// 8.5 us of 27 (256x256 cloth, ten entries a vertex where it touches).  Kept apart from the other passes:
-// compiled into them it cost their occupancy (936 k cloth vertices 47.3 -> 55.2 us a pass).
+// corners read from memory and in parts when they outnumber the rows; a kernel of their rows took 8.5 us before each
+// pass (256x256 cloth on moving bodies, substep 988 -> 716 us).  Kept apart from the other passes: compiled into
+// them it cost their occupancy (substeps of 512 cloth worlds 1,160 -> 1,354 us, of a 256x256 cloth 395 -> 437 us).
 constexpr int kEdgeFace = 4;
 // Added for self-contact, whose rows k_sc_rows evaluates (contacts crowd in a few batches: evaluated in the pass, it
 // took 39 us instead of 12 and 11 of the rows kernel).  Without springs and tets the pass needs no scratch memory:

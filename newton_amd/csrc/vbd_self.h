@@ -547,8 +547,8 @@ __global__ __launch_bounds__(256) void k_sc_extents(SelfParams S, const float* _
 // goes back down to zero (the order within a bucket does not matter: a query keeps the smallest ids
 // by rank, and counts and minima are order-free).
 // Neighbouring primitives meet the same cells, and atomics on one address wait for each other: a wave's lanes with the
-// same bucket share one atomic.  kInsertLanes lanes take a primitive's cells in turn.  64,516 triangles and 97,282 edges
-// in two folded sheets, counting and writing both: one atomic per cell 125 us; shared, 1 lane 59 us, 4 lanes 45 us,
+// same bucket share one atomic.  kInsertLanes lanes take a primitive's cells in turn.  64,516 triangles and 97,282
+// edges in two folded sheets, counting and writing both: one atomic per cell 125 us; shared, 1 lane 59 us, 4 lanes 45 us,
 // 8 lanes 44 us (8 lanes without sharing: 124 us, it is the atomics that bound it).
 constexpr int kInsertLanes = 4;
 __global__ __launch_bounds__(256) void k_sc_grid_insert(SelfParams S, const float* __restrict__ q, int mode,
@@ -935,7 +935,8 @@ __global__ void k_sc_items_count_ee(SelfParams S) {
 }
 
 // Appends the vertex-triangle items (key, role) behind each position's edge-edge items: 16 lanes per vertex, four
-// contacts with four roles each at a time (a lane per slot of every list, mostly empty: 29 -> 17 us at 82,375 contacts).
+// contacts with four roles each at a time (a lane per slot of every list, mostly empty: 29 -> 17 us at 82,375
+// contacts).
 __global__ __launch_bounds__(256) void k_sc_items_vt(SelfParams S) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const int p = (int)(i / 16), role = (int)(i % 4);
@@ -953,7 +954,8 @@ __global__ __launch_bounds__(256) void k_sc_items_vt(SelfParams S) {
 // The items' vertices in their final order; kQL lanes per color position.  Edge-edge: the lanes hold kQL of the
 // vertex's edges, a scan of their counts gives each item's edge.  Vertex-triangle: up to kSortCap items are placed by
 // the rank of their key (keys of one position are distinct), longer lists sorted in place by the first lane.
-// One lane per position filled half a wave per SIMD and sorted alone: three kernels of 56 us -> 15 us at 1,256,356 items.
+// One lane per position filled half a wave per SIMD and sorted alone: three kernels of 56 us -> 15 us at 1,256,356
+// items.
 constexpr int kSortLoad = 4;
 constexpr int kSortCap = kQL * kSortLoad;
 __global__ __launch_bounds__(256) void k_sc_items_finish(SelfParams S) {
@@ -1069,8 +1071,8 @@ __global__ __launch_bounds__(256) void k_sc_rows(SelfParams S, const float* __re
 // ---------------------------------------------------------------------------
 // truncation
 // ---------------------------------------------------------------------------
-// compact list of the recorded collisions: a lane reads the count of one edge or vertex, the work-group's lanes share the
-// contacts of its 256 (one counter atomic each).  Walking all slots instead mostly met empty ones: 35 -> 16 us at
+// compact list of the recorded collisions: a lane reads the count of one edge or vertex, the work-group's lanes share
+// the contacts of its 256 (one counter atomic each).  Walking all slots instead mostly met empty ones: 35 -> 16 us at
 // 545,803 contacts.
 __global__ __launch_bounds__(256) void k_sc_collect(SelfParams S) {
     __shared__ int s_cnt[256];
