@@ -730,8 +730,6 @@ struct KParams {
                           // {w0, w1, w2, 0}
     int list_stride;
     int tri_hi, hinge_lo, hinge_hi, tet_lo, tet_hi, spr_lo, spr_hi;  // lanes that hold each kind (tri_lo = 0)
-    int hinge_damped;      // hinge_damp is read
-    int prev;              // some item reads previous positions
     float inv_dt, dtr;     // 1 / dt and 1 / (dt * dt) of the launch
     // self-contact rows per color position (vbd_self.h) and whether the pass writes q
     int has_self;
@@ -1093,14 +1091,14 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
     __shared__ int s_cb[MAXV + 1];
     __shared__ int s_so[MAXV + 1];
     __shared__ float4 s_q[LIST];    // positions of the listed vertices
-    __shared__ float4 s_p[LIST];    // their q_prev (own vertices always, the others when P.prev)
+    __shared__ float4 s_p[LIST];    // their q_prev (own vertices always, the others with kPrevAll)
     __shared__ __align__(16) float s_rows[ROWS * NC];
     __shared__ float s_acc[MAXV * NC];
 
     const int t = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     // the arguments of the second round trip come in with those of the first
-    asm volatile("" ::"s"(q), "s"(P.q_prev), "s"(P.inertia), "s"(P.disp), "s"(P.mass), "s"(P.prev), "s"(P.dtr));
+    asm volatile("" ::"s"(q), "s"(P.q_prev), "s"(P.inertia), "s"(P.disp), "s"(P.mass), "s"(P.dtr));
     const int bi = batch_base + xcd_remap(blockIdx.x, nb);
     const int b = P.batch_list ? uniform_ints(P.batch_list)[bi] : bi;
     // ---- round trip 1.  No load sits under a per-lane condition (indexes are clamped instead, conditions
@@ -1108,6 +1106,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
     // after another.
     const int* blk = P.batch_blk + (size_t)b * BLK;
     const int v_begin = uniform_ints(blk)[0], nv = uniform_ints(blk)[1], nstatic = uniform_ints(blk)[2];
+    const int flags = uniform_ints(blk)[3];  // vbd_layout::BatchFlags
     const int cbeg = uniform_ints(P.bat_cinfo)[2 * (size_t)b], ncont = uniform_ints(P.bat_cinfo)[2 * (size_t)b + 1];
     const int4 item = reinterpret_cast<const int4*>(P.item_rec)[(size_t)b * BLOCK + t];
     const int id = P.list[(size_t)b * P.list_stride + min(t, P.list_stride - 1)];
@@ -1118,10 +1117,6 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
             const int4* r = reinterpret_cast<const int4*>(P.tri_rec) + 2 * ((size_t)b * P.tri_hi + min(t, P.tri_hi - 1));
             w0 = r[0];
             w1 = r[1];
-        }
-        if (P.hinge_damped) {
-            const int lane = min(max(t, P.hinge_lo), P.hinge_hi - 1) - P.hinge_lo;
-            kdl = P.hinge_damp[(size_t)b * (P.hinge_hi - P.hinge_lo) + lane];
         }
     }
     if constexpr (TET) {
@@ -1161,8 +1156,14 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
     const int kind = item.y >> 12;  // vbd_layout::ItemKind
     const int own_v = vr.x;
     const V3 x = ld3(q, id);
+    if constexpr (CLOTH) {
+        if (flags & vbd_layout::kHingeDamped) {
+            const int lane = min(max(t, P.hinge_lo), P.hinge_hi - 1) - P.hinge_lo;
+            kdl = P.hinge_damp[(size_t)b * (P.hinge_hi - P.hinge_lo) + lane];
+        }
+    }
     // previous positions of the whole list, or of the batch's own vertices (the list's first)
-    const V3 xp = ld3(P.q_prev, P.prev || t < nv ? id : __builtin_amdgcn_readfirstlane(id));
+    const V3 xp = ld3(P.q_prev, (flags & vbd_layout::kPrevAll) || t < nv ? id : __builtin_amdgcn_readfirstlane(id));
     const float m = P.mass[own_v];
     const V3 y = ld3(P.inertia, own_v);
     const V3 own_d = ld3(P.disp, own_v);
@@ -2662,8 +2663,6 @@ int32_t build_layout(VbdContext* c) {
     k.spr_lo = L.shape.spring.lo;
     k.spr_hi = L.shape.spring.hi;
     k.list_stride = L.shape.list_stride;
-    k.hinge_damped = L.shape.hinge_damped ? 1 : 0;
-    k.prev = L.shape.prev ? 1 : 0;
     {
         const bool cloth = L.shape.tri.count() + L.shape.hinge.count() > 0;
         const bool tet = L.shape.tet.count() > 0, spring = L.shape.spring.count() > 0;

@@ -61,7 +61,7 @@ constexpr int kItemWords = 4;    // vertex slots (4 x 8 bits) | item_meta | two 
 constexpr int kTriWords = 8;     // D00 D01 D10 D11 | mu lambda+mu alpha kd
 constexpr int kTetWords = 12;    // Dm^-1 (9) rest_volume alpha kd
 constexpr int kSpringWords = 2;  // ke kd
-constexpr int kBatchWords = 4;   // vbegin nv static_rows 0
+constexpr int kBatchWords = 4;   // vbegin nv static_rows batch_flags
 constexpr int kVertWords = 4;    // v row_start nrows (local | active << 16 | nsprings << 17)
 // Distinct vertices of a batch: its own and their elements' others (a regular cloth's batch has 7 to 9 for each
 // of its own, so the lanes fill first); the work-group stages that many positions in LDS, and a smaller bound
@@ -70,6 +70,13 @@ constexpr int list_cap(int cap) { return cap <= 192 ? 128 : 192; }
 // batch block: header (kBatchWords) then max_v vertex records (unused ones zero),
 // fixed size so a workgroup reads its header and vertex records in one round trip
 inline int block_words(int max_v) { return kBatchWords + max_v * kVertWords; }  // a multiple of 4 words
+
+// batch_flags.  They follow the damping coefficients, which a rebuild may switch from or to zero under a captured graph:
+// in the batch header they are data of the layout, not arguments of the launch.
+enum BatchFlags {
+    kPrevAll = 1,      // some item reads previous positions of the listed vertices (damping, springs)
+    kHingeDamped = 2,  // some hinge has kd > 0 (hinge_damp is read)
+};
 
 enum ItemKind { kNone = 0, kTri = 1, kHinge = 2, kTet = 3, kSpring = 5 };
 // row (9 bits) | slot in the element << 9 (2 bits) | damped << 11 | kind << 12
@@ -112,12 +119,10 @@ struct LaneRange {
 // What a launch is given besides the arrays; equal shapes may be exchanged under a captured graph.
 struct PassShape {
     LaneRange tri, hinge, tet, spring;
-    int list_stride = 0;       // entries of a batch's vertex list
-    bool hinge_damped = false; // some hinge has kd > 0 (hinge_damp is read)
-    bool prev = false;         // some item reads previous positions (damping, springs)
+    int list_stride = 0;  // entries of a batch's vertex list
     bool operator==(const PassShape& o) const {
         return tri == o.tri && hinge == o.hinge && tet == o.tet && spring == o.spring &&
-               list_stride == o.list_stride && hinge_damped == o.hinge_damped && prev == o.prev;
+               list_stride == o.list_stride;
     }
 };
 
@@ -362,7 +367,7 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
         int lane[kLanes];
         for (int i = 0, at = 0; i < kLanes; at += align(b.n[i++])) lane[i] = at;
         int32_t* head = &L.batch_blk[bi * (size_t)L.blk_words];
-        int row = 0;
+        int row = 0, flags = 0;
         for (int s = 0; s < b.nv; ++s) {
             const int v = m.color_particles[b.vb + s];
             const int nr = ntri[v] + nedge[v] + ntet[v];
@@ -395,7 +400,7 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
                     r[2] = fbits(m.edge_rest[e]);
                     r[3] = fbits(bend[0] * m.edge_len[e]);
                     damped = bend[1] > 0.0f;
-                    if (damped) sh.hinge_damped = true;
+                    if (damped) flags |= kHingeDamped;
                     L.hinge_damp[bi * (size_t)sh.hinge.count() + (t - sh.hinge.lo)] = fbits(bend[1] * m.edge_len[e]);
                 } else if (kind == kTet) {
                     const float* mat = &m.tet_mat[3 * (size_t)e];
@@ -417,7 +422,7 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
                     r[3] = fbits(m.spring_rest[sp]);
                     damped = true;  // a spring always reads its endpoints' previous positions
                 }
-                if (damped) sh.prev = true;
+                if (damped) flags |= kPrevAll;
                 r[1] = item_meta(row, slot, damped, kind);
                 ++row;
             });
@@ -425,6 +430,7 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
         head[0] = b.vb;
         head[1] = b.nv;
         head[2] = row;
+        head[3] = flags;
         L.fast_items += row;
     }
     return std::string();

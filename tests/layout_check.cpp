@@ -9,12 +9,16 @@
 
 using namespace vbd_layout;
 
-// v: the model's arrays in HostModel order; stats: {batches, slow vertices, items, list stride}
-extern "C" int check_layout(int N, int T, int E, int K, int S, int C, const float* mass, const int* flags,
-                            const int* tri, const float* tri_mat, const int* edge, const float* bend, const int* tet,
-                            const float* tet_mat, const int* at_off, const int* at, const int* ae_off, const int* ae,
-                            const int* ak_off, const int* ak, const int* spring, const int* color_off,
-                            const int* color_particles, int cap, int max_v, int aligned, long long* stats) {
+#define MODEL_ARGS                                                                                                    \
+    int N, int T, int E, int K, int S, int C, const float *mass, const int *flags, const int *tri,                   \
+        const float *tri_mat, const int *edge, const float *bend, const int *tet, const float *tet_mat,              \
+        const int *at_off, const int *at, const int *ae_off, const int *ae, const int *ak_off, const int *ak,        \
+        const int *spring, const int *color_off, const int *color_particles
+#define MODEL_NAMES                                                                                                    \
+    N, T, E, K, S, C, mass, flags, tri, tri_mat, edge, bend, tet, tet_mat, at_off, at, ae_off, ae, ak_off, ak, spring, \
+        color_off, color_particles
+
+static HostModel host_model(MODEL_ARGS) {
     HostModel m;
     m.N = N, m.T = T, m.E = E, m.K = K, m.S = S;
     m.mass.assign(mass, mass + N);
@@ -43,6 +47,12 @@ extern "C" int check_layout(int N, int T, int E, int K, int S, int C, const floa
     m.spring_kd.assign(S, 1.0f);
     m.color_off.assign(color_off, color_off + C + 1);
     m.color_particles.assign(color_particles, color_particles + N);
+    return m;
+}
+
+// v: the model's arrays in HostModel order; stats: {batches, slow vertices, items, list stride}
+extern "C" int check_layout(MODEL_ARGS, int cap, int max_v, int aligned, long long* stats) {
+    const HostModel m = host_model(MODEL_NAMES);
     PassLayout L;
     if (!build_pass_layout(m, L, cap, max_v, aligned != 0).empty()) return -1;
 
@@ -154,5 +164,39 @@ extern "C" int check_layout(int N, int T, int E, int K, int S, int C, const floa
     for (int v = 0; v < N; ++v) CHECK(done[v]);
     CHECK(items == L.fast_items);
     stats[0] = B, stats[1] = (long long)L.slow_pos.size(), stats[2] = items, stats[3] = sh.list_stride;
+    return 0;
+}
+
+// Layouts that differ in damping only, zero or not, may be written over one another under a captured graph: the same
+// array sizes, batch ranges and launch arguments; the batch flags tell what each batch reads.
+extern "C" int check_damping_edit(MODEL_ARGS, int cap, int max_v, int aligned) {
+    const HostModel base = host_model(MODEL_NAMES);
+    PassLayout L[4];
+    for (int i = 0; i < 4; ++i) {
+        HostModel m = base;
+        for (int t = 0; t < T; ++t) m.tri_mat[5 * (size_t)t + 2] = i & 1 ? 0.5f : 0.0f;
+        for (int k = 0; k < K; ++k) m.tet_mat[3 * (size_t)k + 2] = i & 1 ? 0.5f : 0.0f;
+        for (int e = 0; e < E; ++e) m.edge_bend[2 * (size_t)e + 1] = i & 2 ? 0.25f : 0.0f;
+        if (!build_pass_layout(m, L[i], cap, max_v, aligned != 0).empty()) return -1;
+    }
+    for (int i = 1; i < 4; ++i) {
+        CHECK(L[i].shape == L[0].shape && L[i].batch_blk.size() == L[0].batch_blk.size());
+        CHECK(L[i].item_rec.size() == L[0].item_rec.size() && L[i].list == L[0].list);
+        CHECK(L[i].tri_rec.size() == L[0].tri_rec.size() && L[i].tet_rec.size() == L[0].tet_rec.size());
+        CHECK(L[i].hinge_damp.size() == L[0].hinge_damp.size() && L[i].spr_rec.size() == L[0].spr_rec.size());
+        CHECK(L[i].fast_color_off == L[0].fast_color_off && L[i].slow_color_off == L[0].slow_color_off);
+    }
+    const int B = L[0].fast_color_off[C];
+    for (int i = 0; i < 4; ++i)
+        for (int b = 0; b < B; ++b) {
+            int want = 0;
+            for (int t = 0; t < cap; ++t) {
+                const int meta = L[i].item_rec[((size_t)b * cap + t) * kItemWords + 1], kind = meta >> 12;
+                const bool hinge = kind == kHinge && (i & 2), other = (kind == kTri || kind == kTet) && (i & 1);
+                CHECK((meta >> 11 & 1) == (hinge || other || kind == kSpring));
+                want |= hinge ? kPrevAll | kHingeDamped : (other || kind == kSpring ? kPrevAll : 0);
+            }
+            CHECK(L[i].batch_blk[(size_t)b * L[i].blk_words + 3] == want);
+        }
     return 0;
 }

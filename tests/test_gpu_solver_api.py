@@ -84,6 +84,54 @@ def test_notify_model_changed_keeps_context_shape_and_graphs(cuda_device):
         np.testing.assert_array_equal(s1.particle_qd.cpu().numpy(), qd_ref)
 
 
+@pytest.mark.parametrize("shape", [(192, 1, True), (256, 7, False)])
+def test_damping_edits_reach_a_captured_graph(cuda_device, shape):
+    """Damping of triangles and hinges switched on from zero, and off again, is written into the existing layout
+    (test_pass_layout.py checks that no launch argument depends on it): a graph captured before replays with the new
+    values, bit-exact against the oracle."""
+    import torch
+
+    from newton_amd import scenes
+    from newton_amd.solvers import SolverVBD
+
+    model, state, info = scenes.cloth_hanging(cuda_device, verts_per_side=17)
+    dt = info["dt"]
+    q0, _ = initial(state)
+    qd0 = np.random.default_rng(3).normal(0.0, 0.5, q0.shape).astype(np.float32)
+    qd0[model.particle_inv_mass.cpu().numpy() == 0.0] = 0.0
+    model.tri_materials[:, 2] = 0.0
+    model.edge_bending_properties[:, 1] = 0.0
+    solver = SolverVBD(model, iterations=info["iterations"])
+    solver.set_pass_shape(*shape)
+    s1 = model.state()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        solver.step(state, s1, None, None, dt)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            solver.step(state, s1, None, None, dt)
+    torch.cuda.synchronize()
+    seen = []
+    for tri_kd, edge_kd in ((0.0, 0.0), (1.0, 0.0), (0.0, 1.0e-2), (1.0, 1.0e-2), (0.0, 0.0)):
+        model.tri_materials[:, 2] = tri_kd
+        model.edge_bending_properties[:, 1] = edge_kd
+        solver.notify_model_changed()
+        om = oracle.OracleModel(model)
+        _, q_ref, qd_ref = oracle.step(om, oracle.params(info["iterations"]), q0, qd0, None, None, dt)
+        for _ in range(2):
+            state.particle_q.copy_(torch.as_tensor(q0, device=cuda_device))
+            state.particle_qd.copy_(torch.as_tensor(qd0, device=cuda_device))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(s1.particle_q.cpu().numpy(), q_ref)
+            np.testing.assert_array_equal(s1.particle_qd.cpu().numpy(), qd_ref)
+        seen.append(q_ref)
+    assert all(np.abs(q - seen[0]).max() > 0.0 for q in seen[1:4])
+
+
 def test_pass_shape_survives_context_regrowth(cuda_device):
     """A larger soft-contact buffer re-creates the context; the chosen pass shape is re-applied."""
     from newton_amd import CollisionPipeline, scenes

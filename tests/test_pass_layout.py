@@ -19,7 +19,7 @@ def check(tmp_path_factory):
     so = tmp_path_factory.mktemp("layout") / "layout_check.so"
     subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", str(so), str(HERE / "layout_check.cpp")],
                    check=True)
-    return ctypes.CDLL(str(so)).check_layout
+    return ctypes.CDLL(str(so))
 
 
 def _fan(segments):
@@ -50,10 +50,8 @@ MODELS = {
 }
 
 
-@pytest.mark.parametrize("name", sorted(MODELS))
-@pytest.mark.parametrize("block,aligned", [(256, 0), (256, 1), (192, 0), (192, 1), (128, 0), (128, 1)])
-def test_layout(check, name, block, aligned):
-    m = MODELS[name]()
+def _model_args(m):
+    """The leading arguments of layout_check.cpp's functions, and the arrays they point to."""
     adj = m.soft_mesh_adjacency
     co, cp = color_layout(m)
 
@@ -67,10 +65,28 @@ def test_layout(check, name, block, aligned):
             arr(adj.v_adj_tris_offsets, i), arr(adj.v_adj_tris, i), arr(adj.v_adj_edges_offsets, i),
             arr(adj.v_adj_edges, i), arr(adj.v_adj_tets_offsets, i), arr(adj.v_adj_tets, i),
             arr(m.spring_indices if m.spring_count else None, i), co, cp]
+    return [m.particle_count, m.tri_count, m.edge_count, m.tet_count, int(m.spring_count), len(co) - 1,
+            *[a.ctypes.data_as(ctypes.c_void_p) for a in keep]], keep
+
+
+@pytest.mark.parametrize("name", sorted(MODELS))
+@pytest.mark.parametrize("block,aligned", [(256, 0), (256, 1), (192, 0), (192, 1), (128, 0), (128, 1)])
+def test_layout(check, name, block, aligned):
+    m = MODELS[name]()
+    args, keep = _model_args(m)
     stats = (ctypes.c_longlong * 4)()
-    rc = check(m.particle_count, m.tri_count, m.edge_count, m.tet_count, int(m.spring_count), len(co) - 1,
-               *[a.ctypes.data_as(ctypes.c_void_p) for a in keep], block, block // 12, aligned, stats)
+    rc = check.check_layout(*args, block, block // 12, aligned, stats)
     assert rc == 0, f"layout_check.cpp:{rc}"
     assert stats[0] + stats[1] > 0
     if name == "fan_120":
         assert stats[1] >= 1
+
+
+@pytest.mark.parametrize("name", ["cloth_17", "springs", "cube", "fan_80"])
+@pytest.mark.parametrize("block,aligned", [(256, 0), (192, 1)])
+def test_damping_edit_keeps_the_layout(check, name, block, aligned):
+    """Damping switched from or to zero changes no array size, batch range or launch argument, so a rebuild writes in
+    place under captured graphs."""
+    args, keep = _model_args(MODELS[name]())
+    rc = check.check_damping_edit(*args, block, block // 12, aligned)
+    assert rc == 0, f"layout_check.cpp:{rc}"
