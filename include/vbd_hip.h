@@ -132,7 +132,9 @@ typedef struct VbdSolverParams {
 typedef struct VbdContactsDesc {
     const int32_t* soft_contact_count;  /* [1] device */
     int32_t soft_contact_max;
-    const int32_t* soft_contact_indices; /* [S,3] (p,-1,-1) particle, (v0,v1,-1) edge, (v0,v1,v2) face records */
+    /* [S,3] (p,-1,-1) particle, (v0,v1,-1) edge, (v0,v1,v2) face records; the corners of an edge or face record are
+     * those of one of the model's edges or triangles, or of distinct colors */
+    const int32_t* soft_contact_indices;
     const int32_t* soft_contact_shape;
     const float* soft_contact_body_pos;  /* body frame of the shape's body (world for static shapes) */
     const float* soft_contact_body_vel;

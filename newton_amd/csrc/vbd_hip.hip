@@ -786,6 +786,9 @@ struct KParams {
     const float* c_body_vel;
     const float* c_normal;
     const int* pos_coff;
+    // set for full-surface contexts whose edges or faces hold corners of one color (vbd_layout::PassShape): every
+    // packed entry's row (force 3 + Hessian 9) at the pass start, from k_contact_rows
+    float* crows;
     const float* shape_margin;
     int shape_count;
 };
@@ -869,6 +872,21 @@ __device__ __forceinline__ void eval_packed_contact(const KParams& P, const floa
                                                     V3& f, M3& h) {
     const float4* c4 = reinterpret_cast<const float4*>(P.cpack) + 4 * (size_t)rec;
     eval_contact_rec(P, q, rec, c4[0], c4[1], c4[2], c4[3], dt, f, h);
+}
+
+// The rows of every packed contact entry of the color positions [p_lo, p_hi) at the positions q of the pass start (a
+// grid-stride loop over the device-sized entry range), for contexts with crows: an entry of theirs may read a corner
+// that the same pass moves.
+constexpr int kContactRowsGrid = 1024;  // work-groups of its grid-stride loop
+__global__ __launch_bounds__(256) void k_contact_rows(KParams P, const float* __restrict__ q, int p_lo, int p_hi,
+                                                      float dt) {
+    const int j0 = P.pos_coff[p_lo], j1 = P.pos_coff[p_hi];
+    for (int j = j0 + (int)(blockIdx.x * blockDim.x + threadIdx.x); j < j1; j += (int)(gridDim.x * blockDim.x)) {
+        V3 f;
+        M3 h;
+        eval_packed_contact(P, q, j, dt, f, h);
+        store_row(P.crows + (size_t)kComp * j, f, h);
+    }
 }
 
 // evaluate_spring_force_and_hessian_both_vertices (particle_vbd_kernels.py:1685-1730), the
@@ -1032,7 +1050,8 @@ constexpr int kBatchHdr = vbd_layout::kBatchWords;
 enum PassKinds { kClothKinds = 0, kClothSpringKinds = 1, kTetKinds = 2, kAllKinds = 3 };
 // Added to the kinds of a context whose contacts include edge/face records.  A pass evaluates those itself, their
 // corners read from memory and in parts when they outnumber the rows; a kernel of their rows took 8.5 us before each
-// pass (256x256 cloth on moving bodies, substep 988 -> 716 us).  Kept apart from the other passes: compiled into
+// pass (256x256 cloth on moving bodies, substep 988 -> 716 us).  That kernel, k_contact_rows, serves models whose
+// edges or faces hold corners of one color, where the pass itself moves what the entries read.  Kept apart from the other passes: compiled into
 // them it cost their occupancy (substeps of 512 cloth worlds 1,160 -> 1,354 us, of a 256x256 cloth 395 -> 437 us).
 constexpr int kEdgeFace = 4;
 // Added for self-contact, whose rows k_sc_rows evaluates (contacts crowd in a few batches: evaluated in the pass, it
@@ -1149,7 +1168,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
         if (t < nv) live = own_live = P.w_active[P.p_world[vr.x]] != 0;
         if (!__syncthreads_or(live)) return;
     }
-    const bool par_contacts = nstatic + ncont <= ROWS;
+    // a pass that moves nothing (FORCE_ONLY) may read any corner
+    const bool stored = EF && !FORCE_ONLY && P.crows;
+    const bool par_contacts = !stored && nstatic + ncont <= ROWS;
     const int npar = par_contacts ? ncont : 0;
 
     // ---- round trip 2
@@ -1207,7 +1228,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
         return v3(v.x, v.y, v.z);
     };
     // the batch's packed contact k: its vertex's staged positions, or the corners of an edge/face record, which are of
-    // other colors (no pass moves them while this one reads them)
+    // other colors (no pass moves them while this one reads them; otherwise the rows are stored)
     auto contact = [&](int k, V3& f, M3& h) {
         const float4* c4 = reinterpret_cast<const float4*>(P.cpack) + 4 * (size_t)(cbeg + k);
         const float4 A = c4[0], B = c4[1], C = c4[2], D = c4[3];
@@ -1289,7 +1310,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
         const int c0 = s_cb[cs], c1 = s_cb[cs + 1];
         if (par_contacts) {
             for (int r = c0; r < c1; ++r) ca = ca + s_rows[(nstatic + r) * NC + cc];
-        } else if constexpr (!EF) {
+        } else if constexpr (EF) {
+            if (stored) ca = add_rows_in_order(ca, P.crows + (size_t)kComp * cbeg, c0, c1, full_component<SYM>(cc));
+        } else {
             for (int r = c0; r < c1; ++r) {
                 V3 fc;
                 M3 hc;
@@ -1299,7 +1322,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
         }
     }
     if constexpr (EF) {
-        if (!par_contacts) {
+        if (!par_contacts && !stored) {
             // a part at a time, over the rows already summed (spring rows are still needed)
             const int base = SPRING ? nstatic : 0, room = ROWS - base;
             for (int k0 = 0; k0 < ncont; k0 += room) {
@@ -1465,7 +1488,10 @@ __global__ __launch_bounds__(kBlock) void k_solve_generic(KParams P, float* __re
             for (int j = c0; j < c1; ++j) {
                 V3 fc;
                 M3 hc;
-                eval_packed_contact(P, q, j, dt, fc, hc);
+                if (P.crows && mode == 0)
+                    load_row(P.crows + (size_t)kComp * j, fc, hc);
+                else
+                    eval_packed_contact(P, q, j, dt, fc, hc);
                 cf = add(cf, fc);
                 ch = madd(ch, hc);
             }
@@ -2396,6 +2422,7 @@ struct VbdContext {
     int* pos_coff = nullptr;    // [N+1]
     float* cpack = nullptr;     // [entry_cap * 16]
     int* cpack_ef = nullptr;    // [entry_cap * 8] corners and weights of edge/face entries (full surface only)
+    float* crows = nullptr;     // [entry_cap * 12] contact rows of a pass (full surface with shared_corners only)
     int* cid_to_pack = nullptr; // [cap * 3] packed entry of each (contact, corner), -1 when none
     float* g_tmp = nullptr;     // [N,3] residual scratch
     double* r_part = nullptr;   // residual partial sums, one per first-stage workgroup
@@ -2654,6 +2681,13 @@ int32_t build_layout(VbdContext* c) {
     k.tri_rec = c->lay_tri;
     k.hinge_damp = reinterpret_cast<const float*>(c->lay_hinge_damp);
     k.tet_rec = c->lay_tet;
+    hipFree(c->crows);
+    c->crows = nullptr;
+    if (c->params.soft_contact_full_surface && L.shape.shared_corners) {
+        hipError_t e = hipMalloc(&c->crows, sizeof(float) * kComp * c->entry_cap);
+        if (e != hipSuccess) return fail(VBD_ERR_HIP, std::string("vbd_create: contact rows: ") + hipGetErrorString(e));
+    }
+    k.crows = c->crows;
     c->shape = L.shape;
     k.tri_hi = L.shape.tri.hi;
     k.hinge_lo = L.shape.hinge.lo;
@@ -3173,6 +3207,7 @@ int32_t vbd_destroy(VbdContext* c) {
     hipFree(c->c_state);
     hipFree(c->cpack);
     hipFree(c->cpack_ef);
+    hipFree(c->crows);
     hipFree(c->g_tmp);
     hipFree(c->r_part);
     hipFree(c->r_dev);
@@ -3412,9 +3447,18 @@ int32_t launch_spring_rows(VbdContext* c, hipStream_t s, int j0, int j1, const f
     return VBD_OK;
 }
 
+int32_t launch_contact_rows(VbdContext* c, hipStream_t s, int p_lo, int p_hi, const float* q, float dt) {
+    if (!c->crows || !c->have_contacts || p_hi <= p_lo) return VBD_OK;
+    hipLaunchKernelGGL(k_contact_rows, dim3(kContactRowsGrid), dim3(256), 0, s, c->kp, q, p_lo, p_hi, dt);
+    VBD_LAUNCH_CHECK("k_contact_rows");
+    return VBD_OK;
+}
+
 int32_t launch_color(VbdContext* c, hipStream_t s, int color, float* q, float dt, int mode, float* g) {
     set_dt(c, dt);
     int32_t rc0 = launch_spring_rows(c, s, c->pre_color_off[color], c->pre_color_off[color + 1], q, dt);
+    if (rc0) return rc0;
+    rc0 = launch_contact_rows(c, s, c->color_offsets[color], c->color_offsets[color + 1], q, dt);
     if (rc0) return rc0;
     if (c->self_on) {
         hipLaunchKernelGGL(k_sc_rows, dim3(kSelfGrid), dim3(256), 0, s, c->sp, q, c->kp.q_prev,

@@ -120,9 +120,13 @@ struct LaneRange {
 struct PassShape {
     LaneRange tri, hinge, tet, spring;
     int list_stride = 0;  // entries of a batch's vertex list
+    // Two corners of some edge or triangle share a color (elements without stiffness are not part of the coloring
+    // graph): a pass moves one corner of their edge/face contacts while another's entry reads it, so those entries'
+    // rows are evaluated before the pass.
+    bool shared_corners = false;
     bool operator==(const PassShape& o) const {
         return tri == o.tri && hinge == o.hinge && tet == o.tet && spring == o.spring &&
-               list_stride == o.list_stride;
+               list_stride == o.list_stride && shared_corners == o.shared_corners;
     }
 };
 
@@ -183,6 +187,14 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
     std::vector<int32_t> color_of((size_t)N, -1);
     for (int c = 0; c < C; ++c)
         for (int k = m.color_off[c]; k < m.color_off[c + 1]; ++k) color_of[m.color_particles[k]] = c;
+    auto same = [&](int a, int b) { return a >= 0 && a < N && b >= 0 && b < N && color_of[a] == color_of[b]; };
+    bool shared_corners = false;
+    for (int t = 0; t < m.T && !shared_corners; ++t) {
+        const int32_t* c = &m.tri_idx[3 * (size_t)t];
+        shared_corners = same(c[0], c[1]) || same(c[1], c[2]) || same(c[2], c[0]);
+    }
+    for (int e = 0; e < m.E && !shared_corners; ++e)
+        shared_corners = same(m.edge_idx[4 * (size_t)e + 2], m.edge_idx[4 * (size_t)e + 3]);
     // per-vertex spring items in spring-index order: 2 * spring + endpoint
     std::vector<int32_t> vs_off((size_t)N + 1, 0), vs_item;
     for (int s = 0; s < m.S; ++s)
@@ -224,6 +236,7 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
     L.cap = cap;
     L.max_v = max_v;
     L.blk_words = block_words(max_v);
+    L.shape.shared_corners = shared_corners;
     L.vert_rec.assign((size_t)N * kVertWords, 0);
     L.fast_color_off.assign((size_t)C + 1, 0);
     L.slow_color_off.assign((size_t)C + 1, 0);

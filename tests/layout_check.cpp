@@ -200,3 +200,11 @@ extern "C" int check_damping_edit(MODEL_ARGS, int cap, int max_v, int aligned) {
         }
     return 0;
 }
+
+// 1 when two corners of some edge or triangle share a color, 0 when not
+extern "C" int shares_corners(MODEL_ARGS, int cap, int max_v, int aligned) {
+    const HostModel m = host_model(MODEL_NAMES);
+    PassLayout L;
+    if (!build_pass_layout(m, L, cap, max_v, aligned != 0).empty()) return -1;
+    return L.shape.shared_corners ? 1 : 0;
+}

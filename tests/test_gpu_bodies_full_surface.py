@@ -318,3 +318,60 @@ def test_full_surface_entries_beyond_the_pass_rows_bitexact(cuda_device, extra):
     assert np.isfinite(q).all()
     np.testing.assert_array_equal(s0.particle_q.cpu().numpy(), q)
     np.testing.assert_array_equal(s0.particle_qd.cpu().numpy(), qd)
+
+
+@pytest.mark.parametrize("beta", [0.0, 1.0e4])
+@pytest.mark.parametrize("hub", [False, True])
+def test_full_surface_corners_of_one_color_bitexact(cuda_device, hub, beta):
+    """A cloth of springs on a sphere and a plane: its triangles carry no stiffness, every particle has the same color,
+    and every entry of an edge or face contact reads corners that its own pass moves.  The hub joins 270 particles, more
+    than a pass holds: it takes the generic path, its contacts the same way."""
+    import torch
+
+    from newton_amd import CollisionPipeline, ModelBuilder
+    from newton_amd.solvers import SolverVBD
+
+    b = ModelBuilder(up_axis="Y", gravity=-9.81)
+    b.add_shape_sphere(-1, xform=((0.01, -0.5, 0.004), (0.0, 0.0, 0.0, 1.0)), radius=0.5,
+                       cfg=ModelBuilder.ShapeConfig(ke=1.0e3, kd=1.0, mu=0.3))
+    b.add_ground_plane(cfg=ModelBuilder.ShapeConfig(ke=1.0e3, kd=1.0, mu=0.4))
+    n = 17
+    b.add_cloth_grid(pos=(-0.1, 0.012, 0.1), rot=_quat((1.0, 0.0, 0.0), -math.pi / 2), vel=(0.1, -0.3, 0.0), dim_x=n - 1,
+                     dim_y=n - 1, cell_x=0.012, cell_y=0.012, mass=0.01, tri_ke=0.0, tri_ka=0.0, tri_kd=0.0, edge_ke=0.0,
+                     edge_kd=0.0, particle_radius=0.01)
+    for i in range(n * n):
+        if i % n != n - 1:
+            b.add_spring(i, i + 1, 50.0, 0.01)
+        if i + n < n * n:
+            b.add_spring(i, i + n, 50.0, 0.01)
+    if hub:
+        for i in range(n * n):
+            if i != 144 and i < 271:
+                b.add_spring(144, i, 0.5, 0.0)
+    b.color()
+    assert len(b.particle_color_groups) == 1
+    model = b.finalize(cuda_device)
+    model.soft_contact_ke, model.soft_contact_kd, model.soft_contact_mu = 1.0e3, 1.0, 0.3
+    q, qd = model.particle_q.cpu().numpy().copy(), model.particle_qd.cpu().numpy().copy()
+    margin, dt, substeps, iters = 0.02, 1.0 / 600.0, 4, 3
+    pipe = CollisionPipeline(model, soft_contact_margin=margin, enable_rigid_soft_full_surface_contact=True)
+    contacts = pipe.contacts()
+    solver = SolverVBD(model, iterations=iters, rigid_avbd_beta=beta)
+    s0, s1 = model.state(), model.state()
+    for _ in range(substeps):
+        s0.clear_forces()
+        pipe.collide(s0, contacts)
+        solver.step(s0, s1, None, contacts, dt)
+        s0, s1 = s1, s0
+    torch.cuda.synchronize()
+    assert (solver.layout_stats()["generic_vertices"] > 0) == hub
+    om = _full_oracle(model, pipe)
+    prm = oracle.params(iters, avbd_beta=beta, k_start=-1.0 if beta == 0.0 else solver.rigid_contact_k_start_value)
+    for _ in range(substeps):
+        c = oracle.Contacts(pipe.soft_contact_max)
+        k = oracle.create_soft_contacts(om, q, margin, c)
+        _, q, qd = oracle.step(om, prm, q, qd, None, c, dt)
+    assert np.any(c.indices[:k, 1] >= 0) and np.any(c.indices[:k, 2] >= 0)
+    assert np.isfinite(q).all()
+    np.testing.assert_array_equal(s0.particle_q.cpu().numpy(), q)
+    np.testing.assert_array_equal(s0.particle_qd.cpu().numpy(), qd)

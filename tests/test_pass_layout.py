@@ -90,3 +90,24 @@ def test_damping_edit_keeps_the_layout(check, name, block, aligned):
     args, keep = _model_args(MODELS[name]())
     rc = check.check_damping_edit(*args, block, block // 12, aligned)
     assert rc == 0, f"layout_check.cpp:{rc}"
+
+
+def _spring_cloth(tri_ke, tri_ka):
+    b = ModelBuilder(up_axis="Y")
+    b.add_cloth_grid(pos=(0.0, 0.0, 0.0), rot=(0.0, 0.0, 0.0, 1.0), vel=(0.0, 0.0, 0.0), dim_x=5, dim_y=4, cell_x=0.1,
+                     cell_y=0.1, mass=0.1, tri_ke=tri_ke, tri_ka=tri_ka, tri_kd=0.0, edge_ke=0.0, edge_kd=0.0)
+    for i in range(29):
+        if i % 6 != 5:
+            b.add_spring(i, i + 1, 10.0, 0.0)
+    b.color()
+    return b.finalize("cpu")
+
+
+@pytest.mark.parametrize("name,shared", [("cloth_17", 0), ("springs", 0), ("cube", 0), ("fan_80", 0), ("rope", 0),
+                                         ("springs_only", 1), ("no_area_term", 1)])
+def test_corners_of_one_color_are_found(check, name, shared):
+    """Triangles without stiffness are not part of the coloring graph: their corners, and those of their edges, may
+    share a color, and a color pass then moves what an edge or face contact of the same pass reads."""
+    build = {"springs_only": lambda: _spring_cloth(0.0, 0.0), "no_area_term": lambda: _spring_cloth(1.0e3, 0.0)}
+    args, keep = _model_args(build.get(name, MODELS.get(name))())
+    assert check.shares_corners(*args, 256, 21, 0) == shared
