@@ -1833,6 +1833,19 @@ __global__ __launch_bounds__(256) void k_contact_pack(int n, const int* __restri
     }
 }
 
+// The batch slot of every packed entry's vertex, after the layout was built anew under packed contacts: a pass takes the
+// vertex's staged positions by it.
+__global__ __launch_bounds__(256) void k_contact_slots(int n, const int* __restrict__ vert_rec,
+                                                       const int* __restrict__ pos_coff, float* __restrict__ cpack) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const int slot = vert_rec[4 * k + 3] & 0xffff;
+    for (int j = pos_coff[k]; j < pos_coff[k + 1]; ++j) {
+        int* word = reinterpret_cast<int*>(cpack) + kContactWords * (size_t)j + 1;
+        *word = (*word & kContactEF) | slot;
+    }
+}
+
 // Contact range of every batch from the color-position offsets: the first packed
 // contact and count (cinfo) and the max_v + 1 vertex offsets relative to the first
 // (coff), so the color pass reads them indexed by batch in its first round trip.
@@ -2539,6 +2552,23 @@ void set_batch_particle_ranges(VbdContext* c, const vbd_layout::PassLayout& L) {
     c->bw_key.clear();
 }
 
+int32_t launch_batch_contacts(VbdContext* c, hipStream_t s) {
+    const int nbat = c->fast_color_off.back();
+    if (nbat <= 0) return VBD_OK;
+    hipLaunchKernelGGL(k_batch_contacts, dim3(blocks_for(nbat, 256)), dim3(256), 0, s, nbat, c->lay_batch,
+                       c->blk_words, c->max_v, c->pos_coff, c->bat_cinfo, c->bat_coff);
+    VBD_LAUNCH_CHECK("k_batch_contacts");
+    return VBD_OK;
+}
+
+// The substep's packed contacts under a layout built anew: their vertices' slots and the batches' contact ranges.
+int32_t carry_contacts(VbdContext* c, hipStream_t s) {
+    const int N = c->model.particle_count;
+    hipLaunchKernelGGL(k_contact_slots, dim3(blocks_for(N, 256)), dim3(256), 0, s, N, c->lay_vert, c->pos_coff, c->cpack);
+    VBD_LAUNCH_CHECK("k_contact_slots");
+    return launch_batch_contacts(c, s);
+}
+
 // Reads the model arrays back once and builds the color-pass layout on the host (vbd_layout.h).
 int32_t build_layout(VbdContext* c) {
     const VbdModelDesc* m = &c->model;
@@ -2621,12 +2651,8 @@ int32_t build_layout(VbdContext* c) {
         c->fast_items = L.fast_items;
         set_batch_particle_ranges(c, L);
         // the batches may hold other vertices now: recompute their contact ranges of the current substep
-        const int nbat = c->fast_color_off.back();
-        if (nbat > 0) {
-            hipLaunchKernelGGL(k_batch_contacts, dim3(blocks_for(nbat, 256)), dim3(256), 0, 0, nbat, c->lay_batch,
-                               c->blk_words, c->max_v, c->pos_coff, c->bat_cinfo, c->bat_coff);
-            VBD_LAUNCH_CHECK("k_batch_contacts");
-        }
+        const int32_t rc = carry_contacts(c, 0);
+        if (rc) return rc;
         VBD_HIP_TRY(hipDeviceSynchronize());
         return VBD_OK;
     }
@@ -3295,15 +3321,6 @@ static BodyPoses body_poses(const VbdContext* c) {
     return B;
 }
 
-static int32_t launch_batch_contacts(VbdContext* c, hipStream_t s) {
-    const int nbat = c->fast_color_off.back();
-    if (nbat <= 0) return VBD_OK;
-    hipLaunchKernelGGL(k_batch_contacts, dim3(blocks_for(nbat, 256)), dim3(256), 0, s, nbat, c->lay_batch,
-                       c->blk_words, c->max_v, c->pos_coff, c->bat_cinfo, c->bat_coff);
-    VBD_LAUNCH_CHECK("k_batch_contacts");
-    return VBD_OK;
-}
-
 int32_t vbd_contact_prepare(VbdContext* c, void* stream, const VbdContactsDesc* cd) {
     if (!c) return fail(VBD_ERR_ARG, "vbd_contact_prepare: null context");
     hipStream_t s = (hipStream_t)stream;
@@ -3597,7 +3614,7 @@ int32_t vbd_set_block_shape(VbdContext* c, void* stream, int32_t block) {
     c->block = block;
     int32_t rc = build_layout(c);
     if (rc) return rc;
-    rc = launch_batch_contacts(c, (hipStream_t)stream);
+    rc = carry_contacts(c, (hipStream_t)stream);
     if (rc) return rc;
     VBD_HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
     return VBD_OK;
@@ -3609,7 +3626,7 @@ int32_t vbd_set_aligned_items(VbdContext* c, void* stream, int32_t aligned) {
     c->aligned = aligned;
     int32_t rc = build_layout(c);
     if (rc) return rc;
-    rc = launch_batch_contacts(c, (hipStream_t)stream);
+    rc = carry_contacts(c, (hipStream_t)stream);
     if (rc) return rc;
     VBD_HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
     return VBD_OK;
@@ -3631,7 +3648,7 @@ int32_t vbd_set_pass_shape(VbdContext* c, void* stream, int32_t block, int32_t w
     c->aligned = aligned;
     int32_t rc = build_layout(c);
     if (rc) return rc;
-    rc = launch_batch_contacts(c, (hipStream_t)stream);
+    rc = carry_contacts(c, (hipStream_t)stream);
     if (rc) return rc;
     VBD_HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
     return VBD_OK;
@@ -3676,7 +3693,7 @@ int32_t vbd_autotune(VbdContext* c, void* stream, const float* q, float dt, int3
             c->aligned = align[k];
             rc = build_layout(c);
             if (rc) break;
-            rc = launch_batch_contacts(c, s);
+            rc = carry_contacts(c, s);
             if (rc) break;
         }
         // warm, then time three force-assembly passes over every color (q is only read)
@@ -3703,7 +3720,7 @@ int32_t vbd_autotune(VbdContext* c, void* stream, const float* q, float dt, int3
         c->aligned = align[best];
         rc = build_layout(c);
         if (rc) return rc;
-        rc = launch_batch_contacts(c, s);
+        rc = carry_contacts(c, s);
         if (rc) return rc;
         VBD_HIP_TRY(hipStreamSynchronize(s));
     }

@@ -173,3 +173,36 @@ def test_contact_scalars_are_read_per_step(cuda_device):
     oracle.create_soft_contacts(om, q0, 0.05, oc)
     _, q_ref, _ = oracle.step(om, oracle.params(info["iterations"]), q0, qd0, None, oc, info["dt"])
     np.testing.assert_array_equal(s1.particle_q.cpu().numpy(), q_ref)
+
+
+@pytest.mark.parametrize("before", [(256, 1, False), (192, 7, True)])
+@pytest.mark.parametrize("after", [(128, 1, False), (192, 1, True), (256, 7, False)])
+def test_pass_shape_chosen_between_preparation_and_iterations(cuda_device, before, after):
+    """Contacts packed under one pass shape belong to the same vertices under another: the shape may change between
+    begin_step and iterate, bit-exact against the oracle's step."""
+    import torch
+
+    from newton_amd import CollisionPipeline, scenes
+    from newton_amd.solvers import SolverVBD
+
+    model, state, info = scenes.cloth_drop_on_sphere(cuda_device, verts_per_side=24)
+    state.particle_q[:, 1] = 0.1 + 0.002 * torch.sin(37.0 * state.particle_q[:, 0])  # every particle near the ground
+    q0, qd0 = initial(state)
+    pipe = CollisionPipeline(model, soft_contact_margin=0.02)
+    contacts = pipe.contacts()
+    solver = SolverVBD(model, iterations=4)
+    solver.set_pass_shape(*before)
+    s1 = model.state()
+    pipe.collide(state, contacts)
+    solver.begin_step(state, contacts, info["dt"])
+    solver.iterate(state, info["dt"], 1)
+    solver.set_pass_shape(*after)
+    solver.iterate(state, info["dt"], 3)
+    solver.end_step(state, s1, info["dt"])
+    torch.cuda.synchronize()
+    om = oracle.OracleModel(model)
+    oc = oracle.Contacts(pipe.soft_contact_max)
+    assert oracle.create_soft_contacts(om, q0, 0.02, oc) > 400
+    _, q_ref, qd_ref = oracle.step(om, oracle.params(4), q0, qd0, None, oc, info["dt"])
+    np.testing.assert_array_equal(s1.particle_q.cpu().numpy(), q_ref)
+    np.testing.assert_array_equal(s1.particle_qd.cpu().numpy(), qd_ref)
