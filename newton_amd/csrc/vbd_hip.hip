@@ -35,6 +35,7 @@
 
 #include "vbd_hip.h"
 #include "vbd_layout.h"
+#include "vbd_scalar.h"
 
 namespace {
 
@@ -624,19 +625,14 @@ __device__ void eval_contact(V3 x, V3 x_prev, V3 bx, V3 bv, V3 n, float radius, 
     h_out = hess;
 }
 
-// True when the Frobenius condition number of h is certainly far below 1e6, from single precision alone:
-// ||adj H||_F <= ||H||_F^2 / sqrt(3), so cond <= ||H||_F^3 / (sqrt(3) |det H|); the computed determinant is
-// within 5 roundings of perm|H| <= ||H||_F^3 (3e-7 of it), so |det| >= 4e-6 ||H||_F^3 bounds the condition by
-// 1.6e5.  An overflow or a NaN fails the comparison (the double-precision test decides then); an underflow of a
-// square cannot matter, |det| > 1e-8 keeps ||H||_F above 2e-3.
+// The screen of vbd_scalar.h for the block h with its computed determinant.
 __device__ __forceinline__ bool well_conditioned(const M3& h, float det) {
     float n1 = 0.0f;
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j) n1 += h.m[i][j] * h.m[i][j];
-    const float r = __builtin_amdgcn_rsqf(n1);
-    return fabsf(det) * r * r * r >= 4.0e-6f;
+    return vbd_scalar::certainly_well_conditioned(det, __builtin_amdgcn_rsqf(n1));
 }
 
 // Guarded 3x3 solve, particle_vbd_kernels.py:2701-2706: returns false when |det H| <= 1e-8.  With

@@ -220,6 +220,55 @@ def test_condition_screen_bitexact(cuda_device, mass):
     assert np.array_equal(q_gpu, q_ref) and np.array_equal(qd_gpu, qd_ref)
 
 
+def _held_by_three_springs(dev, stiff, soft):
+    """A particle at the origin on springs along x and y (stiff) and z (soft, stretched) to pinned particles: a block
+    of diagonal about (stiff, stiff, soft)."""
+    from newton_amd import ModelBuilder, ParticleFlags
+
+    b = ModelBuilder(up_axis="Y", gravity=0.0)
+    b.add_particle((0.0, 0.0, 0.0), (0.0, 0.0, 0.0), 1.0, radius=0.01, flags=int(ParticleFlags.ACTIVE))
+    for k in range(3):
+        at = [0.0, 0.0, 0.0]
+        at[k] = 1.0
+        b.add_particle(tuple(at), (0.0, 0.0, 0.0), 0.0, radius=0.01, flags=0)
+        b.add_spring(0, k + 1, soft if k == 2 else stiff, 0.0)
+    b.set_coloring([np.array([0]), np.array([1, 2, 3])])
+    model = b.finalize(dev)
+    model.spring_rest_length[2] = 0.9
+    return model, model.state(), {"dt": 1.0 / 600.0, "iterations": 1}
+
+
+@pytest.mark.parametrize("stiff,soft", [(1.0e16, 1.0e7), (3.0e15, 1.0e9), (1.0e13, 1.0e13), (1.0e18, 1.0e3)])
+def test_determinant_beyond_single_precision_bitexact(cuda_device, stiff, soft):
+    """Blocks whose single-precision determinant overflows while the squared norm does not: ill-conditioned ones are
+    solved in double precision, as the oracle does, which moves the particle."""
+    model, state, info = _held_by_three_springs(cuda_device, stiff, soft)
+    q0, qd0 = initial(state)
+    q_gpu, qd_gpu, _ = gpu_run(model, state, info, 1, solver_kwargs={"fp64_ill_conditioned": True})
+    q_ref, qd_ref, _ = oracle_run(model, q0, qd0, info, 1, fp64_ill_conditioned=True)
+    np.testing.assert_array_equal(q_gpu, q_ref)
+    np.testing.assert_array_equal(qd_gpu, qd_ref)
+    if stiff >= 1.0e6 * soft:
+        assert np.abs(q_ref[0]).max() > 1.0e-4
+
+
+def test_both_block_solves_are_taken_bitexact(cuda_device):
+    """Bead masses whose block conditions lie on both sides of the 1e6 at which the solve turns to double precision
+    (the oracle's result depends on it from 6e-8 down), around and beyond the screen's 1.6e5."""
+    from newton_amd import scenes
+
+    differ = []
+    for mass in (3.0e-7, 1.0e-7, 6.0e-8, 3.0e-8, 1.0e-8, 5.0e-9):
+        model, state, info = scenes.bead_rope_light(cuda_device, mass=mass)
+        q0, qd0 = initial(state)
+        q_gpu, qd_gpu, _ = gpu_run(model, state, info, 10, solver_kwargs={"fp64_ill_conditioned": True})
+        q_ref, qd_ref, _ = oracle_run(model, q0, qd0, info, 10, fp64_ill_conditioned=True)
+        np.testing.assert_array_equal(q_gpu, q_ref)
+        np.testing.assert_array_equal(qd_gpu, qd_ref)
+        differ.append(bool(np.any(oracle_run(model, q0, qd0, info, 10, fp64_ill_conditioned=False)[0] != q_ref)))
+    assert differ == [False, False, True, True, True, True]
+
+
 @pytest.mark.parametrize("scene", ["strip", "springs"])
 @pytest.mark.parametrize("case", ["flat", "tiny_parts", "shrunk", "stretched", "far_out"])
 def test_shared_quotient_ranges_bitexact(cuda_device, scene, case):
