@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <string>
 
+#include "vbd_scalar.h"
 #include "vbd_warmstart.h"
 
 namespace {
@@ -844,19 +845,6 @@ __device__ inline void put_columns(uint16_t* t, int col, int row, uint32_t lo, u
     t[(col + 3) * kTS + row] = (uint16_t)(hi >> 16);
 }
 
-// 1 / (1 + exp(-z)) to about an ulp, as expf and an IEEE division give it, in 11 instructions instead of 40: exp2 of
-// -z log2(e) with the product's low part put back, and the reciprocal with one Newton step.  The exponent is
-// held at 126 (a sigmoid below 2^-126 rounds to it), which keeps infinities out of the Newton step.
-__device__ inline float sigmoid_short(float z) {
-    const float l2e = 1.44269502f, l2e_lo = 1.92596299e-8f, ln2 = 0.693147182f;  // log2(e) in two parts
-    const float p = -z * l2e;
-    const float lo = __builtin_fmaf(-z, l2e, -p) - z * l2e_lo;
-    const float e = __builtin_amdgcn_exp2f(fminf(p, 126.0f));
-    const float d = 1.0f + __builtin_fmaf(e * ln2, lo, e);
-    const float r = __builtin_amdgcn_rcpf(d);
-    return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
-}
-
 // SiLU of the accumulators: the next operand, its columns in LDS, and silu'(z)
 __device__ inline void train_silu(const floatx4 (&acc)[8], bf16x8 (&b)[4], floatx4 (&dsilu)[8], uint16_t* t, int lq,
                                   int row) {
@@ -866,7 +854,7 @@ __device__ inline void train_silu(const floatx4 (&acc)[8], bf16x8 (&b)[4], float
         float h[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const float z = acc[nt][c], s = sigmoid_short(z);
+            const float z = acc[nt][c], s = vbd_scalar::sigmoid_short(z);
             h[c] = z * s;
             dsilu[nt][c] = s * (1.0f + z * (1.0f - s));
         }

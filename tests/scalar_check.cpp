@@ -12,3 +12,7 @@ extern "C" void screen(int n, const float* blocks, int* out) {
         out[i] = vbd_scalar::certainly_well_conditioned(det, 1.0f / sqrtf(n1)) ? 1 : 0;
     }
 }
+
+extern "C" void sigmoid(int n, const float* z, float* out) {
+    for (int i = 0; i < n; ++i) out[i] = vbd_scalar::sigmoid_short(z[i]);
+}

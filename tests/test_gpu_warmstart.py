@@ -162,6 +162,41 @@ def test_gradient_equals_its_pieces(cuda_device, n):
         assert bool((a == b).all())
 
 
+@pytest.mark.parametrize("n", [64, 100])
+def test_gradient_of_large_preactivations(cuda_device, n):
+    """Hidden units far outside the sigmoid's range, up to the largest a BF16 activation holds: SiLU and its derivative
+    are 0 and 0 or z and 1 there, and the gradient is the oracle's."""
+    import torch
+
+    from newton_amd.warmstart import WarmStartMLP
+
+    rng = np.random.default_rng(n)
+    big = np.array([-87.0, -88.0, -89.0, -104.0, -1.0e3, -1.0e4, -3.0e7, -3.3e8, -1.0e10, -1.0e12, -1.0e20, -1.0e30,
+                    -3.0e38, 30.0, 88.0, 1.0e3, 1.0e4], np.float32)
+    named = {name: rng.normal(0, 0.1, shape) for name, shape in mo.SHAPES}
+    for layer in (1, 2, 3):
+        named[f"W{layer}"][:, :len(big)] = 0.0
+        named[f"b{layer}"] = named[f"b{layer}"].reshape(-1)
+        named[f"b{layer}"][:len(big)] = big
+        named[f"W{layer + 1}"][len(big) - 4:len(big)] *= 1.0e-4  # the positive ones are the next layer's inputs
+    p = mo.pack(named).astype(np.float32)
+    mlp = WarmStartMLP(cuda_device, seed=2)
+    mlp.load_params(p)
+    x = _rand_feat(rng, n)
+    t = rng.normal(0, 1, (n, 3)).astype(np.float32)
+    loss, grad = mlp.gradient(_to_dev_bf16(x, cuda_device), torch.as_tensor(t, device=cuda_device))
+    torch.cuda.synchronize()
+    with np.errstate(over="ignore"):
+        ref_loss, ref = mo.loss_and_grad(x, p.astype(np.float64), t, None, bf16=True)
+    g = grad.cpu().numpy().astype(np.float64)
+    assert np.isfinite(g).all() and np.isfinite(ref).all()
+    assert abs(float(loss.item()) - ref_loss) <= 1e-3 * ref_loss
+    G, R = mo.unpack(g), mo.unpack(ref)
+    for name, _ in mo.SHAPES:
+        a, b = G[name].reshape(-1), R[name].reshape(-1)
+        assert np.linalg.norm(a - b) <= 2e-2 * np.linalg.norm(b), name
+
+
 def test_adam_matches_oracle(cuda_device):
     import torch
 

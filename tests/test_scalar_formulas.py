@@ -69,3 +69,30 @@ def test_screen_clears_ordinary_blocks(lib, scale):
         s = np.array([1.0, 1.0, 1.0 / condition])
         cleared, _ = _screen(lib, scale * np.einsum("nij,j,nkj->nik", u, s, u))
         assert cleared.all(), condition
+
+
+def _sigmoid(lib, z):
+    z = np.ascontiguousarray(z, np.float32)
+    out = np.full(len(z), 7.0, np.float32)
+    lib.sigmoid(len(z), z.ctypes.data_as(ctypes.c_void_p), out.ctypes.data_as(ctypes.c_void_p))
+    return out
+
+
+def test_sigmoid_within_its_range(lib):
+    """Against 64 bits: exp2 (an ulp), the product's and the sum's roundings and the reciprocal's leave about three
+    ulps; half an ulp of the argument of exp2 that the low part restores would be worth 40 of them at z = -80."""
+    z = np.concatenate([np.linspace(-87.33, 88.0, 200001), np.random.default_rng(1).normal(0, 3, 100000)])
+    z = z.astype(np.float32)
+    with np.errstate(over="ignore"):
+        ref = 1.0 / (1.0 + np.exp(-z.astype(np.float64)))
+    assert np.max(np.abs(_sigmoid(lib, z) - ref) / ref) <= 4.0 * 2.0 ** -23
+
+
+def test_sigmoid_far_outside_its_range(lib):
+    """0 below 2^-126 and 1 above, up to infinity, as 1 / (1 + expf(-z)) gives them (its denormals aside); the order
+    is kept all the way."""
+    far = np.array([-np.inf, -3.4e38, -1e30, -1e12, -1e10, -3.3e8, -3.0e7, -1e4, -104.0, -89.0], np.float32)
+    assert np.all(_sigmoid(lib, far) == 0.0) and np.all(_sigmoid(lib, -far) == 1.0)
+    z = np.sort(np.concatenate([far, -far, np.linspace(-90, 20, 4001)]).astype(np.float32))
+    s = _sigmoid(lib, z)
+    assert np.all(np.diff(s) >= -2.0 ** -23 * s[1:]) and np.all((s >= 0.0) & (s <= 1.0 + 2.0 ** -23))
