@@ -153,12 +153,13 @@ class WarmStartMLP:
         if n <= 0:
             raise ValueError("empty training batch")
         self._ensure_train_buffers(n)
-        self.step_count += 1
+        step = self.step_count + 1
         _native.ws_check(_native.ws_lib().vbd_ws_train_step(
             self._s(), n, feat.data_ptr(), target.data_ptr(), None if row_weight is None else row_weight.data_ptr(),
             self.packed.data_ptr(), self.params.data_ptr(), self._pgrad.data_ptr(), self._ploss.data_ptr(),
             self.grad.data_ptr(), self.loss.data_ptr(), self.m.data_ptr(), self.v.data_ptr(), float(lr), float(beta1),
-            float(beta2), float(eps), self.step_count), "vbd_ws_train_step")
+            float(beta2), float(eps), step), "vbd_ws_train_step")
+        self.step_count = step
         return self.loss
 
 

@@ -197,6 +197,21 @@ def test_gradient_of_large_preactivations(cuda_device, n):
         assert np.linalg.norm(a - b) <= 2e-2 * np.linalg.norm(b), name
 
 
+def test_failed_training_step_is_not_counted(cuda_device):
+    """A step that raises leaves the Adam step count, and so the next step's bias correction, as it was."""
+    import torch
+
+    from newton_amd.warmstart import WarmStartMLP
+
+    mlp = WarmStartMLP(cuda_device, seed=2)
+    x = torch.zeros((8, 48), dtype=torch.int16, device=cuda_device)
+    with pytest.raises(ValueError):
+        mlp.train_step(x, torch.empty((0, 3), device=cuda_device))
+    assert mlp.step_count == 0
+    mlp.train_step(x, torch.zeros((8, 3), device=cuda_device))
+    assert mlp.step_count == 1
+
+
 def test_adam_matches_oracle(cuda_device):
     import torch
 
