@@ -283,6 +283,7 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
     struct Batch {
         int vb, nv;
         int n[kLanes];     // items of each lane range
+        bool one_hinge_range;
         int list_begin;    // into L.list while the runs are found
         int list_count;
     };
@@ -291,6 +292,24 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
     std::vector<int32_t> stamp((size_t)N, -1), slot_of((size_t)N, 0);
     PassShape& sh = L.shape;
     auto align = [&](int n) { return aligned ? wave_align(n) : n; };
+    // First lane of each range and, at [kLanes], the lanes of all.  A vertex with more kinds than an aligned work-group
+    // has waves (a spring on a cloth with 192 lanes, a cloth with 128) gets its hinges in one range, both forms in a
+    // wave: on the generic path it would take ten times as long (256x256 cloth with springs, 192 aligned lanes,
+    // substep 483 us, 6,900 us).
+    struct Starts {
+        int at[kLanes + 1];
+    };
+    auto starts = [&](const int* n, bool one_hinge_range) {
+        Starts s{};
+        for (int i = 0; i < kLanes; ++i)
+            s.at[i + 1] = s.at[i] + align(n[i]);
+        if (one_hinge_range) {
+            const int saved = align(n[1]) + align(n[2]) - align(n[1] + n[2]);
+            s.at[2] = s.at[1] + n[1];
+            for (int i = 3; i <= kLanes; ++i) s.at[i] -= saved;
+        }
+        return s;
+    };
     for (int c = 0; c < C; ++c) {
         L.fast_color_off[c] = (int32_t)batches.size();
         L.slow_color_off[c] = (int32_t)L.slow_pos.size();
@@ -310,9 +329,10 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
             while (k < kend && b.nv < max_v) {
                 const int v = m.color_particles[k];
                 const int add[kLanes] = {ntri[v], nopp[v], nedge[v] - nopp[v], ntet[v], nspr[v]};
-                int lanes = 0;
-                for (int i = 0; i < kLanes; ++i) lanes += align(b.n[i] + add[i]);
-                if (lanes > cap) break;
+                int n[kLanes];
+                for (int i = 0; i < kLanes; ++i) n[i] = b.n[i] + add[i];
+                if (b.nv == 0 && starts(n, false).at[kLanes] > cap) b.one_hinge_range = true;
+                if (starts(n, b.one_hinge_range).at[kLanes] > cap) break;
                 const size_t before = seen.size();
                 meet(v);
                 for_items(v, [&](int, int, int, const int32_t* e, int n) {
@@ -349,12 +369,9 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
                 if (slot_of[v] < 0) lists.push_back(v);
             b.list_count = (int)lists.size() - b.list_begin;
             sh.list_stride = std::max(sh.list_stride, b.list_count);
-            int at = 0;
+            const Starts first = starts(b.n, b.one_hinge_range);
             LaneRange* ranges[kLanes] = {&sh.tri, &sh.hinge, &sh.hinge, &sh.tet, &sh.spring};
-            for (int i = 0; i < kLanes; ++i) {
-                ranges[i]->cover(at, at + b.n[i]);
-                at += align(b.n[i]);
-            }
+            for (int i = 0; i < kLanes; ++i) ranges[i]->cover(first.at[i], first.at[i] + b.n[i]);
             batches.push_back(b);
         }
     }
@@ -377,8 +394,9 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
         std::memcpy(&L.list[bi * (size_t)sh.list_stride], list, sizeof(int32_t) * (size_t)b.list_count);
         for (int i = b.list_count; i < sh.list_stride; ++i) L.list[bi * (size_t)sh.list_stride + i] = list[0];
         for (int i = 0; i < b.list_count; ++i) slot_of[list[i]] = i;
+        const Starts first = starts(b.n, b.one_hinge_range);
         int lane[kLanes];
-        for (int i = 0, at = 0; i < kLanes; at += align(b.n[i++])) lane[i] = at;
+        for (int i = 0; i < kLanes; ++i) lane[i] = first.at[i];
         int32_t* head = &L.batch_blk[bi * (size_t)L.blk_words];
         int row = 0, flags = 0;
         for (int s = 0; s < b.nv; ++s) {

@@ -111,3 +111,27 @@ def test_corners_of_one_color_are_found(check, name, shared):
     build = {"springs_only": lambda: _spring_cloth(0.0, 0.0), "no_area_term": lambda: _spring_cloth(1.0e3, 0.0)}
     args, keep = _model_args(build.get(name, MODELS.get(name))())
     assert check.shares_corners(*args, 256, 21, 0) == shared
+
+
+def _spring_tet_cloth():
+    """A cloth whose corner carries a spring and a tet cube: five kinds at one vertex, more than 256 aligned lanes."""
+    b = ModelBuilder(up_axis="Y")
+    b.add_soft_grid(pos=(0.0, 0.0, 0.0), rot=(0.0, 0.0, 0.0, 1.0), vel=(0.0, 0.0, 0.0), dim_x=2, dim_y=2, dim_z=2,
+                    cell_x=0.1, cell_y=0.1, cell_z=0.1, density=100.0, k_mu=1.0e3, k_lambda=1.0e3, k_damp=0.0,
+                    tri_ke=1.0e3, tri_ka=1.0e3, tri_kd=0.0, edge_ke=0.1, edge_kd=0.0)
+    b.add_spring(0, b.particle_count - 1, 10.0, 0.0)
+    b.color(include_bending=True)
+    return b.finalize("cpu")
+
+
+@pytest.mark.parametrize("name,block", [("cloth_17", 128), ("strip", 128), ("worlds", 128), ("cloth_17", 192),
+                                        ("springs", 192), ("springs", 256), ("cube", 128), ("five_kinds", 256)])
+def test_wave_aligned_ranges_hold_what_fits(check, name, block):
+    """Wave-aligned layouts send no vertex to the generic path whose kinds fit with both forms of its hinges in one
+    range."""
+    m = _spring_tet_cloth() if name == "five_kinds" else MODELS[name]()
+    args, keep = _model_args(m)
+    stats = (ctypes.c_longlong * 4)()
+    rc = check.check_layout(*args, block, block // 12, 1, stats)
+    assert rc == 0, f"layout_check.cpp:{rc}"
+    assert stats[1] == 0
