@@ -1066,6 +1066,11 @@ __device__ __forceinline__ int full_component(int k) {
 typedef const __attribute__((address_space(4))) int* UniformInts;
 __device__ __forceinline__ UniformInts uniform_ints(const int* p) { return (UniformInts)(uintptr_t)p; }
 
+// c ? a : b by components: the conditional of whole vectors selects an address and keeps both in scratch memory
+__device__ __forceinline__ int4 pick(bool c, int4 a, int4 b) {
+    return make_int4(c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z, c ? a.w : b.w);
+}
+
 template <bool SYM, bool FORCE_ONLY>
 __device__ __forceinline__ void put_row(float* __restrict__ row, V3 f, const M3& h) {
     row[0] = f.x;
@@ -1141,8 +1146,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
             const int4 a0 = r[0], a1 = r[1], a2 = r[2];
             // lanes of another kind keep their own record's words
             const bool mine = !(CLOTH || SPRING) || item.y >> 12 == vbd_layout::kTet;
-            w0 = mine ? a0 : w0;
-            w1 = mine ? a1 : w1;
+            w0 = pick(mine, a0, w0);
+            w1 = pick(mine, a1, w1);
             w2 = a2;
         }
     }

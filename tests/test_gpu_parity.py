@@ -220,6 +220,36 @@ def test_condition_screen_bitexact(cuda_device, mass):
     assert np.array_equal(q_gpu, q_ref) and np.array_equal(qd_gpu, qd_ref)
 
 
+@pytest.mark.parametrize("shape", [(256, 1, 0), (256, 7, 1), (192, 1, 1), (128, 1, 0)])
+def test_cloth_springs_and_tets_in_one_model_bitexact(cuda_device, shape):
+    """Every element kind in one pass: cloth with springs over a tet cube with a stiff skin on the ground, damped."""
+    from newton_amd import ModelBuilder
+    from newton_amd.solvers import SolverVBD
+
+    b = ModelBuilder(up_axis="Y", gravity=-9.81)
+    b.add_ground_plane(cfg=ModelBuilder.ShapeConfig(ke=1.0e4, kd=1.0, mu=0.5))
+    b.add_soft_grid(pos=(0.0, 0.005, 0.0), rot=(0.0, 0.0, 0.0, 1.0), vel=(0.0, -0.3, 0.0), dim_x=4, dim_y=3, dim_z=3,
+                    cell_x=0.05, cell_y=0.05, cell_z=0.05, density=300.0, k_mu=1.0e4, k_lambda=1.0e4, k_damp=1.0e-3,
+                    tri_ke=1.0e2, tri_ka=1.0e2, tri_kd=1.0e-3, edge_ke=0.05, edge_kd=1.0e-4, particle_radius=0.01)
+    tets = b.particle_count
+    b.add_cloth_grid(pos=(-0.05, 0.162, 0.25), rot=(-np.sqrt(0.5), 0.0, 0.0, np.sqrt(0.5)), vel=(0.0, -0.4, 0.0),
+                     dim_x=9, dim_y=9, cell_x=0.03, cell_y=0.03, mass=0.01, tri_ke=1.0e3, tri_ka=1.0e3, tri_kd=1.0e-3,
+                     edge_ke=0.1, edge_kd=1.0e-3, particle_radius=0.01)
+    for i in range(tets, tets + 60):
+        b.add_spring(i, i + 1, 30.0, 0.01)
+    b.color(include_bending=True)
+    model = b.finalize(cuda_device)
+    model.soft_contact_ke, model.soft_contact_kd, model.soft_contact_mu = 1.0e4, 1.0, 0.5
+    state, info = model.state(), {"dt": 1.0 / 600.0, "iterations": 4}
+    q0, qd0 = initial(state)
+    solver = SolverVBD(model, iterations=4)
+    solver.set_pass_shape(*shape)
+    q_gpu, qd_gpu, _ = gpu_run(model, state, info, 6, solver=solver)
+    q_ref, qd_ref, _ = oracle_run(model, q0, qd0, info, 6)
+    np.testing.assert_array_equal(q_gpu, q_ref)
+    np.testing.assert_array_equal(qd_gpu, qd_ref)
+
+
 def _held_by_three_springs(dev, stiff, soft):
     """A particle at the origin on springs along x and y (stiff) and z (soft, stretched) to pinned particles: a block
     of diagonal about (stiff, stiff, soft)."""

@@ -170,6 +170,37 @@ def test_layers_on_ground_with_body_contacts_bitexact(cuda_device):
     np.testing.assert_array_equal(qd_gpu, qd_ref)
 
 
+@pytest.mark.parametrize("extra", ["springs", "tets", "both"])
+def test_layers_with_springs_and_tets_bitexact(cuda_device, extra):
+    """Self-contact of two sheets beside springs on the lower one and a tet cube with a stiff skin: a pass of every
+    element kind with self-contact rows."""
+    from newton_amd import ModelBuilder
+    from newton_amd.sim.builder import cloth_grid_mesh, quat_from_axis_angle
+
+    b = ModelBuilder(up_axis="Y", gravity=-9.81)
+    b.add_ground_plane(cfg=ModelBuilder.ShapeConfig(ke=1.0e3, kd=0.0, mu=0.5))
+    verts, tris = cloth_grid_mesh(7, 7, 0.02, 0.02)
+    for k in range(2):
+        b.add_cloth_mesh(pos=(0.003 * k, 0.01 * k, 0.004 * k), rot=quat_from_axis_angle((1.0, 0.0, 0.0), math.pi / 2),
+                         scale=1.0, vel=(0.0, -2.0 * k, 0.0), vertices=verts, indices=tris, density=0.1, tri_ke=1e3,
+                         tri_ka=1e3, tri_kd=1e-4, edge_ke=0.01, edge_kd=1e-4)
+    if extra != "tets":
+        for i in range(40):
+            b.add_spring(i, i + 1, 20.0, 0.01)
+    if extra != "springs":
+        b.add_soft_grid(pos=(0.3, 0.0, 0.0), rot=(0.0, 0.0, 0.0, 1.0), vel=(0.0, 0.0, 0.0), dim_x=2, dim_y=2, dim_z=2,
+                        cell_x=0.03, cell_y=0.03, cell_z=0.03, density=200.0, k_mu=1e3, k_lambda=1e3, k_damp=1e-3,
+                        tri_ke=10.0, tri_ka=10.0, tri_kd=1e-4, edge_ke=0.01, edge_kd=0.0)
+    b.color(include_bending=True)
+    model = b.finalize(cuda_device)
+    model.soft_contact_ke, model.soft_contact_kd, model.soft_contact_mu = 2.0e3, 1.0, 0.3
+    dt = 1.0 / 600.0
+    q_gpu, qd_gpu = _run_gpu(model, SC, 8, dt)
+    q_ref, qd_ref = _run_oracle(model, SC, 8, dt)
+    np.testing.assert_array_equal(q_gpu, q_ref)
+    np.testing.assert_array_equal(qd_gpu, qd_ref)
+
+
 def test_self_contact_residual_matches_oracle(cuda_device):
     import torch
 
