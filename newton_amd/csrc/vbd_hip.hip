@@ -1039,21 +1039,7 @@ __device__ __forceinline__ float add_rows_in_order(float ca, const float* __rest
 // the header and positions gathered per element), 256x256 cloth 7.6 us (10.9).
 constexpr int kBatchHdr = vbd_layout::kBatchWords;
 
-// Element kinds a pass holds.  Every contribution of a cloth pass (triangles, hinges, springs, contacts with
-// shapes) has a Hessian that is symmetric bit for bit, so its rows hold 9 numbers instead of 12: less LDS
-// (more work-groups per CU) and fewer lanes in the sums.  Tet and self-contact Hessians are symmetric
-// only up to rounding.
-enum PassKinds { kClothKinds = 0, kClothSpringKinds = 1, kTetKinds = 2, kAllKinds = 3 };
-// Added to the kinds of a context whose contacts include edge/face records.  A pass evaluates those itself, their
-// corners read from memory and in parts when they outnumber the rows; a kernel of their rows took 8.5 us before each
-// pass (256x256 cloth on moving bodies, substep 988 -> 716 us).  That kernel, k_contact_rows, serves models whose
-// edges or faces hold corners of one color, where the pass itself moves what the entries read.  Kept apart from the other passes: compiled into
-// them it cost their occupancy (substeps of 512 cloth worlds 1,160 -> 1,354 us, of a 256x256 cloth 395 -> 437 us).
-constexpr int kEdgeFace = 4;
-// Added for self-contact, whose rows k_sc_rows evaluates (contacts crowd in a few batches: evaluated in the pass, it
-// took 39 us instead of 12 and 11 of the rows kernel).  Without springs and tets the pass needs no scratch memory:
-// 12.4 -> 11.3 us (two sheets of 128x128).
-constexpr int kSelfRows = 8;
+using namespace vbd_layout::pass_kinds;
 
 // component k of a row -> its place in {f (3), H row-major (9)}
 template <bool SYM>
@@ -2459,7 +2445,7 @@ struct VbdContext {
     int* lay_hinge_damp = nullptr;
     int* lay_tet = nullptr;
     vbd_layout::PassShape shape;  // lane ranges and strides of the uploaded layout
-    int variant = 0;              // k_solve_fast's element kinds (PassKinds)
+    int variant = 0;              // k_solve_fast's element kinds (vbd_layout::pass_kinds)
     int* lay_slow = nullptr;
     int* lay_spr = nullptr;
     int* lay_pre = nullptr;
@@ -2724,16 +2710,7 @@ int32_t build_layout(VbdContext* c) {
     k.spr_lo = L.shape.spring.lo;
     k.spr_hi = L.shape.spring.hi;
     k.list_stride = L.shape.list_stride;
-    {
-        const bool cloth = L.shape.tri.count() + L.shape.hinge.count() > 0;
-        const bool tet = L.shape.tet.count() > 0, spring = L.shape.spring.count() > 0;
-        if ((tet && (cloth || spring)) || (c->params.self_contact && (tet || spring)))
-            c->variant = kAllKinds;
-        else
-            c->variant = tet ? kTetKinds : (spring ? kClothSpringKinds : kClothKinds);
-        if (c->params.soft_contact_full_surface) c->variant += kEdgeFace;
-        if (c->params.self_contact) c->variant += kSelfRows;
-    }
+    c->variant = vbd_layout::kinds_of_pass(L.shape, c->params.soft_contact_full_surface != 0, c->params.self_contact != 0);
     k.slow_pos = c->lay_slow;
     k.has_spring = m->spring_count > 0;
     k.spring_idx = m->spring_indices;
@@ -3006,28 +2983,18 @@ std::string noalloc_scratch(int32_t** out) {
     return std::string();
 }
 
-template <int BLOCK, int WAVES, bool FORCE_ONLY>
-void launch_kinds(VbdContext* c, hipStream_t s, int b0, int nb, float* q, float dt, int mode, float* g) {
-    const dim3 grid(nb), block(BLOCK);
-    switch (c->variant) {
-#define PASS_OF_KINDS(K)                                                                                          \
-    case K:                                                                                                        \
-        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, K, FORCE_ONLY>), grid, block, 0, s, q, b0, nb, dt, mode, g, \
-                           c->kp);                                                                                 \
-        break;
-        PASS_OF_KINDS(kClothKinds)
-        PASS_OF_KINDS(kClothSpringKinds)
-        PASS_OF_KINDS(kTetKinds)
-        PASS_OF_KINDS(kAllKinds)
-        PASS_OF_KINDS(kClothKinds + kEdgeFace)
-        PASS_OF_KINDS(kClothSpringKinds + kEdgeFace)
-        PASS_OF_KINDS(kTetKinds + kEdgeFace)
-        PASS_OF_KINDS(kAllKinds + kEdgeFace)
-        PASS_OF_KINDS(kClothKinds + kSelfRows)
-        PASS_OF_KINDS(kAllKinds + kSelfRows)
-        PASS_OF_KINDS(kClothKinds + kSelfRows + kEdgeFace)
-        PASS_OF_KINDS(kAllKinds + kSelfRows + kEdgeFace)
-#undef PASS_OF_KINDS
+// The pass compiled for the context's kinds, one of kInstantiated.
+template <int BLOCK, int WAVES, bool FORCE_ONLY, size_t I = 0>
+int32_t launch_kinds(VbdContext* c, hipStream_t s, int b0, int nb, float* q, float dt, int mode, float* g) {
+    if constexpr (I == sizeof(kInstantiated) / sizeof(kInstantiated[0])) {
+        return fail(VBD_ERR_STATE, "k_solve_fast: no instantiation for element kinds " + std::to_string(c->variant));
+    } else {
+        if (c->variant != kInstantiated[I])
+            return launch_kinds<BLOCK, WAVES, FORCE_ONLY, I + 1>(c, s, b0, nb, q, dt, mode, g);
+        hipLaunchKernelGGL((k_solve_fast<BLOCK, WAVES, kInstantiated[I], FORCE_ONLY>), dim3(nb), dim3(BLOCK), 0, s, q,
+                           b0, nb, dt, mode, g, c->kp);
+        VBD_LAUNCH_CHECK("k_solve_fast");
+        return VBD_OK;
     }
 }
 
@@ -3437,25 +3404,15 @@ void set_dt(VbdContext* c, float dt) {
 int32_t launch_fast(VbdContext* c, hipStream_t s, int b0, int nb, float* q, float dt, int mode, float* g,
                     bool force_only = false) {
     if (mode == 1 && force_only) {
-        if (c->block == 128)
-            launch_kinds<128, 1, true>(c, s, b0, nb, q, dt, mode, g);
-        else if (c->block == 192)
-            launch_kinds<192, 1, true>(c, s, b0, nb, q, dt, mode, g);
-        else
-            launch_kinds<256, 1, true>(c, s, b0, nb, q, dt, mode, g);
-    } else if (c->block == 128) {
-        launch_kinds<128, 1, false>(c, s, b0, nb, q, dt, mode, g);
-    } else if (c->block == 192 && c->waves == 7) {
-        launch_kinds<192, 7, false>(c, s, b0, nb, q, dt, mode, g);
-    } else if (c->block == 192) {
-        launch_kinds<192, 1, false>(c, s, b0, nb, q, dt, mode, g);
-    } else if (c->waves == 7) {
-        launch_kinds<256, 7, false>(c, s, b0, nb, q, dt, mode, g);
-    } else {
-        launch_kinds<256, 1, false>(c, s, b0, nb, q, dt, mode, g);
+        if (c->block == 128) return launch_kinds<128, 1, true>(c, s, b0, nb, q, dt, mode, g);
+        if (c->block == 192) return launch_kinds<192, 1, true>(c, s, b0, nb, q, dt, mode, g);
+        return launch_kinds<256, 1, true>(c, s, b0, nb, q, dt, mode, g);
     }
-    VBD_LAUNCH_CHECK("k_solve_fast");
-    return VBD_OK;
+    if (c->block == 128) return launch_kinds<128, 1, false>(c, s, b0, nb, q, dt, mode, g);
+    if (c->block == 192 && c->waves == 7) return launch_kinds<192, 7, false>(c, s, b0, nb, q, dt, mode, g);
+    if (c->block == 192) return launch_kinds<192, 1, false>(c, s, b0, nb, q, dt, mode, g);
+    if (c->waves == 7) return launch_kinds<256, 7, false>(c, s, b0, nb, q, dt, mode, g);
+    return launch_kinds<256, 1, false>(c, s, b0, nb, q, dt, mode, g);
 }
 
 int32_t launch_spring_rows(VbdContext* c, hipStream_t s, int j0, int j1, const float* q, float dt) {

@@ -130,6 +130,39 @@ struct PassShape {
     }
 };
 
+namespace pass_kinds {
+// Element kinds a pass holds.  Every contribution of a cloth pass (triangles, hinges, springs, contacts with
+// shapes) has a Hessian that is symmetric bit for bit, so its rows hold 9 numbers instead of 12: less LDS
+// (more work-groups per CU) and fewer lanes in the sums.  Tet and self-contact Hessians are symmetric
+// only up to rounding.
+constexpr int kClothKinds = 0, kClothSpringKinds = 1, kTetKinds = 2, kAllKinds = 3;
+// Added to the kinds of a context whose contacts include edge/face records.  A pass evaluates those itself, their
+// corners read from memory and in parts when they outnumber the rows; a kernel of their rows took 8.5 us before each
+// pass (256x256 cloth on moving bodies, substep 988 -> 716 us).  That kernel, k_contact_rows, serves models whose
+// edges or faces hold corners of one color, where the pass itself moves what the entries read.  Kept apart from the
+// other passes: compiled into them it cost their occupancy (substeps of 512 cloth worlds 1,160 -> 1,354 us, of a
+// 256x256 cloth 395 -> 437 us).
+constexpr int kEdgeFace = 4;
+// Added for self-contact, whose rows k_sc_rows evaluates (contacts crowd in a few batches: evaluated in the pass, it
+// took 39 us instead of 12 and 11 of the rows kernel).
+constexpr int kSelfRows = 8;
+// What the pass is compiled for.
+constexpr int kInstantiated[] = {
+    kClothKinds, kClothSpringKinds, kTetKinds, kAllKinds, kClothKinds + kEdgeFace, kClothSpringKinds + kEdgeFace,
+    kTetKinds + kEdgeFace, kAllKinds + kEdgeFace, kClothKinds + kSelfRows, kAllKinds + kSelfRows,
+    kClothKinds + kSelfRows + kEdgeFace, kAllKinds + kSelfRows + kEdgeFace};
+}  // namespace pass_kinds
+
+// The kinds a layout's passes run with.
+inline int kinds_of_pass(const PassShape& sh, bool full_surface, bool self_contact) {
+    using namespace pass_kinds;
+    const bool cloth = sh.tri.count() + sh.hinge.count() > 0;
+    const bool tet = sh.tet.count() > 0, spring = sh.spring.count() > 0;
+    int kinds = tet ? kTetKinds : (spring ? kClothSpringKinds : kClothKinds);
+    if ((tet && (cloth || spring)) || (self_contact && (tet || spring))) kinds = kAllKinds;
+    return kinds + (full_surface ? kEdgeFace : 0) + (self_contact ? kSelfRows : 0);
+}
+
 struct PassLayout {
     std::vector<int32_t> fast_color_off;  // [C+1] into batch records
     std::vector<int32_t> slow_color_off;  // [C+1] into slow_pos

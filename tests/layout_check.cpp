@@ -226,3 +226,24 @@ extern "C" int shares_corners(MODEL_ARGS, int cap, int max_v, int aligned) {
     if (!build_pass_layout(m, L, cap, max_v, aligned != 0).empty()) return -1;
     return L.shape.shared_corners ? 1 : 0;
 }
+
+// Every combination of element ranges and contact kinds has a compiled pass that holds its kinds.
+extern "C" int check_kinds() {
+    using namespace pass_kinds;
+    for (int mask = 0; mask < 64; ++mask) {
+        PassShape sh;
+        if (mask & 1) sh.tri.cover(0, 10);
+        if (mask & 2) sh.hinge.cover(10, 20);
+        if (mask & 4) sh.tet.cover(20, 30);
+        if (mask & 8) sh.spring.cover(30, 40);
+        const int kinds = kinds_of_pass(sh, mask & 16, mask & 32), elems = kinds & 3;
+        bool found = false;
+        for (int k : kInstantiated) found = found || k == kinds;
+        CHECK(found);
+        CHECK(!(mask & 3) || elems != kTetKinds);
+        CHECK(!(mask & 4) || elems == kTetKinds || elems == kAllKinds);
+        CHECK(!(mask & 8) || elems == kClothSpringKinds || elems == kAllKinds);
+        CHECK(((kinds & kEdgeFace) != 0) == ((mask & 16) != 0) && ((kinds & kSelfRows) != 0) == ((mask & 32) != 0));
+    }
+    return 0;
+}

@@ -135,3 +135,8 @@ def test_wave_aligned_ranges_hold_what_fits(check, name, block):
     rc = check.check_layout(*args, block, block // 12, 1, stats)
     assert rc == 0, f"layout_check.cpp:{rc}"
     assert stats[1] == 0
+
+
+def test_every_combination_of_kinds_has_a_pass(check):
+    rc = check.check_kinds()
+    assert rc == 0, f"layout_check.cpp:{rc}"
