@@ -708,7 +708,8 @@ struct KParams {
     const int* batch_blk;
     const int* item_rec;    // [B * lanes] 16-byte items
     const int* list;        // [B * list_stride] vertex lists
-    const int* tri_rec;     // [B * (tri_hi - tri_lo)] and so on: the wider parts of the records
+    const int* tri_rec;     // [B * (tri_hi - tri_lo)] and so on: the wider parts of the records (passes with tets: all
+                            // in tet_rec)
     const int* tet_rec;
     const int* spr_rec;
     const float* hinge_damp;
@@ -1052,11 +1053,6 @@ __device__ __forceinline__ int full_component(int k) {
 typedef const __attribute__((address_space(4))) int* UniformInts;
 __device__ __forceinline__ UniformInts uniform_ints(const int* p) { return (UniformInts)(uintptr_t)p; }
 
-// c ? a : b by components: the conditional of whole vectors selects an address and keeps both in scratch memory
-__device__ __forceinline__ int4 pick(bool c, int4 a, int4 b) {
-    return make_int4(c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z, c ? a.w : b.w);
-}
-
 template <bool SYM, bool FORCE_ONLY>
 __device__ __forceinline__ void put_row(float* __restrict__ row, V3 f, const M3& h) {
     row[0] = f.x;
@@ -1118,7 +1114,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
     const int id = P.list[(size_t)b * P.list_stride + min(t, P.list_stride - 1)];
     int4 w0 = make_int4(0, 0, 0, 0), w1 = w0, w2 = w0;
     float kdl = 0.0f;
-    if constexpr (CLOTH) {
+    if constexpr (CLOTH && !TET) {
         if (64 * wave < P.tri_hi) {
             const int4* r = reinterpret_cast<const int4*>(P.tri_rec) + 2 * ((size_t)b * P.tri_hi + min(t, P.tri_hi - 1));
             w0 = r[0];
@@ -1129,15 +1125,12 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
         if (64 * wave < P.tet_hi && 64 * wave + 63 >= P.tet_lo) {
             const int lane = min(max(t, P.tet_lo), P.tet_hi - 1) - P.tet_lo;
             const int4* r = reinterpret_cast<const int4*>(P.tet_rec) + 3 * ((size_t)b * (P.tet_hi - P.tet_lo) + lane);
-            const int4 a0 = r[0], a1 = r[1], a2 = r[2];
-            // lanes of another kind keep their own record's words
-            const bool mine = !(CLOTH || SPRING) || item.y >> 12 == vbd_layout::kTet;
-            w0 = pick(mine, a0, w0);
-            w1 = pick(mine, a1, w1);
-            w2 = a2;
+            w0 = r[0];
+            w1 = r[1];
+            w2 = r[2];
         }
     }
-    if constexpr (SPRING) {
+    if constexpr (SPRING && !TET) {
         if (P.spr_hi > P.spr_lo) {
             const int lane = min(max(t, P.spr_lo), P.spr_hi - 1) - P.spr_lo;
             const int2 r = reinterpret_cast<const int2*>(P.spr_rec)[(size_t)b * (P.spr_hi - P.spr_lo) + lane];
@@ -2588,6 +2581,7 @@ int32_t build_layout(VbdContext* c) {
     if (err.empty() && hm.E > 0) rd(hm.adj_edge, m->v_adj_edges, (size_t)hm.adj_edge_off[hm.N]);
     if (err.empty() && hm.K > 0) rd(hm.adj_tet, m->v_adj_tets, (size_t)hm.adj_tet_off[hm.N]);
     hm.S = m->spring_count;
+    hm.self_contact = c->params.self_contact != 0;
     rd(hm.spring_idx, m->spring_indices, 2 * (size_t)hm.S);
     rd(hm.spring_rest, m->spring_rest_length, (size_t)hm.S);
     rd(hm.spring_ke, m->spring_stiffness, (size_t)hm.S);

@@ -15,8 +15,9 @@
 // batch's vertex list, from the batch number alone, in the same round trip as
 // the batch header: item t of batch b is item_rec[b * cap + t]; the wider part
 // of a triangle (tet, spring) record sits in an array with one slot for each
-// lane that holds that kind in any batch ([tri_lo, tri_hi) and so on).  Slots
-// that a batch does not use are never read.  Items name their vertices by 8-bit
+// lane that holds that kind in any batch ([tri_lo, tri_hi) and so on), or, for
+// passes of every kind, in the slots of the widest kind.  Slots
+// that a batch does not use are never used.  Items name their vertices by 8-bit
 // slots of the batch's vertex list (the batch's own vertices first), whose
 // positions the work-group stages in LDS: a hinge item is 16 bytes, and a
 // position is gathered once per batch instead of once per element.
@@ -97,6 +98,7 @@ struct HostModel {
     int S = 0;
     std::vector<int32_t> spring_idx;
     std::vector<float> spring_rest, spring_ke, spring_kd;
+    bool self_contact = false;  // of the solver: decides the kinds of a pass (kinds_of_pass)
 };
 
 // Lanes [lo, hi) that hold one kind of item in any batch (empty when lo == hi).
@@ -118,7 +120,7 @@ struct LaneRange {
 
 // What a launch is given besides the arrays; equal shapes may be exchanged under a captured graph.
 struct PassShape {
-    LaneRange tri, hinge, tet, spring;
+    LaneRange tri, hinge, tet, spring;  // tet: of every kind with a record where they share an array
     int list_stride = 0;  // entries of a batch's vertex list
     // Two corners of some edge or triangle share a color (elements without stiffness are not part of the coloring
     // graph): a pass moves one corner of their edge/face contacts while another's entry reads it, so those entries'
@@ -414,12 +416,19 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
     // ---- the records
     const size_t B = batches.size();
     sh.list_stride = (sh.list_stride + 3) & ~3;
+    // A pass of every kind reads one record a lane, of any kind, from the array of the widest: an array a kind, it read
+    // the slots of each in every batch (cloth of 128x128 and eight tet cubes, substep 285 us, 271 us so).
+    const bool shared_rec = (kinds_of_pass(sh, false, m.self_contact) & 3) == pass_kinds::kAllKinds;
+    if (shared_rec) {
+        sh.tet.cover(sh.tri.lo, sh.tri.hi);
+        sh.tet.cover(sh.spring.lo, sh.spring.hi);
+    }
     L.batch_blk.assign(B * (size_t)L.blk_words, 0);
     L.item_rec.assign(B * (size_t)cap * kItemWords, 0);
     L.list.assign(B * (size_t)sh.list_stride, 0);
-    L.tri_rec.assign(B * (size_t)sh.tri.count() * kTriWords, 0);
+    L.tri_rec.assign(shared_rec ? 0 : B * (size_t)sh.tri.count() * kTriWords, 0);
     L.tet_rec.assign(B * (size_t)sh.tet.count() * kTetWords, 0);
-    L.spr_rec.assign(B * (size_t)sh.spring.count() * kSpringWords, 0);
+    L.spr_rec.assign(shared_rec ? 0 : B * (size_t)sh.spring.count() * kSpringWords, 0);
     L.hinge_damp.assign(B * (size_t)sh.hinge.count(), 0);
     for (size_t bi = 0; bi < B; ++bi) {
         const Batch& b = batches[bi];
@@ -449,9 +458,13 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
                 for (int i = 0; i < n; ++i) slots |= (uint32_t)slot_of[who[i]] << (8 * i);
                 r[0] = (int32_t)slots;
                 bool damped = false;
+                auto record = [&](std::vector<int32_t>& own, const LaneRange& range, int words) {
+                    return shared_rec ? &L.tet_rec[(bi * (size_t)sh.tet.count() + (t - sh.tet.lo)) * kTetWords]
+                                      : &own[(bi * (size_t)range.count() + (t - range.lo)) * words];
+                };
                 if (kind == kTri) {
                     const float* mat = &m.tri_mat[5 * (size_t)e];
-                    int32_t* w = &L.tri_rec[(bi * (size_t)sh.tri.count() + (t - sh.tri.lo)) * kTriWords];
+                    int32_t* w = record(L.tri_rec, sh.tri, kTriWords);
                     for (int q = 0; q < 4; ++q) w[q] = fbits(m.tri_pose[4 * (size_t)e + q]);
                     w[4] = fbits(mat[0]);
                     w[5] = fbits(lame_sum(mat[0], mat[1]));
@@ -469,7 +482,7 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
                 } else if (kind == kTet) {
                     const float* mat = &m.tet_mat[3 * (size_t)e];
                     const float* dm = &m.tet_pose[9 * (size_t)e];
-                    int32_t* w = &L.tet_rec[(bi * (size_t)sh.tet.count() + (t - sh.tet.lo)) * kTetWords];
+                    int32_t* w = record(L.tet_rec, sh.tet, kTetWords);
                     for (int q = 0; q < 9; ++q) w[q] = fbits(dm[q]);
                     w[9] = fbits(rest_volume(dm));
                     w[10] = fbits(rest_ratio(mat[0], mat[1]));
@@ -479,7 +492,7 @@ inline std::string build_pass_layout(const HostModel& m, PassLayout& L, int cap 
                     damped = mat[2] > 0.0f;
                 } else {  // e indexes vs_item
                     const int sp = vs_item[e] >> 1;
-                    int32_t* w = &L.spr_rec[(bi * (size_t)sh.spring.count() + (t - sh.spring.lo)) * kSpringWords];
+                    int32_t* w = record(L.spr_rec, sh.spring, kSpringWords);
                     w[0] = fbits(m.spring_ke[sp]);
                     w[1] = fbits(m.spring_kd[sp]);
                     r[2] = pre_row[e];

@@ -43,8 +43,9 @@ static HostModel host_model(MODEL_ARGS) {
     m.spring_idx.assign(spring, spring + 2 * S);
     m.spring_rest.resize(S);
     for (int s = 0; s < S; ++s) m.spring_rest[s] = (float)s;
-    m.spring_ke.assign(S, 1.0f);
-    m.spring_kd.assign(S, 1.0f);
+    m.spring_ke.resize(S);
+    m.spring_kd.resize(S);
+    for (int s = 0; s < S; ++s) m.spring_ke[s] = 2.0f + s, m.spring_kd[s] = 0.5f + s;
     m.color_off.assign(color_off, color_off + C + 1);
     m.color_particles.assign(color_particles, color_particles + N);
     return m;
@@ -62,6 +63,10 @@ extern "C" int check_layout(MODEL_ARGS, int cap, int max_v, int aligned, long lo
     CHECK(L.batch_blk.size() == (size_t)B * L.blk_words && L.item_rec.size() == (size_t)B * cap * kItemWords);
     CHECK(L.list.size() == (size_t)B * sh.list_stride && sh.list_stride <= list_cap(cap) && sh.tri.lo == 0);
     CHECK(sh.tri.hi <= cap && sh.hinge.hi <= cap && sh.tet.hi <= cap && sh.spring.hi <= cap);
+    // records of every kind share one array when a pass holds every kind
+    const bool shared = (kinds_of_pass(sh, false, false) & 3) == pass_kinds::kAllKinds;
+    CHECK(!shared || (L.tri_rec.empty() && L.spr_rec.empty()));
+    if (shared) CHECK(sh.tet.hi >= sh.tri.hi && sh.tet.hi >= sh.spring.hi && (sh.tri.count() == 0 || sh.tet.lo == 0));
     std::vector<int> color_of(N);
     for (int c = 0; c < C; ++c)
         for (int k = color_off[c]; k < color_off[c + 1]; ++k) color_of[color_particles[k]] = c;
@@ -109,6 +114,9 @@ extern "C" int check_layout(MODEL_ARGS, int cap, int max_v, int aligned, long lo
                     CHECK(t < sh.tri.hi);
                     std::memcpy(&f, &r[2], 4);
                     elem = (int)f, n = 3, who = &m.tri_idx[3 * (size_t)elem];
+                    const int32_t* w = shared ? &L.tet_rec[((size_t)b * sh.tet.count() + t - sh.tet.lo) * kTetWords]
+                                              : &L.tri_rec[((size_t)b * sh.tri.count() + t) * kTriWords];
+                    CHECK(w[4] == fbits(m.tri_mat[5 * (size_t)elem]) && w[7] == fbits(m.tri_mat[5 * (size_t)elem + 2]));
                 } else if (kind == kHinge) {
                     CHECK(t >= sh.hinge.lo && t < sh.hinge.hi);
                     std::memcpy(&f, &r[2], 4);
@@ -121,6 +129,9 @@ extern "C" int check_layout(MODEL_ARGS, int cap, int max_v, int aligned, long lo
                     CHECK(kind == kSpring && t >= sh.spring.lo && t < sh.spring.hi);
                     std::memcpy(&f, &r[3], 4);
                     elem = (int)f, n = 2, who = &m.spring_idx[2 * (size_t)elem];
+                    const int32_t* w = shared ? &L.tet_rec[((size_t)b * sh.tet.count() + t - sh.tet.lo) * kTetWords]
+                                              : &L.spr_rec[((size_t)b * sh.spring.count() + t - sh.spring.lo) * kSpringWords];
+                    CHECK(w[0] == fbits(m.spring_ke[elem]) && w[1] == fbits(m.spring_kd[elem]));
                 }
                 if (aligned) {  // a wave evaluates one kind, and one form of a hinge, only
                     const int32_t* first = &L.item_rec[((size_t)b * cap + (t & ~63)) * kItemWords];

@@ -37,6 +37,17 @@ def _fan(segments):
     return b.finalize("cpu")
 
 
+def _spring_tet_cloth():
+    """A cloth whose corner carries a spring and a tet cube: five kinds at one vertex, more than 256 aligned lanes."""
+    b = ModelBuilder(up_axis="Y")
+    b.add_soft_grid(pos=(0.0, 0.0, 0.0), rot=(0.0, 0.0, 0.0, 1.0), vel=(0.0, 0.0, 0.0), dim_x=2, dim_y=2, dim_z=2,
+                    cell_x=0.1, cell_y=0.1, cell_z=0.1, density=100.0, k_mu=1.0e3, k_lambda=1.0e3, k_damp=0.0,
+                    tri_ke=1.0e3, tri_ka=1.0e3, tri_kd=0.0, edge_ke=0.1, edge_kd=0.0)
+    b.add_spring(0, b.particle_count - 1, 10.0, 0.0)
+    b.color(include_bending=True)
+    return b.finalize("cpu")
+
+
 MODELS = {
     "strip": lambda: scenes.cloth_strip_pinned("cpu")[0],
     "cloth_17": lambda: scenes.cloth_hanging("cpu", verts_per_side=17)[0],
@@ -47,6 +58,7 @@ MODELS = {
     "fan_40": lambda: _fan(40),    # 120 items, 81 vertices: every packed shape holds it
     "fan_80": lambda: _fan(80),    # 240 items, 161 vertices: only the widest shape holds it
     "fan_120": lambda: _fan(120),  # generic path
+    "five_kinds": _spring_tet_cloth,
 }
 
 
@@ -82,7 +94,7 @@ def test_layout(check, name, block, aligned):
         assert stats[1] >= 1
 
 
-@pytest.mark.parametrize("name", ["cloth_17", "springs", "cube", "fan_80"])
+@pytest.mark.parametrize("name", ["cloth_17", "springs", "cube", "fan_80", "five_kinds"])
 @pytest.mark.parametrize("block,aligned", [(256, 0), (192, 1)])
 def test_damping_edit_keeps_the_layout(check, name, block, aligned):
     """Damping switched from or to zero changes no array size, batch range or launch argument, so a rebuild writes in
@@ -113,23 +125,12 @@ def test_corners_of_one_color_are_found(check, name, shared):
     assert check.shares_corners(*args, 256, 21, 0) == shared
 
 
-def _spring_tet_cloth():
-    """A cloth whose corner carries a spring and a tet cube: five kinds at one vertex, more than 256 aligned lanes."""
-    b = ModelBuilder(up_axis="Y")
-    b.add_soft_grid(pos=(0.0, 0.0, 0.0), rot=(0.0, 0.0, 0.0, 1.0), vel=(0.0, 0.0, 0.0), dim_x=2, dim_y=2, dim_z=2,
-                    cell_x=0.1, cell_y=0.1, cell_z=0.1, density=100.0, k_mu=1.0e3, k_lambda=1.0e3, k_damp=0.0,
-                    tri_ke=1.0e3, tri_ka=1.0e3, tri_kd=0.0, edge_ke=0.1, edge_kd=0.0)
-    b.add_spring(0, b.particle_count - 1, 10.0, 0.0)
-    b.color(include_bending=True)
-    return b.finalize("cpu")
-
-
 @pytest.mark.parametrize("name,block", [("cloth_17", 128), ("strip", 128), ("worlds", 128), ("cloth_17", 192),
                                         ("springs", 192), ("springs", 256), ("cube", 128), ("five_kinds", 256)])
 def test_wave_aligned_ranges_hold_what_fits(check, name, block):
     """Wave-aligned layouts send no vertex to the generic path whose kinds fit with both forms of its hinges in one
     range."""
-    m = _spring_tet_cloth() if name == "five_kinds" else MODELS[name]()
+    m = MODELS[name]()
     args, keep = _model_args(m)
     stats = (ctypes.c_longlong * 4)()
     rc = check.check_layout(*args, block, block // 12, 1, stats)
