@@ -290,7 +290,8 @@ __global__ __launch_bounds__(kFeatBlock) void k_features(int n, const int* __res
 // of a predicted correction fast and its smooth ones slowly.
 constexpr int kSmoothMaxWidth = 12;
 
-// W > 0: the width at compile time (3 and 6: one and two fields); 0: width at run time.
+// W > 0: the width at compile time (3 and 6: one and two fields; 1: a scalar, for which the run-time width's selects
+// cost more than its loads, eight sweeps of 144 particles 23.1 -> 15.2 us); 0: width at run time.
 // Bound: memory.  Six index loads and then six gathers are in flight at a time (one dependent pair after another
 // before), and an XCD's particles share its L2: 1,048,576 particles of width 3 13.5 us a sweep, 4.7 TB/s (26.4 us).
 template <int W>
@@ -1225,7 +1226,9 @@ int32_t vbd_ws_smooth(void* stream, int32_t n, int32_t width, const int32_t* nbr
     float* dst = tmp;
     for (int k = 0; k < sweeps; ++k) {
         const dim3 grid(blocks_for(n, 256)), block(256);
-        if (width == 3)
+        if (width == 1)
+            hipLaunchKernelGGL(k_smooth<1>, grid, block, 0, s, n, width, nbr_off, nbr, active, src, dst);
+        else if (width == 3)
             hipLaunchKernelGGL(k_smooth<3>, grid, block, 0, s, n, width, nbr_off, nbr, active, src, dst);
         else if (width == 6)
             hipLaunchKernelGGL(k_smooth<6>, grid, block, 0, s, n, width, nbr_off, nbr, active, src, dst);

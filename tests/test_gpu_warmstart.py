@@ -406,7 +406,7 @@ def test_smooth_matches_oracle(cuda_device):
 
 
 @pytest.mark.parametrize("n", [1, 63, 65, 255, 257, 2049, 5003])
-@pytest.mark.parametrize("width", [3, 6, 5])
+@pytest.mark.parametrize("width", [3, 6, 5, 1])
 def test_smooth_and_features_on_irregular_rings(cuda_device, n, width):
     """Rings of 0 to 20 neighbours (more than are loaded together), some particles inactive, sizes around the
     work-group's and the wave's: the low-pass bit for bit, and feature rows that do not depend on their place."""
