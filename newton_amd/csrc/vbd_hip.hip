@@ -1113,6 +1113,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
     const int4 item = reinterpret_cast<const int4*>(P.item_rec)[(size_t)b * BLOCK + t];
     const int id = P.list[(size_t)b * P.list_stride + min(t, P.list_stride - 1)];
     int4 w0 = make_int4(0, 0, 0, 0), w1 = w0, w2 = w0;
+    int2 spr = make_int2(0, 0);  // apart from w0: choosing between them here would wait for both
     float kdl = 0.0f;
     if constexpr (CLOTH && !TET) {
         if (64 * wave < P.tri_hi) {
@@ -1133,10 +1134,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
     if constexpr (SPRING && !TET) {
         if (P.spr_hi > P.spr_lo) {
             const int lane = min(max(t, P.spr_lo), P.spr_hi - 1) - P.spr_lo;
-            const int2 r = reinterpret_cast<const int2*>(P.spr_rec)[(size_t)b * (P.spr_hi - P.spr_lo) + lane];
-            const bool mine = item.y >> 12 == vbd_layout::kSpring;
-            w0.x = mine ? r.x : w0.x;
-            w0.y = mine ? r.y : w0.y;
+            spr = reinterpret_cast<const int2*>(P.spr_rec)[(size_t)b * (P.spr_hi - P.spr_lo) + lane];
         }
     }
     const int4 vr = reinterpret_cast<const int4*>(blk + kBatchHdr)[min(t, MAXV - 1)];
@@ -1257,8 +1255,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WAVES))) 
                 if (item.z >= 0)
                     load_row(P.spr_rows + kComp * (size_t)item.z, fe, he);
                 else
-                    eval_spring(at(0), at(1), prev(0), prev(1), __int_as_float(item.w), __int_as_float(w0.x),
-                                __int_as_float(w0.y), dt, slot, fe, he);
+                    eval_spring(at(0), at(1), prev(0), prev(1), __int_as_float(item.w),
+                                __int_as_float(TET ? w0.x : spr.x), __int_as_float(TET ? w0.y : spr.y), dt, slot, fe,
+                                he);
             }
         }
         put_row<SYM, FORCE_ONLY>(s_rows + row * NC, fe, he);
