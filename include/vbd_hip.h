@@ -199,7 +199,8 @@ int32_t vbd_destroy(VbdContext* ctx);
  * (element materials, rest data, flags, masses).  SolverVBD.notify_model_changed
  * (newton/_src/solvers/solver.py:375-410, solver_vbd.py:851-856).  When the new layout has the
  * shape of the old one (same array sizes, per-color batch ranges and batch width: the case of
- * material and rest-data edits that leave every element's stiffness non-zero) it is written into
+ * material and rest-data edits that leave every element's stiffness non-zero; damping may be switched
+ * from or to zero) it is written into
  * the existing device buffers, so graphs captured before stay valid and see the new values.
  * Otherwise (elements switched to or from zero stiffness, particles activated or deactivated,
  * new color groups) the layout is re-allocated and graphs captured before this call must be

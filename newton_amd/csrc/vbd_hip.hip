@@ -354,7 +354,7 @@ __device__ __forceinline__ M3 nvd_skew(float inv_len, V3 nh, V3 v) {
 // matrices (:730-741) and its 0/1 mask selection contribute signed zeros only, and a sign factored out of a
 // product or a sum changes no other bit.  The pass layout puts slots 0, 1 and slots 2, 3 into lanes of their own,
 // so in a wave-aligned layout a wave runs one of the two forms (548 -> 380 and 470 vector instructions a hinge,
-// with the shared square roots and reciprocals above: pass of 512 cloth worlds 60.7 -> 52.0 us).
+// with the shared square roots and reciprocals above: pass of 512 cloth worlds, no contacts, 60.7 -> 52.0 us).
 // k = ke * rest_length and kdl = kd * rest_length come from the caller.
 template <typename Prev>
 __device__ __forceinline__ void eval_bending(V3 x0, V3 x1, V3 x2, V3 x3, Prev prev, float rest_angle, float k,
@@ -1036,8 +1036,9 @@ __device__ __forceinline__ float add_rows_in_order(float ca, const float* __rest
 //   c  the vertex's lane solves the 3x3 block and writes displacement and position
 // Bound: vector instructions and the waits of one work-group's chain.  The items are read coalesced from fixed
 // slots and the positions once per batch, no load waits for another's branch, and six to seven waves a SIMD cover
-// what waits are left: 936 k cloth vertices in 512 worlds, 52.0 us a pass (65.2 us with element records found through
-// the header and positions gathered per element), 256x256 cloth 7.6 us (10.9).
+// what waits are left: 936 k cloth vertices in 512 worlds, no contacts, 53 us a pass (68 us with element records found
+// through the header and positions gathered per element), 256x256 cloth 7.7 us (11.2); with the ground contacts of
+// landing worlds 59 us, with those of the draped cloth 8.7 us.
 constexpr int kBatchHdr = vbd_layout::kBatchWords;
 
 using namespace vbd_layout::pass_kinds;
@@ -3150,7 +3151,7 @@ int32_t vbd_create(const VbdModelDesc* m, const VbdSolverParams* prm, VbdContext
     k.write_q = 1;
     // Cloth starts with 192-lane work-groups and wave-aligned items: a regular mesh fills one wave with triangles,
     // one with the hinges opposite its vertices and one with those on them, ten vertices a batch (pass of a
-    // 256x256 cloth 7.6 us, 8.6 us with 256 packed lanes; of a 32x32 one 4.3 and 5.0 us).  A mesh with vertices too
+    // 256x256 cloth, no contacts, 7.7 us, 8.6 us with 256 packed lanes; of a 32x32 one 4.3 and 5.0 us).  A mesh with vertices too
     // large for that shape, tets (16.3 us either way for 128 cubes) and springs (a fourth range) start with 256
     // packed lanes.
     int32_t rc = VBD_OK;

@@ -477,7 +477,8 @@ __global__ __launch_bounds__(kBlock) void k_forward(int n, const uint16_t* __res
 // activations are rounded to BF16 right after); the biases are the accumulators' first values.
 // Bound: the 384 SiLUs a row, two quarter-rate instructions each (about 85 us per million rows, 120 with the
 // multiplies); without the barriers of an LDS exchange the other waves' products fill in beside them:
-// 1,048,576 rows 118.5 us, 690 TFLOP/s (215 us with activations exchanged through LDS), 16,384 rows 9.2 us (17.7).
+// 1,048,576 rows 127 us, 650 TFLOP/s (223 us with activations exchanged through LDS; 137 to 140 us on other cards and
+// under a kernel trace), 16,384 rows 9.2 us (17.7).
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kFrag1 = 0;                      // layer 1: k to 64 (zero past 48), then eight tiles of 16 columns
@@ -1261,7 +1262,8 @@ int32_t vbd_ws_forward(void* stream, int32_t n, const uint16_t* feat, const uint
     // One work-group per CU (its weights fill half the LDS), with as few waves as give every group of 16 rows its
     // own: a short call pays for loading the weights and one chain of layers (16,384 rows: 4 waves 9.2 us, 8 waves
     // 9.7, 16 waves 12.3).  32 rows a wave read the weights half as often but leave more of the last round idle: they
-    // win from about four rounds on (400,000 rows 56.3 us against 61.9, 1,048,576 rows 122.8 against 118.5).
+    // win from about four rounds on (16 and 32 rows a wave timed in turn: 400,000 rows 56.3 and 61.9 us, 1,048,576 rows
+    // 122.8 and 118.5 us).
     hipStream_t s = (hipStream_t)stream;
     const int g16 = blocks_for(n, 16), g32 = blocks_for(n, 32);
     if (g16 <= 4 * cus)

@@ -209,8 +209,9 @@ def test_fp64_ill_conditioned_mode_bitexact(cuda_device):
 
 @pytest.mark.parametrize("mass", [1.0e-2, 1.0e-3, 1.0e-4, 1.0e-5, 1.0e-6])
 def test_condition_screen_bitexact(cuda_device, mass):
-    """Block conditions from about 1 to 1e4, on both sides of the single-precision screen (2e5 at most) that lets
-    well-conditioned blocks skip the double-precision estimate: the oracle always evaluates that estimate."""
+    """Block conditions from about 1 to 1e4, most of which the single-precision screen clears: with the estimate skipped
+    or evaluated the solve is the single-precision one of the oracle, which always evaluates it.  That the screen never
+    clears a block beyond 1e6 is test_scalar_formulas.py's; conditions around and beyond it follow below."""
     from newton_amd import scenes
 
     model, state, info = scenes.bead_rope_light(cuda_device, mass=mass)
