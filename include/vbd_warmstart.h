@@ -65,7 +65,8 @@ int32_t vbd_ws_pack(void* stream, const float* params, uint16_t* packed);
 int32_t vbd_ws_forward(void* stream, int32_t n, const uint16_t* feat, const uint16_t* packed, const float* params,
                        float* out);
 
-/* Training step pieces for a batch of rows.
+/* Training step pieces for a batch of rows: the gradient in three calls, with H and Z in memory.  The reference that
+ * vbd_ws_gradient below is tested against; training itself takes that one or vbd_ws_train_step.
  * forward_train additionally saves H (BF16 [n,3,128]) and Z (FP32 [n,3,128]).
  * backward: loss = mean over rows and the 3 outputs of (out - target)^2 * w_row
  * (row_weight may be NULL = 1); writes per-workgroup partial gradients

@@ -379,7 +379,7 @@ __global__ void k_pack(const float* __restrict__ prm, uint16_t* __restrict__ pk)
     pk[e] = f2bf(v);
 }
 
-// ---- forward ---------------------------------------------------------------------
+// ---- forward of the separate training pieces (the tests' reference; training takes k_gradient) ----
 // One hidden layer for the wave's 16 rows: acc = A (16 x K) * Wt^T, A read from
 // LDS rows (stride kStride) or, for the first layer, from the feature rows.
 template <int K>
@@ -477,7 +477,7 @@ __global__ __launch_bounds__(kBlock) void k_forward(int n, const uint16_t* __res
 // activations are rounded to BF16 right after); the biases are the accumulators' first values.
 // Bound: the 384 SiLUs a row, two quarter-rate instructions each (about 85 us per million rows, 120 with the
 // multiplies); without the barriers of an LDS exchange the other waves' products fill in beside them:
-// 1,048,576 rows 127 us, 650 TFLOP/s (223 us with activations exchanged through LDS; 137 to 140 us on other cards and
+// 1,048,576 rows 127 us, 650 TFLOP/s (223 us with activations exchanged through LDS; 137 to 144 us on other cards and
 // under a kernel trace), 16,384 rows 9.2 us (17.7).
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
